@@ -63,6 +63,52 @@ MA_HD T smin(T a, T b) { return (b < a) ? b : a; }
 template <class T>
 MA_HD T smax(T a, T b) { return (a < b) ? b : a; }
 
+// ---- arithmetic of the paired-face kernels ----
+
+// a / b without the range scaling and the special cases of a full division:
+// FP64 the same Newton steps and correction as the full IEEE sequence, so the
+// same (correctly rounded) bits while a, b and a / b stay well inside the
+// normal range (8 instructions instead of 11, one of them a reciprocal
+// estimate either way); FP32 a * rcp(b), the bits of the 2.5-ulp division this
+// library is built with, which scales its operands by powers of two around
+// the same product.  Callers know the ranges (TameCheck, find_pairs).
+template <class T>
+MA_HD T quick_div(T a, T b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(T) == 8) {
+    T y = __builtin_amdgcn_rcp(b);
+    T e = __builtin_fma(-b, y, T(1));
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-b, y, T(1));
+    y = __builtin_fma(y, e, y);
+    const T q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  } else {
+    return a * __builtin_amdgcn_rcpf(b);
+  }
+#else
+  return a / b;
+#endif
+}
+
+// a / b from the correctly rounded reciprocal y = 1 / b, correctly rounded as
+// long as nothing underflows or overflows: P. W. Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34 (1990): one product, the exact remainder, one correction.
+template <class T>
+MA_HD T div_by(T a, T b, T y) {
+  const T q = a * y;
+  if constexpr (sizeof(T) == 8) return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+  else return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+}
+
+// A quotient or square root on a kTame path: quick forms; otherwise the full ones.
+template <bool kTame, class T>
+MA_HD T div_if(T a, T b) {
+  if constexpr (kTame) return quick_div(a, b);
+  else return a / b;
+}
+
 // Geometry-only part of the Roe flux: the area vector, its norm and the unit
 // normal, tangent and binormal (Roe_Flux.h:100-118).  It depends on the face
 // alone, so the solver computes it once per face at setup, with the same
@@ -373,7 +419,146 @@ struct RoeFlux {
     flux[3] = f3;
     flux[4] = f4;
   }
+
+  // The same flux through a face whose area vector has one nonzero component,
+  // p along axis D: flux_frame's operations on axis_frame_t's frame with the
+  // terms that are +-0 there left out (a sum they are added to keeps its value
+  // for finite operands; only the sign of an exact zero can differ).  With
+  // n = s e_D (s the sign of p), t = -s e_{D+2}, b = e_{D+1} the signs of the
+  // two shear waves cancel.  About 230 operations instead of 380.
+  template <int D, class T>
+  MA_HD void flux_axis(const T* pl, const T* pr, T* flux, T p) const {
+    constexpr int G = (D + 1) % 3, E = (D + 2) % 3;
+    const T efix = T(0.1), gm1 = T(0.4), half = T(0.5);
+    const T rl = pl[0], rr = pr[0];
+    const T* ul = pl + 1;
+    const T* ur = pr + 1;
+    const T p_l = pressure(pl), h_l = enthalpy(pl);
+    const T ht_l = h_l + half * (ul[0] * ul[0] + ul[1] * ul[1] + ul[2] * ul[2]);
+    const T mf_l = rl * (p * ul[D]);
+    const T p_r = pressure(pr), h_r = enthalpy(pr);
+    const T ht_r = h_r + half * (ur[0] * ur[0] + ur[1] * ur[1] + ur[2] * ur[2]);
+    const T mf_r = rr * (p * ur[D]);
+    const T psum = p_l + p_r;
+    T f[5];
+    f[0] = half * (mf_l + mf_r);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      T a = mf_l * ul[k] + mf_r * ur[k];
+      if (k == D) a = a + p * psum;
+      f[1 + k] = half * a;
+    }
+    f[4] = half * (mf_l * ht_l + mf_r * ht_r);
+
+    const T nn = fabs(p), s = copysign(T(1), p);
+    const T srl = sqrt(rl), srr = sqrt(rr);
+    const T denom = quick_div(T(1.0), srl + srr);  // root sums: always well inside the normal range
+    const T alpha = srl * denom;
+    const T beta = T(1.0) - alpha;
+    T u[3], dq[5];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) u[k] = alpha * ul[k] + beta * ur[k];
+    const T h = alpha * h_l + beta * h_r +
+                half * alpha * beta *
+                    ((ur[0] - ul[0]) * (ur[0] - ul[0]) + (ur[1] - ul[1]) * (ur[1] - ul[1]) +
+                     (ur[2] - ul[2]) * (ur[2] - ul[2]));
+    const T c = sqrt(gm1 * h);
+    const T vn = s * u[D];
+    const T ke = half * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+    const T cc = c * c;
+    const T ci2 = T(1.0) / cc;
+    const T hci2 = half * ci2;
+    dq[0] = rr - rl;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) dq[1 + k] = rr * ur[k] - rl * ul[k];
+    dq[4] = (rr * ht_r - p_r) - (rl * ht_l - p_l);
+
+    const T cbar = c * nn;
+    const T ubar = p * u[D];
+    const T cfl = fabs(ubar) + cbar;
+    const T eig1 = ubar + cbar, eig2 = ubar - cbar, eig3 = ubar;
+    T a1 = fabs(eig1), a2 = fabs(eig2), a3 = fabs(eig3);
+    const T ep = efix * cfl;
+    if (a1 < ep) a1 = half * (eig1 * eig1 + ep * ep) / ep;
+    if (a2 < ep) a2 = half * (eig2 * eig2 + ep * ep) / ep;
+    if (a3 < ep) a3 = half * (eig3 * eig3 + ep * ep) / ep;
+    const T s1 = half * (eig1 + a1) - half * (eig1 - a1);
+    const T s2 = half * (eig2 + a2) - half * (eig2 - a2);
+    const T s3 = half * (eig3 + a3) - half * (eig3 - a3);
+
+    const T kh = ke - h, gkh = gm1 * kh, sc = s * c;
+    T gu[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) gu[k] = gm1 * u[k];
+    T x0 = (gkh + c * (c - vn)) * dq[0];
+    T x1 = (gkh + c * (c + vn)) * dq[0];
+    T x2 = kh * dq[0];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (k == D) {
+        x0 += (sc - gu[k]) * dq[1 + k];
+        x1 += (-sc - gu[k]) * dq[1 + k];
+      } else {
+        const T g = gu[k] * dq[1 + k];
+        x0 -= g;
+        x1 -= g;
+      }
+      x2 -= u[k] * dq[1 + k];
+    }
+    x0 += gm1 * dq[4];
+    x1 += gm1 * dq[4];
+    x2 += dq[4];
+    const T l0 = s1 * x0, l1 = s2 * x1, l2 = s3 * x2;
+    const T l3 = s3 * (u[E] * dq[0] - dq[1 + E]);
+    const T l4 = s3 * (dq[1 + G] - u[G] * dq[0]);
+
+    const T hk = h + ke;
+    flux[0] = f[0] - half * (hci2 * l0 + hci2 * l1 - gm1 * ci2 * l2);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      T x;
+      if (k == D) {
+        x = (u[k] + sc) * hci2 * l0;
+        x += (u[k] - sc) * hci2 * l1;
+      } else {
+        const T uh = u[k] * hci2;
+        x = uh * l0;
+        x += uh * l1;
+      }
+      x -= gu[k] * ci2 * l2;
+      if (k == E) x -= l3;
+      if (k == G) x += l4;
+      flux[1 + k] = f[1 + k] - half * x;
+    }
+    T x = (hk + c * vn) * hci2 * l0;
+    x += (hk - c * vn) * hci2 * l1;
+    x += (cc - gm1 * hk) * ci2 * l2;
+    x -= u[E] * l3;
+    x += u[G] * l4;
+    flux[4] = f[4] - half * x;
+  }
 };
+
+// A policy may offer flux_axis for faces along an axis (RoeFlux does); others
+// get the face frame.
+template <class Inv, class T, class = void>
+struct takes_axis : std::false_type {};
+template <class Inv, class T>
+struct takes_axis<Inv, T,
+                  decltype(std::declval<const Inv&>().template flux_axis<0, T>(
+                               std::declval<const T*>(), std::declval<const T*>(), std::declval<T*>(), T()),
+                           void())> : std::true_type {};
+
+template <int D, class Inv, class T>
+MA_HD void inviscid_flux_axis(const Inv& inv, const T* vl, const T* vr, T* F, T p) {
+  if constexpr (takes_axis<Inv, T>::value) {
+    inv.template flux_axis<D, T>(vl, vr, F, p);
+  } else {
+    T a[3] = {T(0), T(0), T(0)};
+    a[D] = p;
+    inviscid_flux(inv, vl, vr, F, frame_from_area_t<T>(a));
+  }
+}
 
 // Thermal conductivity mu * Cp / Pr, Cp = 1006 (GasModel.h:100-106).
 struct NewtonianViscousFlux {
@@ -403,6 +588,34 @@ struct NewtonianViscousFlux {
       vflux[4] += kc * g[4][i] * a[i];
     }
   }
+  // The same through a face along axis D, p the nonzero component of its area
+  // vector: the terms of the two zero components, +-0 for finite gradients,
+  // are left out.  Uses gradient components (1,0) (2,1) (3,2), (k+1,D),
+  // (D+1,k) and (4,D) only.
+  template <int D, class T>
+  MA_HD void compute_flux_axis(const T g[5][3], const T* V, T p, T* vflux) const {
+    const T temp = V[4];
+    const T root = sqrt(temp);
+    const T mu = T(1.458e-6) * temp * root / (temp + T(110.4));
+    const T kc = mu * T(1006.0) / T(prandtl);
+    T div = g[1][0] + g[2][1] + g[3][2];
+    // FP32: the correctly rounded quotient, as the general form's compiles to.
+    // No float is within 2^-27 of making div / 3 a rounding boundary, so the
+    // double product decides every rounding, subnormal results included.
+    const T third = sizeof(T) == 4 ? T(double(div) * (1.0 / 3.0)) : div / T(3.);
+    vflux[0] = T(0.0);
+    T e = T(0.0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      T tij = T(0.5) * (g[i + 1][D] + g[D + 1][i]);
+      if (i == D) tij = tij - third;
+      const T m = T(2) * mu * tij;
+      vflux[1 + i] = m * p;
+      e += m * V[i + 1] * p;
+      if (i == D) e += kc * g[4][D] * p;
+    }
+    vflux[4] = e;
+  }
 };
 
 struct NoViscousFlux {
@@ -410,6 +623,8 @@ struct NoViscousFlux {
   double prandtl;
   template <class T>
   MA_HD void compute_flux(const T[5][3], const T*, const T*, T*) const {}
+  template <int D, class T>
+  MA_HD void compute_flux_axis(const T[5][3], const T*, T, T*) const {}
 };
 
 // ---- boundary policies ----
@@ -510,15 +725,21 @@ struct VenkatLimiter {
   // formula to dumax (du > 1e-40) or dumin (du < -1e-40); the bound is
   // selected first and the formula evaluated once, with the same operations,
   // so a wavefront whose lanes take both branches does one division, not two.
-  template <class T>
+  template <class T, bool kTame = false>
   static MA_HD T limit(T dumax, T dumin, T du, T deltax3) {
     T beta = 1;
     T eps2 = deltax3 * beta * beta * beta;
     const T d = du > T(0) ? dumax : dumin;
     T num = (d * d + eps2) * du + T(2) * du * du * d;
     T den = du * (d * d + T(2) * du * du + d * du + eps2);
-    const T phi = num / den;
-    return (du > T(1e-40) || du < -T(1e-40)) ? phi : T(1);
+    if constexpr (kTame && sizeof(T) == 4) {
+      // du may be small enough to make den subnormal, which the reciprocal
+      // does not take; the scaling is exact
+      num *= T(0x1p24);
+      den *= T(0x1p24);
+    }
+    const T phi = div_if<kTame>(num, den);
+    return fabs(du) > T(1e-40) ? phi : T(1);
   }
 };
 
@@ -526,12 +747,16 @@ struct VanAlbadaLimiter {
   enum { kind = 1 };
   // VanAlbadaLimiter.h:45-65 (defined but never called by the reference).
   // As in VenkatLimiter, the bound is selected before the one division.
-  template <class T>
+  template <class T, bool kTame = false>
   static MA_HD T limit(T dumax, T dumin, T du, T /*deltax3*/) {
     const T eps = T(2.220446049250313080847e-16);  // DBL_EPSILON
     const T d = du > eps ? dumax : dumin;
-    const T q = d / du;
-    const T y = (du > eps || du < -eps) ? q : T(2);
+    const T q = d / du;  // (a full division: d can be tiny beside du)
+    const T y = fabs(du) > eps ? q : T(2);
+    if constexpr (kTame) {  // no branch: the quotient is discarded where y >= 2
+      const T f = quick_div(T(4) * y - y * y, y * y - T(4) * y + T(8));
+      return y < T(2) ? smin(smax(f, T(0.0)), T(1.0)) : T(1);
+    }
     T phi = 1;
     if (y < T(2)) {
       phi = (T(4) * y - y * y) / (y * y - T(4) * y + T(8));

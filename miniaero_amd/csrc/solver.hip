@@ -26,6 +26,9 @@
 //            V buffer (stage 3: the next step's, from the new U; R itself
 //            is stored on stage 3 only)
 //
+// Meshes whose faces all lie along the axes run k_grad_pair and k_flux_pair
+// instead, with their own layout and no boundary launch (pair.hpp).
+//
 // Determinism and parity.  The reference scatters face results into cells
 // with atomics; with one thread the additions land in a fixed order: internal
 // faces in the permuted order (stable by left cell), then boundary faces.  At
@@ -129,6 +132,13 @@ struct DevMesh {
   int axis;
   // 1: no cell has an empty slot (every cell of a hexahedral mesh has six faces)
   int full;
+  // Paired meshes (pair.hpp) only: plane length of their arrays (nc rounded
+  // up to 64) and geometry tables in the arithmetic type, shared like gtab's
+  // (see slot_geo there)
+  int ns;
+  int nsrec, nfrec;
+  const void* __restrict__ stab;
+  const void* __restrict__ ptab;
 };
 
 struct Inflow {
@@ -149,6 +159,9 @@ struct TileMap {
   const int* __restrict__ cptr;   // ntiles + 1: cells of tile b are [cptr[b], cptr[b+1])
   const int* __restrict__ tcase;  // ntiles: the case (independent mesh) tile b belongs to
   const int* __restrict__ fgid;   // parallel to faces: the face's record in DevMesh::gtab
+  // paired meshes: ptr, lr and fgid describe the lists of flux_tile_pair, and
+  // slot16 (6 planes of nc: LDS index << 1 | side) replaces slot
+  const unsigned short* __restrict__ slot16;
 };
 
 template <class S, class T>
@@ -413,21 +426,13 @@ __global__ __launch_bounds__(kBlock) void k_init(DevMesh m, const double* __rest
 // The stage state is FP64; V is stored in the arithmetic type T.
 template <class T>
 __device__ __forceinline__ void prim_cell(int nc, const double* __restrict__ Un, const double* __restrict__ R,
-                                          double alpha, T* __restrict__ V, int c) {
+                                          double alpha, int c, T* w) {
   double u[5], v[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) u[k] = Un[(size_t)k * nc + c] + alpha * R[(size_t)k * nc + c];
   ma::primitives(u, v);
 #pragma unroll
-  for (int k = 0; k < 5; ++k) V[(size_t)k * nc + c] = T(v[k]);
-}
-
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_prim(int nc, const double* __restrict__ Un,
-                                                 const double* __restrict__ R, double alpha,
-                                                 T* __restrict__ V) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < nc) prim_cell(nc, Un, R, alpha, V, c);
+  for (int k = 0; k < 5; ++k) w[k] = T(v[k]);
 }
 
 
@@ -1133,6 +1138,31 @@ __global__ __launch_bounds__(kBlock) void k_copy(long long n2, const double2* __
   if (i < n2) b[i] = a[i];
 }
 
+#include "pair.hpp"
+
+// pair: V is laid out for the paired kernels (m.ns long planes, pair.hpp).
+template <class T>
+__device__ __forceinline__ void prim_cell_any(const DevMesh& m, const double* __restrict__ Un,
+                                              const double* __restrict__ R, double alpha, T* __restrict__ V, int c,
+                                              bool pair) {
+  T w[5];
+  prim_cell(m.nc, Un, R, alpha, c, w);
+  if (pair) {
+    put_five(V, m.ns, (unsigned)c, w);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) V[(size_t)k * m.nc + c] = w[k];
+  }
+}
+
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_prim(DevMesh m, const double* __restrict__ Un,
+                                                 const double* __restrict__ R, double alpha,
+                                                 T* __restrict__ V, int pair) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < m.nc) prim_cell_any(m, Un, R, alpha, V, c, pair != 0);
+}
+
 // ------------------------------------------------- multi-case launches --
 // Several independent single-case runs advanced by the same launches (the
 // served form's continuous batching): each workgroup finds its case from a
@@ -1178,7 +1208,8 @@ __global__ __launch_bounds__(kBlock) void k_prim_multi(const CaseView* __restric
   const CaseView& v = cv[k];
   if (!v.prim0) return;
   const int c = (g - start[k]) * kBlock + threadIdx.x;
-  if (c < v.m.nc) prim_cell(v.m.nc, v.U[v.parity ^ parity], v.R, alpha, static_cast<T*>(v.V[0]), c);
+  if (c < v.m.nc)
+    prim_cell_any(v.m, v.U[v.parity ^ parity], v.R, alpha, static_cast<T*>(v.V[0]), c, false);
 }
 
 template <bool kSecondOrder, bool kFaceVals, class Limiter, class T>
@@ -1327,7 +1358,7 @@ __device__ __forceinline__ bool grid_sync(unsigned* gsync, unsigned& gen, long l
 template <bool kViscousSO, class T>
 constexpr int kStepsWaves = sizeof(T) == 8 ? (kViscousSO ? 1 : 2) : 1;
 
-template <bool SO, class Inv, class Visc, class Lim, class T>
+template <bool SO, class Inv, class Visc, class Lim, class T, bool kPair>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(kStepsWaves<SO && Visc::isViscous, T>)))
 void k_steps(PersistArgs a, Inv inv, Visc visc) {
   // TimeSolverExplicitRK4.h:187-195: alpha = {0, 1/2, 1/2, 1}, beta = {1/6,
@@ -1365,7 +1396,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
     if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
     if (it == 0 && a.prim0) {
       for (int c = blockIdx.x * kTile + threadIdx.x; c < m.nc; c += G * kTile)
-        prim_cell(m.nc, Un, a.R, 0.0, static_cast<T*>(a.V[0]), c);
+        prim_cell_any(m, Un, a.R, 0.0, static_cast<T*>(a.V[0]), c, kPair);
       if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
     }
     for (int irk = 0; irk < 4; ++irk) {
@@ -1377,6 +1408,10 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
           const int b = xcd * a.per_blocks + j;
           if (b * kBlock >= m.nc) break;  // uniform over the workgroup
           const int c = b * kBlock + threadIdx.x;
+          if constexpr (kPair) {
+            if (c < m.nc) grad_pair<SO, FV, Lim, T>(m, a.nbr, Vs, rec, static_cast<T*>(a.fv), (unsigned)c);
+            continue;
+          }
           T out[kRec];
           if (c < m.nc)
             grad_cell<SO, FV, Lim, T, 2>(m, a.nbr, Vs, rec, static_cast<T*>(a.fv), c, out);
@@ -1387,7 +1422,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
         }
         if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
       }
-      if (nbf > 0) {
+      if (!kPair && nbf > 0) {  // (paired meshes: boundary faces are in the tiles' lists)
         for (int i = blockIdx.x * kTile + threadIdx.x; i < nbf; i += G * kTile)
           bc_face<Inv, ma::ReferenceBoundaries>(m, Vs, inv, visc.prandtl, a.inflow, a.bc_case,
                                                 static_cast<T*>(a.bc), i);
@@ -1397,9 +1432,14 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
       for (int j = j0; j < a.t.per_xcd; j += xstride) {
         const int tile = xcd * a.t.per_xcd + j;
         if (tile >= a.t.ntiles) break;  // uniform over the workgroup
-        flux_tile<SO, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, static_cast<const T*>(a.bc),
-                                    irk == 0 ? Un : Uacc, Uacc, a.R, a.dt, beta(irk), inv, visc, Un, Vn,
-                                    alpha_next(irk), irk == 3 ? 1 : 0);
+        if constexpr (kPair)
+          flux_tile_pair<SO, true, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, a.inflow, irk == 0 ? Un : Uacc,
+                                                 Uacc, a.R, a.dt, beta(irk), inv, visc, Un, Vn, alpha_next(irk),
+                                                 irk == 3 ? 1 : 0);
+        else
+          flux_tile<SO, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, static_cast<const T*>(a.bc),
+                                      irk == 0 ? Un : Uacc, Uacc, a.R, a.dt, beta(irk), inv, visc, Un, Vn,
+                                      alpha_next(irk), irk == 3 ? 1 : 0);
         __syncthreads();  // the LDS is reused by the next tile
       }
       if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
@@ -1462,6 +1502,8 @@ struct ma_solver {
   void* grad = nullptr;  // gradient records (kRec values per cell: gradient, limiter)
   void* fv = nullptr;  // kMaxSlots x 5 planes: extrapolated face values (inviscid second order)
   bool fp32 = false;
+  bool pair = false;          // runs the paired-mesh kernels and array layouts (pair.hpp)
+  bool wall = false;          // some boundary face is a no-slip wall
   // Cases (independent meshes stepped together; a plain run is one case).
   int ncases = 1;
   std::vector<ma_options> case_opt;
@@ -1711,6 +1753,17 @@ void cell_order(const ma_mesh_data* md, const TileShape& shape, std::vector<int>
   }
 }
 
+// What the paired-mesh kernels (pair.hpp) read instead of the general slot
+// and tile tables; ok when the mesh is paired (find_pairs).
+struct PairPlan {
+  bool ok = false;
+  int max_faces = 64;                    // longest tile list, padding included
+  std::vector<int> nbr, ent;             // kMaxSlots planes of nc: (low, high) along x, y, z
+  std::vector<int> srec, frec;           // slot record -> geometry record << 1 | side; face record -> geometry record
+  std::vector<int> ptr, lr, gid;         // tile lists, lr 2 per entry (see flux_tile_pair)
+  std::vector<unsigned short> slot;      // kMaxSlots planes of nc: list index << 1 | side
+};
+
 // Everything the device needs, computed on the host (no GPU involved).
 struct Layout {
   // frees every array of `other` (used to release merged parts)
@@ -1728,7 +1781,47 @@ struct Layout {
   // every area vector has at most one nonzero component and every cell
   // volume has a finite reciprocal in FP32 and FP64 (DevMesh::axis)
   bool axis = false;
+  bool wall = false;  // some boundary face is MA_BC_NOSLIP
+  PairPlan pair;
 };
+
+// Every index the paired kernels will use, checked on the host before any upload.
+ma_status validate_pairs(const Layout& L) {
+  const PairPlan& P = L.pair;
+  const int nc = L.nc, ntiles = L.ntiles;
+  const size_t ng = L.geo.size() / kGeoVals;
+  auto bad = [](const char* what) { return ma::fail(MA_ERR_INVALID, std::string("layout: paired ") + what); };
+  if (P.nbr.size() != (size_t)kMaxSlots * nc || P.ent.size() != P.nbr.size() || P.slot.size() != P.nbr.size() ||
+      (int)P.ptr.size() != ntiles + 1 || P.gid.size() * 2 != P.lr.size() ||
+      (size_t)P.ptr[ntiles] > P.gid.size() || (size_t)P.max_faces * 5 * sizeof(double) > 65536)
+    return bad("sizes");
+  for (size_t i = 0; i < P.nbr.size(); ++i)
+    if (P.nbr[i] < 0 || P.nbr[i] >= nc || P.ent[i] < 0 || (size_t)P.ent[i] >= P.srec.size()) return bad("slots");
+  for (int x : P.srec)
+    if (x < 0 || (size_t)(x >> 1) >= ng) return bad("slot records");
+  for (int x : P.frec)
+    if (x < 0 || (size_t)x >= ng) return bad("face records");
+  for (int b = 0; b < ntiles; ++b) {
+    const int f0 = P.ptr[b], n = P.ptr[b + 1] - f0;
+    if (n < 0 || n % 64 || n > P.max_faces) return bad("tile lists");
+    for (int q = f0; q < f0 + n; ++q) {
+      const int x = P.lr[2 * (size_t)q], r = P.lr[2 * (size_t)q + 1], l = x < 0 ? -1 : x & ((1 << kCellBits) - 1);
+      if (x >= 0 ? x >> kCellBits != P.lr[2 * (size_t)(q - (q - f0) % 64)] >> kCellBits || x >> kCellBits > 2
+                 : (q - f0) % 64 == 0)
+        return bad("tile chunks");
+      if (l >= nc || r >= nc || P.gid[q] < 0 || (size_t)P.gid[q] >= P.frec.size() || (l >= 0 && r < 0 && (~r >> 2) >= L.nbf))
+        return bad("tile faces");
+    }
+    for (int c = L.tile_cptr[b]; c < L.tile_cptr[b + 1]; ++c)
+      for (int s = 0; s < kMaxSlots; ++s) {
+        const int e = P.slot[(size_t)s * nc + c], j = e >> 1;
+        if (j >= n || P.lr[2 * (size_t)(f0 + j)] < 0 ||
+            ((e & 1) ? P.lr[2 * (size_t)(f0 + j) + 1] : P.lr[2 * (size_t)(f0 + j)] & ((1 << kCellBits) - 1)) != c)
+          return bad("tile slots");
+      }
+  }
+  return MA_OK;
+}
 
 // Every index a kernel will use, checked on the host before any upload.
 ma_status validate_layout(const Layout& L) {
@@ -1788,7 +1881,7 @@ ma_status validate_layout(const Layout& L) {
     }
   }
   }
-  return MA_OK;
+  return L.pair.ok ? validate_pairs(L) : MA_OK;
 }
 
 // Concatenation of independent cases' layouts into one: cells, internal faces,
@@ -1835,7 +1928,25 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
   M.fgeo.assign(M.nf, 0);
   M.geo.clear();
   M.axis = true;
-  for (int k = 0; k < n; ++k) M.axis = M.axis && parts[k].axis;
+  M.pair.ok = true;
+  M.wall = false;
+  for (int k = 0; k < n; ++k) {
+    M.axis = M.axis && parts[k].axis;
+    M.pair.ok = M.pair.ok && parts[k].pair.ok;
+    M.wall = M.wall || parts[k].wall;
+  }
+  if (M.pair.ok) {
+    size_t entries = 0;
+    for (int k = 0; k < n; ++k) {
+      entries += parts[k].pair.gid.size();
+      M.pair.max_faces = std::max(M.pair.max_faces, parts[k].pair.max_faces);
+    }
+    for (auto* v : {&M.pair.nbr, &M.pair.ent}) v->assign((size_t)kMaxSlots * nc, 0);
+    M.pair.slot.assign((size_t)kMaxSlots * nc, 0);
+    M.pair.ptr.assign(1, 0);
+    M.pair.lr.reserve(2 * entries);
+    M.pair.gid.reserve(entries);
+  }
   tile_case.assign(M.ntiles, 0);
   case_tiles.assign(n + 1, 0);
   bc_case.assign(std::max(1, M.nbf), 0);
@@ -1892,6 +2003,27 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
     }
     {  // this part's geometry records follow the earlier parts'
       const int r0 = (int)(M.geo.size() / kGeoVals);
+      if (M.pair.ok) {
+        const PairPlan& P = L.pair;
+        const int s0 = (int)M.pair.srec.size(), p0 = (int)M.pair.frec.size();
+        for (int q = 0; q < kMaxSlots; ++q)
+          for (int c = 0; c < lnc; ++c) {
+            const size_t to_ = (size_t)q * nc + co[k] + c, from = (size_t)q * lnc + c;
+            M.pair.nbr[to_] = co[k] + P.nbr[from];
+            M.pair.ent[to_] = s0 + P.ent[from];
+            M.pair.slot[to_] = P.slot[from];
+          }
+        const int e0 = M.pair.ptr.back();
+        for (int b = 0; b < L.ntiles; ++b) M.pair.ptr.push_back(e0 + P.ptr[b + 1]);
+        for (size_t q = 0; q < P.gid.size(); ++q) {
+          const int l = P.lr[2 * q], r = P.lr[2 * q + 1];
+          M.pair.lr.push_back(l < 0 ? l : co[k] + l);
+          M.pair.lr.push_back(l < 0 ? r : r >= 0 ? co[k] + r : ~(~r + (bo[k] << 2)));
+          M.pair.gid.push_back(p0 + P.gid[q]);
+        }
+        for (int x : P.srec) M.pair.srec.push_back(x + 2 * r0);
+        for (int x : P.frec) M.pair.frec.push_back(x + r0);
+      }
       for (int f = 0; f < lnf; ++f) M.fgeo[gf(f)] = r0 + L.fgeo[f];
       M.geo.insert(M.geo.end(), L.geo.begin(), L.geo.end());
     }
@@ -1965,7 +2097,171 @@ void dedupe_geometry(Layout& L) {
   }
 }
 
-ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, Layout& L) {
+// Whether the mesh is paired -- every cell has six faces, two per axis, one on
+// its low side and one on its high side, every area vector has exactly one
+// nonzero component, positive on internal faces (left to right is up the axis)
+// -- with geometry inside the bounds under which the quotients of a tame stage
+// (pair.hpp) stay in the normal range; then the tables of the paired kernels.
+// Bounds: |area| in [2^-37, 2^100], volume in [2^-100, 2^24], displacements at
+// most 2^50 with squared length at least 2^-56, and largest area times largest
+// displacement at most 2^14 volumes, so that a gradient times a displacement
+// is at most 2^17 times the largest primitive: FP64 limiter terms stay below
+// 2^(3 (100 + 17) + 6), FP32 ones, scaled by 2^24, below 2^(3 (16 + 17) + 3 + 24),
+// and an FP32 limiter is at least 2^-56 / 2^(2 (16 + 17) + 2).
+void find_pairs(Layout& L) {
+  PairPlan& P = L.pair;
+  P = PairPlan();
+  const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
+  if (!L.axis) return;
+  const size_t ng = L.geo.size() / kGeoVals;
+  std::vector<signed char> axis_of(ng, -1);
+  std::vector<double> amax(ng), dmax(ng);
+  for (size_t r = 0; r < ng; ++r) {
+    const double* q = &L.geo[r * kGeoVals];
+    for (int d = 0; d < 3; ++d)
+      if (q[d] != 0.0) axis_of[r] = (signed char)d;
+    if (axis_of[r] < 0) return;
+    amax[r] = std::fabs(q[axis_of[r]]);
+    if (!(amax[r] >= 0x1p-37 && amax[r] <= 0x1p100)) return;
+    for (int k = 3; k < 9; ++k) dmax[r] = std::max(dmax[r], std::fabs(q[k]));
+    if (!(dmax[r] <= 0x1p50) || !(q[3] * q[3] + q[4] * q[4] + q[5] * q[5] >= 0x1p-56)) return;
+  }
+  for (int f = 0; f < nif; ++f) {
+    const double* q = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
+    if (!(q[axis_of[L.fgeo[f]]] > 0.0) || !(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) return;
+  }
+  P.nbr.assign((size_t)kMaxSlots * nc, -1);
+  P.ent.assign((size_t)kMaxSlots * nc, -1);
+  for (int c = 0; c < nc; ++c) {
+    double am = 0.0, dm = 0.0;
+    for (int q = 0; q < kMaxSlots; ++q) {
+      const int e = L.slot[(size_t)q * nc + c];
+      if (e < 0) return;
+      const int f = e >> 1, side = e & 1, r = L.fgeo[f], d = axis_of[r];
+      const double a = L.geo[(size_t)r * kGeoVals + d];
+      const int s = 2 * d + ((side ? -a : a) > 0.0 ? 1 : 0);
+      if (P.ent[(size_t)s * nc + c] >= 0) return;
+      P.ent[(size_t)s * nc + c] = (r << 1) | side;
+      P.nbr[(size_t)s * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
+      am = std::max(am, amax[r]);
+      dm = std::max(dm, dmax[r]);
+    }
+    if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) return;
+  }
+  // Tile lists in chunks of 64 entries of one axis: the faces inside the tile
+  // by left cell, a chunk per axis and block of 64 cells (blocks with few
+  // faces share one), then the faces shared with other tiles (low side, high
+  // side, by the tile's own cell) and the boundary faces.  Chunk r of the
+  // three axes and chunk r of the shared faces follow each other.
+  std::vector<int> tile_of(nc);
+  for (int b = 0; b < ntiles; ++b)
+    for (int d = L.tile_cptr[b]; d < L.tile_cptr[b + 1]; ++d) tile_of[d] = b;
+  P.ptr.assign(1, 0);
+  P.slot.assign((size_t)kMaxSlots * nc, 0);
+  std::vector<int> pos(nf);  // list index of a face in the tile being built
+  using Key = std::pair<unsigned long long, int>;
+  std::vector<Key> keys[3];
+  std::vector<std::pair<int, int>> chunks[4];  // (axis, first key), by axis; shared and boundary faces
+  std::vector<int> lens[4];
+  for (int b = 0; b < ntiles; ++b) {
+    const int c0 = L.tile_cptr[b], c1 = L.tile_cptr[b + 1];
+    for (auto& k : keys) k.clear();
+    auto add = [&](int f, int cls, int cell) {
+      keys[axis_of[L.fgeo[f]]].push_back({((unsigned long long)cls << 32) | (unsigned)cell, f});
+    };
+    for (int q = L.tptr[b]; q < L.tptr[b + 1]; ++q) {
+      const int f = L.tfaces[q], l = L.fl[f], r = L.fr[f];
+      const bool inl = tile_of[l] == b, inr = tile_of[r] == b;
+      add(f, inl && inr ? 0 : inr ? 1 : 2, inl ? l : r);
+    }
+    for (int c = c0; c < c1; ++c)
+      for (int q = 0; q < kMaxSlots; ++q) {
+        const int f = L.slot[(size_t)q * nc + c] >> 1;
+        if (f >= nif) add(f, 3, c);
+      }
+    for (int q = 0; q < 4; ++q) {
+      chunks[q].clear();
+      lens[q].clear();
+    }
+    for (int d = 0; d < 3; ++d) {
+      std::vector<Key>& K = keys[d];
+      std::sort(K.begin(), K.end());
+      auto block = [&](int i) { return (K[i].first >> 32) ? 1 << 30 : ((int)(K[i].first & 0xffffffffu) - c0) / 64; };
+      const int nk = (int)K.size();
+      for (int i = 0; i < nk;) {
+        int j = i;
+        const bool inside = !(K[i].first >> 32);
+        while (j < nk && j - i < 64 && inside == !(K[j].first >> 32)) {
+          int e = j;  // whole blocks inside the tile, single faces otherwise
+          while (e < nk && (e == j || (inside && block(e) == block(j)))) ++e;
+          if (e - i > 64) break;
+          j = e;
+        }
+        chunks[inside ? d : 3].push_back({d, i});
+        lens[inside ? d : 3].push_back(j - i);
+        i = j;
+      }
+    }
+    int n = 0;
+    for (size_t r = 0, left = 1; left; ++r) {
+      left = 0;
+      for (int q = 0; q < 4; ++q) {
+        if (r >= chunks[q].size()) continue;
+        left = 1;
+        const int d = chunks[q][r].first, i = chunks[q][r].second;
+        for (int k = i; k < i + lens[q][r]; ++k) {
+          const int f = keys[d][k].second;
+          pos[f] = n++;
+          P.lr.push_back(L.fl[f] | (d << kCellBits));
+          P.lr.push_back(f < nif ? L.fr[f] : ~(((f - nif) << 2) | (L.fkind[f] - 1)));
+          P.gid.push_back(L.fgeo[f]);
+        }
+        for (; n % 64; ++n) {
+          P.lr.push_back(-1);
+          P.lr.push_back(-1);
+          P.gid.push_back(0);
+        }
+      }
+    }
+    P.ptr.push_back(P.ptr.back() + n);
+    P.max_faces = std::max(P.max_faces, n);
+    if ((size_t)P.max_faces * 5 * sizeof(double) > 65536) {  // e.g. long thin tiles of consecutive cells
+      P = PairPlan();
+      return;
+    }
+    // summation order: internal faces in slot order, then the boundary faces
+    // by kind (in slot order within a kind), the order of TimeSolverExplicitRK4.h:428-475
+    for (int c = c0; c < c1; ++c) {
+      int w = 0;
+      for (int kind = 0; kind <= MA_BC_INFLOW; ++kind)
+        for (int q = 0; q < kMaxSlots; ++q) {
+          const int e = L.slot[(size_t)q * nc + c], f = e >> 1;
+          if ((f < nif ? 0 : L.fkind[f]) != kind) continue;
+          P.slot[(size_t)w++ * nc + c] = (unsigned short)((pos[f] << 1) | (e & 1));
+        }
+    }
+  }
+  // records renumbered in the order the kernels meet them
+  auto renumber = [](std::vector<int>& ids, size_t most, std::vector<int>& rec) {
+    std::vector<int> now(most, -1);
+    for (int& x : ids) {
+      if (now[x] < 0) {
+        now[x] = (int)rec.size();
+        rec.push_back(x);
+      }
+      x = now[x];
+    }
+  };
+  renumber(P.ent, 2 * ng, P.srec);
+  renumber(P.gid, ng, P.frec);
+  if (P.srec.size() >= (1u << 28)) {  // 32-bit byte offsets into the record planes
+    P = PairPlan();
+    return;
+  }
+  P.ok = true;
+}
+
+ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, bool pairs, Layout& L) {
   const int nc = md->num_owned_cells;
   L.nc = nc;
   const ma_faces& I = md->internal_faces;
@@ -2167,6 +2463,8 @@ ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, Layout& L)
   L.ntiles = ntiles;
   L.max_faces = max_faces;
   dedupe_geometry(L);
+  for (int f = nif; f < nf; ++f) L.wall = L.wall || fkind[f] == MA_BC_NOSLIP;
+  if (pairs) find_pairs(L);
   return MA_OK;
 }
 
@@ -2252,7 +2550,10 @@ struct RunPlan {
   std::vector<int> tile_case, case_tiles, bc_case, cell_case, case_cell_off;
 };
 
-ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, RunPlan& P) {
+// pairs: meshes that qualify get the paired kernels' tables (find_pairs).  The
+// served form plans without: there, where cases come and go in launches of
+// many, the paired kernels are not used.
+ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, bool pairs, RunPlan& P) {
   if (!valid_shape(shape)) return ma::fail(MA_ERR_INVALID, "tile shape: extents >= 1 with product <= 256, or all 0");
   P.case_cell_off.assign(ncases + 1, 0);
   long long total_cells = 0, total_faces = 0;
@@ -2269,7 +2570,7 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
   ma_status st = MA_OK;
   Layout& L = P.L;
   if (ncases == 1) {
-    if ((st = plan_layout(mds[0], shape, L))) return st;
+    if ((st = plan_layout(mds[0], shape, pairs, L))) return st;
     P.all_lattice = L.dims[0] > 0;
     P.tile_case.assign(L.ntiles, 0);
     P.case_tiles = {0, L.ntiles};
@@ -2284,7 +2585,7 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
     auto worker = [&] {
       for (int k = next++; k < ncases; k = next++) {
         try {
-          status[k] = plan_layout(mds[k], shape, parts[k]);
+          status[k] = plan_layout(mds[k], shape, pairs, parts[k]);
           if (status[k]) message[k] = ma::last_error();
         } catch (const std::bad_alloc&) {
           status[k] = MA_ERR_NOMEM;
@@ -2316,43 +2617,19 @@ void plan_stats(const Layout& L, long long* stats) {
   stats[6] = L.derive_frame ? 1 : 0;
 }
 
-// Device arrays of one run from its plan: the layout, the per-case
-// parameters and the work buffers.  With s->counting set nothing is
-// allocated or copied; s->arena_used is then the device bytes the run needs.
-// The plan is only read, so one plan can build many runs (the served form
-// keeps plans of the mesh shapes it has seen).
-ma_status build_planned(ma_solver* s, const RunPlan& P) {
+// Tables of the general kernels: per-face planes, slot and neighbour lists, tile lists.
+ma_status upload_general(ma_solver* s, const Layout& L) {
   ma_status st = MA_OK;
-  const int ncases = s->ncases;
-  s->all_lattice = P.all_lattice;
-  const Layout& L = P.L;
-  const std::vector<int>& tile_case = P.tile_case;
-  const std::vector<int>& case_tiles = P.case_tiles;
-  const std::vector<int>& bc_case = P.bc_case;
-  const std::vector<int>& cell_case = P.cell_case;
   const int nc = L.nc, nif = L.nif, nf = L.nf;
-  const long long nbf = L.nbf;
-  if (!s->counting) {
-    s->case_cell_off = P.case_cell_off;
-    s->dev_of = L.dev_of;
-  }
   DevMesh& m = s->m;
-  m.nc = nc;
-  m.nif = nif;
-  m.nf = nf;
-  double *dvol, *dxc, *dfn, *dffr = nullptr, *dfw;
-  int *dslot, *dfl, *dfr, *dorg;
+  double *dfn, *dffr = nullptr;
+  int *dslot, *dfl, *dfr;
   signed char* dkind;
-  if ((st = upload(s, &dvol, L.vol)) || (st = upload(s, &dxc, L.xc)) || (st = upload(s, &dslot, L.slot)) ||
-      (st = upload(s, &dfn, L.fn)) || (!L.derive_frame && (st = upload(s, &dffr, L.ffr))) ||
-      (st = upload(s, &dorg, L.org_of)) ||
-      (st = upload(s, &dfl, L.fl)) || (st = upload(s, &dfr, L.fr)) ||
-      (st = upload(s, &dkind, L.fkind)) || (st = upload(s, &dfw, L.fwall)))
+  if ((st = upload(s, &dslot, L.slot)) || (st = upload(s, &dfn, L.fn)) ||
+      (!L.derive_frame && (st = upload(s, &dffr, L.ffr))) || (st = upload(s, &dfl, L.fl)) ||
+      (st = upload(s, &dfr, L.fr)) || (st = upload(s, &dkind, L.fkind)))
     return st;
-  m.vol = dvol;
-  s->xc = dxc;
   m.slot = dslot;
-  s->org = dorg;
   m.fn = dfn;
   m.fn32 = nullptr;
   if (s->fp32) {  // the area vector in FP32 for the FP32-arithmetic kernels
@@ -2375,7 +2652,6 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   m.fl = dfl;
   m.fr = dfr;
   m.fkind = dkind;
-  m.fwall = dfw;
   // neighbour planes: the cell across each slot's internal face, else the cell itself
   {
     int* dnbr = nullptr;
@@ -2394,12 +2670,9 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
     s->nbr = dnbr;
   }
 
-  int *dtptr, *dtfaces, *dtslot, *dtcptr, *dtcase;
-  if ((st = upload(s, &dtptr, L.tptr)) || (st = upload(s, &dtfaces, L.tfaces)) || (st = upload(s, &dtslot, L.tslot)) ||
-      (st = upload(s, &dtcptr, L.tile_cptr)) || (st = upload(s, &dtcase, tile_case)))
+  int *dtptr, *dtfaces, *dtslot;
+  if ((st = upload(s, &dtptr, L.tptr)) || (st = upload(s, &dtfaces, L.tfaces)) || (st = upload(s, &dtslot, L.tslot)))
     return st;
-  s->t.ntiles = L.ntiles;
-  s->t.per_xcd = (L.ntiles + kXcds - 1) / kXcds;
   s->t.max_faces = L.max_faces;
   s->t.ptr = dtptr;
   s->t.faces = dtfaces;
@@ -2431,8 +2704,6 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
     s->t.lr = dlr;
   }
   s->t.slot = dtslot;
-  s->t.cptr = dtcptr;
-  s->t.tcase = dtcase;
   // face geometry records, and each tile face's record index
   {
     void* dg = nullptr;
@@ -2463,6 +2734,119 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
     if (st) return st;
     m.sgeo = dsg;
   }
+  return MA_OK;
+}
+
+// Geometry tables of the paired kernels in the arithmetic type (DevMesh::stab,
+// ptab), the values general records hold.
+template <class T>
+ma_status upload_pair_geo(ma_solver* s, const Layout& L) {
+  const PairPlan& P = L.pair;
+  const size_t ns = P.srec.size(), nf = P.frec.size();
+  T *ds = nullptr, *dp = nullptr;
+  ma_status st = MA_OK;
+  if (s->counting) {
+    if ((st = s->alloc(&ds, 4 * ns)) || (st = s->alloc(&dp, 8 * nf))) return st;
+  } else {
+    constexpr int W = 16 / (int)sizeof(T);  // values of a vector
+    auto at = [](std::vector<T>& h, size_t n, int k, size_t i) -> T& { return h[((size_t)(k / W) * n + i) * W + k % W]; };
+    auto area = [&](int r) {  // the nonzero component, exactly
+      const double* q = &L.geo[(size_t)r * kGeoVals];
+      return q[0] + q[1] + q[2];
+    };
+    std::vector<T> hs(4 * ns, T(0)), hp(8 * nf, T(0));
+    for (size_t i = 0; i < ns; ++i) {
+      const int r = P.srec[i] >> 1, side = P.srec[i] & 1;
+      at(hs, ns, 0, i) = T(side ? -area(r) : area(r));
+      for (int d = 0; d < 3; ++d) at(hs, ns, 1 + d, i) = T(L.geo[(size_t)r * kGeoVals + 3 + 3 * side + d]);
+    }
+    for (size_t i = 0; i < nf; ++i) {
+      at(hp, nf, 0, i) = T(area(P.frec[i]));
+      for (int d = 0; d < 6; ++d) at(hp, nf, 1 + d, i) = T(L.geo[(size_t)P.frec[i] * kGeoVals + 3 + d]);
+    }
+    if ((st = upload(s, &ds, hs)) || (st = upload(s, &dp, hp))) return st;
+  }
+  s->m.stab = ds;
+  s->m.ptab = dp;
+  s->m.nsrec = (int)ns;
+  s->m.nfrec = (int)nf;
+  return MA_OK;
+}
+
+// Tables of the paired kernels (pair.hpp).
+ma_status upload_paired(ma_solver* s, const Layout& L) {
+  const PairPlan& P = L.pair;
+  ma_status st = MA_OK;
+  int *dptr, *dlr, *dgid, *dids = nullptr;
+  unsigned short* dslot;
+  const int nc = L.nc, ns = (nc + 63) / 64 * 64;
+  s->m.ns = ns;
+  if ((st = upload(s, &dptr, P.ptr)) || (st = upload(s, &dlr, P.lr)) || (st = upload(s, &dgid, P.gid)) ||
+      (st = upload(s, &dslot, P.slot)) || (st = s->fp32 ? upload_pair_geo<float>(s, L) : upload_pair_geo<double>(s, L)))
+    return st;
+  if (s->counting) {
+    st = s->alloc(&dids, (size_t)12 * ns);
+  } else {  // see slot_ids
+    std::vector<int> h((size_t)12 * ns, 0);
+    for (int k = 0; k < 12; ++k) {
+      const int* from = k < 6 ? &P.nbr[(size_t)k * nc] : &P.ent[(size_t)(k - 6) * nc];
+      for (int c = 0; c < nc; ++c) h[((size_t)(k / 4) * ns + c) * 4 + k % 4] = from[c];
+    }
+    st = upload(s, &dids, h);
+  }
+  if (st) return st;
+  s->nbr = dids;
+  s->m.axis = s->m.full = 1;
+  s->t.ptr = dptr;
+  s->t.lr = reinterpret_cast<const int2*>(dlr);
+  s->t.fgid = dgid;
+  s->t.slot16 = dslot;
+  s->t.max_faces = P.max_faces;
+  return MA_OK;
+}
+
+// Device arrays of one run from its plan: the layout, the per-case
+// parameters and the work buffers.  With s->counting set nothing is
+// allocated or copied; s->arena_used is then the device bytes the run needs.
+// The plan is only read, so one plan can build many runs (the served form
+// keeps plans of the mesh shapes it has seen).
+ma_status build_planned(ma_solver* s, const RunPlan& P) {
+  ma_status st = MA_OK;
+  const int ncases = s->ncases;
+  s->all_lattice = P.all_lattice;
+  const Layout& L = P.L;
+  const std::vector<int>& tile_case = P.tile_case;
+  const std::vector<int>& case_tiles = P.case_tiles;
+  const std::vector<int>& bc_case = P.bc_case;
+  const std::vector<int>& cell_case = P.cell_case;
+  const int nc = L.nc, nf = L.nf;
+  const long long nbf = L.nbf;
+  if (!s->counting) {
+    s->case_cell_off = P.case_cell_off;
+    s->dev_of = L.dev_of;
+  }
+  DevMesh& m = s->m;
+  m.nc = nc;
+  m.nif = L.nif;
+  m.nf = nf;
+  double *dvol, *dxc, *dfw;
+  int* dorg;
+  if ((st = upload(s, &dvol, L.vol)) || (st = upload(s, &dxc, L.xc)) || (st = upload(s, &dorg, L.org_of)) ||
+      (st = upload(s, &dfw, L.fwall)))
+    return st;
+  m.vol = dvol;
+  s->xc = dxc;
+  s->org = dorg;
+  m.fwall = dfw;
+  s->wall = L.wall;
+  s->pair = L.pair.ok;
+  int *dtcptr, *dtcase;
+  if ((st = upload(s, &dtcptr, L.tile_cptr)) || (st = upload(s, &dtcase, tile_case))) return st;
+  s->t.ntiles = L.ntiles;
+  s->t.per_xcd = (L.ntiles + kXcds - 1) / kXcds;
+  s->t.cptr = dtcptr;
+  s->t.tcase = dtcase;
+  if ((st = s->pair ? upload_paired(s, L) : upload_general(s, L))) return st;
 
   // per-case parameters
   std::vector<double> dt0(ncases), cfl(ncases), zero(ncases, 0.0);
@@ -2530,12 +2914,13 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
 
   const size_t n5 = (size_t)5 * nc;
   const size_t tsize = s->fp32 ? sizeof(float) : sizeof(double);
+  const size_t np = s->pair ? (size_t)s->m.ns : (size_t)nc;  // plane length of V, grad and fv
   if ((st = s->alloc(&s->U[0], n5)) || (st = s->alloc(&s->U[1], n5)) || (st = s->alloc(&s->R, n5)) ||
-      (st = s->alloc_bytes(&s->V, n5 * tsize)) || (st = s->alloc_bytes(&s->V2, n5 * tsize)) ||
-      (st = s->alloc_bytes(&s->grad, (size_t)kRec * nc * tsize)) ||
+      (st = s->alloc_bytes(&s->V, 5 * np * tsize)) || (st = s->alloc_bytes(&s->V2, 5 * np * tsize)) ||
+      (st = s->alloc_bytes(&s->grad, (size_t)kRec * np * tsize)) ||
       (s->opt.second_order_space && !s->opt.viscous &&
-       (st = s->alloc_bytes(&s->fv, (size_t)kMaxSlots * n5 * tsize))) ||
-      (st = s->alloc_bytes(&s->bc, (size_t)5 * std::max<long long>(nbf, 1) * tsize)) ||
+       (st = s->alloc_bytes(&s->fv, (size_t)kMaxSlots * 5 * np * tsize))) ||
+      (!s->pair && (st = s->alloc_bytes(&s->bc, (size_t)5 * std::max<long long>(nbf, 1) * tsize))) ||
       (st = s->alloc(&s->partial, (size_t)std::max(1, s->t.ntiles))) || (st = s->alloc(&s->counter, 1)) ||
       (st = s->alloc(&s->gsync, 4)) ||
       (st = s->alloc(&s->norm_partial, (size_t)5 * std::max(1, s->t.ntiles))) ||
@@ -2543,14 +2928,14 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
     return st;
   if (s->counting) return MA_OK;
   MA_HIP(hipMemsetAsync(s->R, 0, n5 * sizeof(double), s->stream));
-  MA_HIP(hipMemsetAsync(s->grad, 0, (size_t)kRec * nc * tsize, s->stream));
+  MA_HIP(hipMemsetAsync(s->grad, 0, (size_t)kRec * np * tsize, s->stream));
   MA_HIP(hipStreamSynchronize(s->stream));
   return MA_OK;
 }
 
 ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds) {
   RunPlan P;
-  ma_status st = plan_run(ncases, mds, s->shape, P);
+  ma_status st = plan_run(ncases, mds, s->shape, true, P);
   if (st) return st;
   return build_planned(s, P);
 }
@@ -2560,6 +2945,12 @@ inline int resident(const ma_solver* s, int per) {
   if (s->wg_per_cu <= 0) return per;
   return std::max(1, std::min(per, s->wg_per_cu * std::max(1, s->cus / kXcds)));
 }
+
+// Threads of a paired flux workgroup: one wavefront per 64-entry chunk of the
+// longest list up to kPairMaxThreads (small tiles: every face is evaluated in
+// one round, and a tile's cells, a third of its entries at most, fit the same
+// threads), else 4 wavefronts walking the chunks.
+inline int pair_threads(int max_faces) { return max_faces <= kPairMaxThreads ? max_faces : kTile; }
 
 template <bool SO, class Inv, class Visc, class Lim, class T>
 void run_stage(ma_solver* s, int irk) {
@@ -2578,7 +2969,8 @@ void run_stage(ma_solver* s, int irk) {
   T* Vn = static_cast<T*>((irk & 1) ? s->V : s->V2);
   if (irk == 0 && !s->v0_valid) {
     s->launch("k_prim", [&] {
-      hipLaunchKernelGGL(k_prim<T>, dim3(nb), dim3(kBlock), 0, s->stream, m.nc, Un, s->R, alpha[0], Vs);
+      hipLaunchKernelGGL(k_prim<T>, dim3(nb), dim3(kBlock), 0, s->stream, m, Un, s->R, alpha[0], Vs,
+                         s->pair ? 1 : 0);
     });
   }
   // inviscid second order: extrapolated face values for the flux kernel;
@@ -2588,6 +2980,31 @@ void run_stage(ma_solver* s, int irk) {
   Visc visc{effective_prandtl(s->opt)};
   const Inv inv{};
   const int nbf = m.nf - m.nif;
+  if (s->pair) {
+    // paired mesh: gradients, then the flux tiles with the boundary faces in them
+    if (SO || Visc::isViscous) {
+      s->launch(SO ? "k_grad_limiter" : "k_grad", [&] {
+        const int per = (nb + kXcds - 1) / kXcds;
+        hipLaunchKernelGGL((k_grad_pair<SO, FV, Lim, T>), dim3(per * kXcds), dim3(kBlock), 0, s->stream, m, s->nbr,
+                           static_cast<const T*>(Vs), FV ? nullptr : static_cast<T*>(s->grad),
+                           static_cast<T*>(s->fv), per);
+      });
+    }
+    constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
+    const auto kern = s->wg_per_cu > 0
+                          ? (s->wall ? k_flux_pair<SO, true, true, Inv, Visc, T> : k_flux_pair<SO, VW, true, Inv, Visc, T>)
+                          : (s->wall ? k_flux_pair<SO, true, false, Inv, Visc, T>
+                                     : k_flux_pair<SO, VW, false, Inv, Visc, T>);
+    s->launch("k_flux", [&] {
+      hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
+                         (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
+                         static_cast<const T*>(FV ? s->fv : s->grad), s->inflow_dev, irk == 0 ? Un : Uacc, Uacc,
+                         s->R, s->dt_dev, beta[irk], inv, visc, Un, Vn, irk < 3 ? alpha[irk + 1] : alpha[0],
+                         irk == 3 ? 1 : 0);
+    });
+    if (irk == 3) s->v0_valid = true;  // V now holds the next step's stage-0 primitives
+    return;
+  }
   if (SO || Visc::isViscous) {
     // the gradient kernel; its workgroups past the cell blocks compute the
     // boundary faces (k_bc's work, timed with it)
@@ -2689,9 +3106,9 @@ template <bool SO, class Inv, class Visc, class Lim, class T>
 ma_status run_persistent(ma_solver* s, int nsteps) {
   if (nsteps == 0) return MA_OK;
   constexpr bool FV = SO && !Visc::isViscous;
-  const auto kern = k_steps<SO, Inv, Visc, Lim, T>;
+  const auto kern = s->pair ? k_steps<SO, Inv, Visc, Lim, T, true> : k_steps<SO, Inv, Visc, Lim, T, false>;
   const size_t lds = std::max((size_t)s->t.max_faces * 5 * sizeof(T),
-                              FV ? (size_t)0 : (size_t)kBlock * kStageRow<T> * sizeof(T));
+                              FV || s->pair ? (size_t)0 : (size_t)kBlock * kStageRow<T> * sizeof(T));
   int coop = 0, per_cu = 0, wall_khz = 0;
   MA_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, s->device));
   if (!coop) return ma::fail(MA_ERR_UNSUPPORTED, "persistent steps: the device has no cooperative launch");
@@ -2811,11 +3228,11 @@ ma_status ensure_stage0_prims(ma_solver* s) {
   const int nc = s->m.nc;
   const double* Un = s->U[s->cur];
   if (s->fp32)
-    hipLaunchKernelGGL(k_prim<float>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, Un, s->R, 0.0,
-                       static_cast<float*>(s->V));
+    hipLaunchKernelGGL(k_prim<float>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, s->m, Un, s->R, 0.0,
+                       static_cast<float*>(s->V), s->pair ? 1 : 0);
   else
-    hipLaunchKernelGGL(k_prim<double>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, Un, s->R, 0.0,
-                       static_cast<double*>(s->V));
+    hipLaunchKernelGGL(k_prim<double>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, s->m, Un, s->R, 0.0,
+                       static_cast<double*>(s->V), s->pair ? 1 : 0);
   MA_HIP(hipGetLastError());
   s->v0_valid = true;
   return MA_OK;
@@ -2866,15 +3283,19 @@ ma_status download_aos(ma_solver* s, const S* dsrc, int ncomp, double* host) {
 template <class S>
 ma_status download_records(ma_solver* s, const S* dsrc, double* grad, double* lim) {
   const int nc = s->m.nc;
-  std::vector<S> tmp((size_t)kRec * nc);
+  const size_t np = s->pair ? (size_t)s->m.ns : (size_t)nc;
+  constexpr int W = 16 / (int)sizeof(S);
+  std::vector<S> tmp((size_t)kRec * np);
   MA_HIP(hipMemcpyAsync(tmp.data(), dsrc, tmp.size() * sizeof(S), hipMemcpyDeviceToHost, s->stream));
   MA_HIP(hipStreamSynchronize(s->stream));
   for (int c = 0; c < nc; ++c) {
-    const S* r = &tmp[(size_t)s->dev_of[c] * kRec];
+    const size_t d = s->dev_of[c];
+    // a block per cell, or planes of vectors on paired meshes
+    auto at = [&](int j) { return s->pair ? tmp[((size_t)(j / W) * np + d) * W + j % W] : tmp[d * kRec + j]; };
     if (grad)
-      for (int j = 0; j < 15; ++j) grad[(size_t)c * 15 + j] = r[j];
+      for (int j = 0; j < 15; ++j) grad[(size_t)c * 15 + j] = at(j);
     if (lim)
-      for (int k = 0; k < 5; ++k) lim[(size_t)c * 5 + k] = r[15 + k];
+      for (int k = 0; k < 5; ++k) lim[(size_t)c * 5 + k] = at(15 + k);
   }
   return MA_OK;
 }
@@ -2888,7 +3309,7 @@ extern "C" ma_status ma_batch_plan(int ncases, const ma_mesh_data* const* meshes
   RunPlan P;
   ma_status st = MA_OK;
   try {
-    st = plan_run(ncases, meshes, kDefaultShape, P);
+    st = plan_run(ncases, meshes, kDefaultShape, true, P);
   } catch (const std::bad_alloc&) {
     st = ma::fail(MA_ERR_NOMEM, "plan: out of host memory");
   }
@@ -3184,6 +3605,11 @@ template <class Lim, class T>
 void stage3_gradients(ma_solver* s) {
   const int nb = nblocks(s->m.nc);
   const int per = (nb + kXcds - 1) / kXcds;
+  if (s->pair) {
+    hipLaunchKernelGGL((k_grad_pair<true, true, Lim, T>), dim3(per * kXcds), dim3(kBlock), 0, s->stream, s->m, s->nbr,
+                       static_cast<const T*>(s->V2), static_cast<T*>(s->grad), static_cast<T*>(s->fv), per);
+    return;
+  }
   // no boundary-face blocks: the grid is the cell blocks alone
   hipLaunchKernelGGL((k_grad<true, true, Lim, T, 0, Inviscid>), dim3(per * kXcds), dim3(kBlock), 0, s->stream,
                      s->m, s->nbr, static_cast<const T*>(s->V2), static_cast<T*>(s->grad), static_cast<T*>(s->fv),
@@ -3492,7 +3918,7 @@ ma_status plan_layout_shared(const ma_mesh_data* md, const ma_options* opt, std:
   try {
     std::shared_ptr<LayoutPlan> lp = std::make_shared<LayoutPlan>();
     lp->shape = shape;
-    if ((st = plan_run(1, &md, shape, lp->P))) return st;
+    if ((st = plan_run(1, &md, shape, false, lp->P))) return st;
     const Layout& L = lp->P.L;
     lp->host_bytes = vbytes(L.dev_of) + vbytes(L.org_of) + vbytes(L.tile_cptr) + vbytes(L.tptr) +
                      vbytes(L.tfaces) + vbytes(L.slot) + vbytes(L.tslot) + vbytes(L.fl) + vbytes(L.fr) +
@@ -3657,7 +4083,8 @@ ma_status multi_set(Multi* M, ma_solver* const* cases, const int* parity, int n)
   M->cases.assign(cases, cases + n);
   for (int k = 0; k < n; ++k) {
     ma_solver* s = cases[k];
-    if (s->ncases != 1 || s->fp32 != M->fp32) return ma::fail(MA_ERR_INVALID, "multi: incompatible case");
+    if (s->ncases != 1 || s->fp32 != M->fp32 || s->pair)
+      return ma::fail(MA_ERR_INVALID, "multi: incompatible case");
     CaseView& v = M->h_views[b][k];
     v.m = s->m;
     v.t = s->t;
