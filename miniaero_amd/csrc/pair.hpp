@@ -668,7 +668,8 @@ __global__ __launch_bounds__(kPairMaxThreads) __attribute__((amdgpu_waves_per_eu
 void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restrict__ rec,
                  const Inflow* __restrict__ inflows, const double* Uacc_in, double* Uacc_out,
                  double* __restrict__ R, const double* __restrict__ dt_dev, double beta, Inv inv, Visc visc,
-                 const double* __restrict__ Un, T* Vnext, double alpha_next, int last) {
+                 const double* __restrict__ Un, T* Vnext, double alpha_next, int last,
+                 double* __restrict__ time_dev) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T* lds = reinterpret_cast<T*>(lds_raw);  // 5 planes of t.max_faces
   const int xcd = blockIdx.x % kXcds;
@@ -679,12 +680,14 @@ void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restr
       if (tile >= t.ntiles) break;  // uniform over the workgroup
       flux_tile_pair<SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
                                               beta, inv, visc, Un, Vnext, alpha_next, last);
+      advance_time(t, tile, dt_dev, time_dev);
       __syncthreads();  // the LDS is reused by the next tile
     }
   } else {
     const int tile = xcd * t.per_xcd + blockIdx.x / kXcds;
-    if (tile < t.ntiles)  // uniform over the workgroup
-      flux_tile_pair<SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
-                                              beta, inv, visc, Un, Vnext, alpha_next, last);
+    if (tile >= t.ntiles) return;  // uniform over the workgroup
+    flux_tile_pair<SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
+                                            beta, inv, visc, Un, Vnext, alpha_next, last);
+    advance_time(t, tile, dt_dev, time_dev);
   }
 }
