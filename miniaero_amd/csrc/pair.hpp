@@ -1,8 +1,11 @@
-// pair.hpp -- kernels for paired meshes: every cell has six faces, two per
-// axis, one on each side, and every face's area vector lies along an axis (box
-// meshes, stretched or not, as far as their area vectors are exactly axial;
-// find_pairs in solver.hip decides).  Solvers and batches use them where every
-// case qualifies; the served form does not (plan_run).
+// pair.hpp -- kernels for meshes of cells with six faces each (find_pairs in
+// solver.hip has the conditions).  Two forms: axial meshes, where a cell has
+// two faces per axis, one on each side, and every area vector lies along an
+// axis (box meshes, stretched or not), and skew meshes (kSkew: ramps, boxes
+// whose area vectors carry rounding noise), where the slots stay in slot order
+// and faces along no axis are a class of their own in the tiles' lists.
+// Solvers and batches use them where every case qualifies with the same form;
+// the served form does not (plan_run).
 // Included by solver.hip inside its anonymous namespace.
 //
 // What bounds the general kernels on such meshes is the vector memory path of
@@ -15,7 +18,7 @@
 // the data return busy 91%).  So the work is ordered by axis, and the arrays
 // are laid out for 16-byte loads of consecutive cells:
 //
-//   gradients    a cell's slots are (low, high) along x, y, z.  Only the two
+//   gradients    axial: a cell's slots are (low, high) along x, y, z.  Only the two
 //                faces of an axis contribute to that component of the
 //                gradient, and two terms add to the same sum in either order,
 //                so the reference's summation order is kept without following
@@ -42,6 +45,8 @@
 // viscous 211 x 127 x 45 plate 99 -> 53, 139 -> 117; 48 batched FP32 shock
 // tubes 320 -> 194, 384 -> 318; 4096-cell FP64 plate 10.3 -> 5.3, 14.3 -> 7.3;
 // first-order 64 x 16 x 16 shock tube 14.1 with its boundary launch -> 5.2.
+// Skew: FP64 321 x 157 x 11 ramp 126 -> 74, 120 -> 97; 2240-cell ramp 13.1 -> 7.0,
+// 10.5 -> 8.0 (its boundary faces were in the gradient launch).
 // At 2.1M cells the flux kernel still has its address and data units busy 89%
 // and 92% (VALU 37%), the gradient kernel its data return 86%.
 //
@@ -54,6 +59,8 @@
 // told to fit.
 template <class Visc, class T>
 constexpr int kPairFluxWaves = sizeof(T) == 4 ? 5 : Visc::isViscous ? 3 : 4;
+
+constexpr int kSkewFace = 3;  // class of a tile's chunk of faces that are along no axis
 
 constexpr int kPairMaxThreads = 384;  // flux workgroup: up to 6 wavefronts (see pair_threads)
 
@@ -171,25 +178,40 @@ struct TameCheck {
   __device__ __forceinline__ bool tiny() const { return kDiv && e < (kD ? -740 : -40); }
 };
 
-// Slot geometry of record i: the outward area component along the face's axis
-// and x_f - x_c, 4 values as whole vectors, planes of m.nsrec.  (Face geometry,
-// m.ptab: the area component, x_f - x_left, x_f - x_right and a zero, 8 values,
-// planes of m.nfrec.)  Records are numbered in the order the kernels meet
-// them, so the lanes of a load read consecutive records where they differ.
+// Slot geometry of record i (m.stab): the outward area component along the
+// face's axis and x_f - x_c, 4 values as whole vectors in planes of m.nsrec; on
+// skew meshes the outward area vector and x_f - x_c, 6 values.  (Face geometry,
+// m.ptab, planes of m.nfrec: the area component, x_f - x_left, x_f - x_right,
+// 7 values; skew: the area vector in front, 9.)  Records are numbered in the
+// order the kernels meet them, so the lanes of a load read consecutive records
+// where they differ.
+template <bool kSkew>
+constexpr int kAreaVals = kSkew ? 3 : 1;
+template <bool kSkew, class T>
+constexpr int kSlotVecs = (kAreaVals<kSkew> + 3 + kVec<T> - 1) / kVec<T>;
+template <bool kSkew, class T>
+constexpr int kFaceVecs = (kAreaVals<kSkew> + 6 + kVec<T> - 1) / kVec<T>;
+// vectors j0 to j1 - 1 of record i
 template <class T>
-__device__ __forceinline__ void slot_geo(const DevMesh& m, unsigned i, T* q) {
+__device__ __forceinline__ void slot_vecs(const DevMesh& m, unsigned i, int j0, int j1, T* q) {
 #pragma unroll
-  for (int j = 0; j < 4 / kVec<T>; ++j) get_vec(static_cast<const T*>(m.stab), j, m.nsrec, i, q + j * kVec<T>);
+  for (int j = j0; j < j1; ++j) get_vec(static_cast<const T*>(m.stab), j, m.nsrec, i, q + j * kVec<T>);
 }
 
 // A cell's neighbours (itself across a boundary face) and slot records: 3
-// planes of int4, neighbours 0 to 5 then records 0 to 5.
+// planes of int4, neighbours 0 to 5 then records 0 to 5 (skew meshes: with the
+// cell's side of the face, 1 the right one, above kCellBits).
+template <bool kSkew>
 __device__ __forceinline__ void slot_ids(const DevMesh& m, const int* __restrict__ nbr, unsigned c, unsigned* nb,
                                          unsigned* ent) {
   const int4* p = reinterpret_cast<const int4*>(nbr);
   const int4 a = at(p, c * 16u), b = at(p + m.ns, c * 16u), d = at(p + (size_t)2 * m.ns, c * 16u);
   nb[0] = a.x, nb[1] = a.y, nb[2] = a.z, nb[3] = a.w, nb[4] = b.x, nb[5] = b.y;
   ent[0] = b.z, ent[1] = b.w, ent[2] = d.x, ent[3] = d.y, ent[4] = d.z, ent[5] = d.w;
+  if constexpr (kSkew) {
+#pragma unroll
+    for (int s = 0; s < kMaxSlots; ++s) ent[s] = (unsigned)cell_of((int)ent[s]);
+  }
 }
 
 // Value k of element i in five-value planes, and of a record in 20-value planes.
@@ -204,22 +226,27 @@ __device__ __forceinline__ size_t rec_at(int k, int n, unsigned i) {
 
 // Gradients of the velocities with full divisions, for a wavefront with tiny
 // ones (TameCheck): replaces r[3] to r[11].
-template <class T>
+template <bool kSkew, class T>
 __device__ __forceinline__ void tiny_gradients(const DevMesh& m, const int* __restrict__ nbr, const T* __restrict__ V,
                                                T vol, unsigned c, const T* vc, T* r) {
   unsigned ent[kMaxSlots], nb[kMaxSlots];
-  slot_ids(m, nbr, c, nb, ent);
+  slot_ids<kSkew>(m, nbr, c, nb, ent);
 #pragma unroll
   for (int s = 0; s < kMaxSlots; ++s) {
     T vn[5];
     get_five(V, m.ns, nb[s], vn);
-    const T sn = static_cast<const T*>(m.stab)[(size_t)ent[s] * kVec<T>];
+    T q[kSlotVecs<kSkew, T> * kVec<T>];
+    slot_vecs(m, ent[s], 0, (kAreaVals<kSkew> + kVec<T> - 1) / kVec<T>, q);
 #pragma unroll
     for (int k = 1; k < 4; ++k) {
-      const T t = T(0.5) * (vc[k] + vn[k]) * sn;
-      const T q = T(double(t) / double(vol));  // correctly rounded, as in grad_pair_slow
-      T& g = r[3 * k + s / 2];
-      g = (s & 1) ? g + q : q;
+      const T base = T(0.5) * (vc[k] + vn[k]);
+#pragma unroll
+      for (int d = 0; d < kAreaVals<kSkew>; ++d) {
+        const T t = base * q[d];
+        const T x = T(double(t) / double(vol));  // correctly rounded, as in grad_pair_slow
+        T& g = r[3 * k + (kSkew ? d : s / 2)];
+        g = s > (kSkew ? 0 : s / 2 * 2) ? g + x : x;
+      }
     }
   }
 }
@@ -228,11 +255,12 @@ __device__ __forceinline__ void tiny_gradients(const DevMesh& m, const int* __re
 // stencil outside the tame range: one variable at a time (few registers: the
 // fast path sets the kernel's occupancy), full divisions, the off-axis terms
 // of the Green-Gauss sums as 0 * x.  Same values as grad_cell's general loop.
-template <bool SO, bool FV, class Limiter, class T>
+template <bool kSkew, bool SO, bool FV, class Limiter, class T>
 __device__ void grad_pair_slow(const DevMesh& m, const int* __restrict__ nbr, const T* __restrict__ V,
                                T* __restrict__ rec, T* __restrict__ fv, unsigned c) {
   const int n = m.ns;
   auto id = [&](int k) { return (unsigned)nbr[((size_t)(k / 4) * n + c) * 4 + k % 4]; };  // see slot_ids
+  auto record = [&](int s) { return kSkew ? (unsigned)cell_of((int)id(6 + s)) : id(6 + s); };
   const T vol = T(m.vol[c]);
   const T rvol = T(1) / vol;
 #pragma unroll 1
@@ -242,14 +270,18 @@ __device__ void grad_pair_slow(const DevMesh& m, const int* __restrict__ nbr, co
 #pragma unroll 1
     for (int s = 0; s < kMaxSlots; ++s) {
       const T vn = V[five_at<T>(k, n, id(s))];
-      const T sn = static_cast<const T*>(m.stab)[(size_t)id(6 + s) * kVec<T>];
-      // the low slot's face has the cell on its right (a boundary face's two
-      // values are the same)
-      const T vl = (s & 1) ? vc : vn, vr = (s & 1) ? vn : vc;
+      T q[kSlotVecs<kSkew, T> * kVec<T>];
+      slot_vecs(m, record(s), 0, (kAreaVals<kSkew> + kVec<T> - 1) / kVec<T>, q);
+      // which side the cell is on: an axial mesh's low slots have it on their
+      // right, and a skew mesh's order of the two decides only which of two
+      // values one of which is NaN is kept, so it is looked up (a boundary
+      // face's two values are the same)
+      const bool left = kSkew ? !slot_of((int)id(6 + s)) : (s & 1) != 0;
+      const T vl = left ? vc : vn, vr = left ? vn : vc;
       const T base = T(0.5) * (vl + vr);
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const T gg = base * (d == s / 2 ? sn : T(0));
+        const T gg = base * (kSkew ? q[d] : d == s / 2 ? q[0] : T(0));
         if constexpr (sizeof(T) == 8) g[d] += gg / vol;
         else if constexpr (FV) g[d] += T(double(gg) / double(vol));  // correctly rounded
         else g[d] += gg * rvol;
@@ -262,8 +294,9 @@ __device__ void grad_pair_slow(const DevMesh& m, const int* __restrict__ nbr, co
     if constexpr (SO) {
 #pragma unroll 1
       for (int s = 0; s < kMaxSlots; ++s) {
-        T q[4];
-        slot_geo(m, id(6 + s), q);
+        T qs[kSlotVecs<kSkew, T> * kVec<T>];
+        slot_vecs(m, record(s), 0, kSlotVecs<kSkew, T>, qs);
+        const T* q = qs + kAreaVals<kSkew> - 1;
         const T dist = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
         const T du = q[1] * g[0] + q[2] * g[1] + q[3] * g[2];
         lim = ma::smin(lim, Limiter::limit(mx - vc, mn - vc, du, dist));
@@ -272,8 +305,9 @@ __device__ void grad_pair_slow(const DevMesh& m, const int* __restrict__ nbr, co
     if constexpr (FV) {
 #pragma unroll 1
       for (int s = 0; s < kMaxSlots; ++s) {
-        T q[4];
-        slot_geo(m, id(6 + s), q);
+        T qs[kSlotVecs<kSkew, T> * kVec<T>];
+        slot_vecs(m, record(s), 0, kSlotVecs<kSkew, T>, qs);
+        const T* q = qs + kAreaVals<kSkew> - 1;
         const T du = q[1] * g[0] + q[2] * g[1] + q[3] * g[2];
         fv[(size_t)5 * s * n + five_at<T>(k, n, c)] = vc + du * lim;
       }
@@ -294,13 +328,14 @@ __device__ void grad_pair_slow(const DevMesh& m, const int* __restrict__ nbr, co
 // reciprocal, no terms of the zero area components, one instruction per
 // minimum and maximum (the minimum over the faces of min(v_L, v_R) is the
 // minimum of the cell and its neighbours), short quotients in the limiter.
-template <bool SO, bool FV, class Limiter, class T>
+template <bool kSkew, bool SO, bool FV, class Limiter, class T>
 __device__ __forceinline__ void grad_pair(const DevMesh& m, const int* __restrict__ nbr, const T* __restrict__ V,
                                           T* __restrict__ rec, T* __restrict__ fv, unsigned c) {
   const int n = m.ns;
   unsigned ent[kMaxSlots], nb[kMaxSlots];
-  slot_ids(m, nbr, c, nb, ent);
-  T vc[5], geo[kMaxSlots][4], mn[5], mx[5];
+  slot_ids<kSkew>(m, nbr, c, nb, ent);
+  constexpr int A = kAreaVals<kSkew>, AV = (A + kVec<T> - 1) / kVec<T>, SV = kSlotVecs<kSkew, T>;
+  T vc[5], geo[kMaxSlots][SV * kVec<T>], mn[5], mx[5];
   get_five(V, n, c, vc);
   const T vol = T(at(m.vol, c * 8u));
   // the reciprocal, correctly rounded (div_by needs that); the FP32 record
@@ -315,30 +350,34 @@ __device__ __forceinline__ void grad_pair(const DevMesh& m, const int* __restric
 #pragma unroll
   for (int s = 0; s < kMaxSlots; ++s) {
     T vn[5];
-    get_vec(static_cast<const T*>(m.stab), 0, m.nsrec, ent[s], geo[s]);
+    slot_vecs(m, ent[s], 0, AV, geo[s]);
     get_five(V, n, nb[s], vn);
     tame.take(vn);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       mn[k] = vmin(mn[k], vn[k]);
       mx[k] = vmax(mx[k], vn[k]);
-      const T t = T(0.5) * (vc[k] + vn[k]) * geo[s][0];
-      const T q = kMul ? t * rvol : ma::div_by(t, vol, rvol);
-      T& g = r[3 * k + s / 2];
-      g = (s & 1) ? g + q : q;
+      const T base = T(0.5) * (vc[k] + vn[k]);
+#pragma unroll
+      for (int d = 0; d < A; ++d) {
+        const T t = base * geo[s][d];
+        const T q = kMul ? t * rvol : ma::div_by(t, vol, rvol);
+        T& g = r[3 * k + (kSkew ? d : s / 2)];
+        g = s > (kSkew ? 0 : s / 2 * 2) ? g + q : q;
+      }
     }
   }
   if (__any(tame.bad(mn, mx))) {
     // through an opaque index: sharing loads with the fast path would keep
     // their registers over it (155 instead of 73 in the FP32 record form)
     asm volatile("" : "+v"(c));
-    grad_pair_slow<SO, FV, Limiter, T>(m, nbr, V, rec, fv, c);
+    grad_pair_slow<kSkew, SO, FV, Limiter, T>(m, nbr, V, rec, fv, c);
     return;
   }
   if (!kMul && __any(tame.tiny())) {
     unsigned c2 = c;
     asm volatile("" : "+v"(c2));
-    tiny_gradients(m, nbr, V, vol, c2, vc, r);
+    tiny_gradients<kSkew>(m, nbr, V, vol, c2, vc, r);
   }
   T dus[FV ? kMaxSlots : 1][5];
 #pragma unroll
@@ -350,8 +389,8 @@ __device__ __forceinline__ void grad_pair(const DevMesh& m, const int* __restric
   if constexpr (SO) {
 #pragma unroll
     for (int s = 0; s < kMaxSlots; ++s) {
-      T* q = geo[s];
-      if constexpr (kVec<T> == 2) get_vec(static_cast<const T*>(m.stab), 1, m.nsrec, ent[s], q + 2);
+      const T* q = geo[s] + A - 1;
+      slot_vecs(m, ent[s], AV, SV, geo[s]);
       const T dist = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
 #pragma unroll
       for (int k = 0; k < 5; ++k) {
@@ -376,13 +415,13 @@ __device__ __forceinline__ void grad_pair(const DevMesh& m, const int* __restric
   }
 }
 
-template <bool SO, bool FV, class Limiter, class T>
+template <bool kSkew, bool SO, bool FV, class Limiter, class T>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGradWaves<SO, T>)))
 void k_grad_pair(DevMesh m, const int* __restrict__ nbr, const T* __restrict__ V, T* __restrict__ rec,
                  T* __restrict__ fv, int per_xcd) {
   const int b = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;  // XCD-aware, see k_flux
   const int c = b * kBlock + threadIdx.x;
-  if (c < m.nc) grad_pair<SO, FV, Limiter, T>(m, nbr, V, rec, fv, (unsigned)c);
+  if (c < m.nc) grad_pair<kSkew, SO, FV, Limiter, T>(m, nbr, V, rec, fv, (unsigned)c);
 }
 
 // State outside a boundary face of kind MA_BC_* whose area vector is p along
@@ -474,14 +513,64 @@ __device__ __forceinline__ void axis_flux(const T* vl, const T* vright, const T 
   }
 }
 
+// Flux of a face of any area vector a (class kSkewFace of a tile's list): the
+// general kernels' operations, with axis_flux's arguments.
+template <bool kWall, class Inv, class Visc, class T>
+__device__ __forceinline__ void skew_flux(const T* vl, const T* vright, const T gavg[5][3], const T* a, int kind,
+                                          T winv, const Inflow* __restrict__ inflow, const Inv& inv,
+                                          const Visc& visc, T* F) {
+  const ma::FaceFrameT<T> fr = ma::frame_from_area_t<T>(a);
+  T vr[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) vr[k] = vright[k];
+  if (kind == MA_BC_TANGENT || kind == MA_BC_NOSLIP) ma::mirror_state(vl, fr, vr);
+  if (kind == MA_BC_INFLOW) {
+    double vi[5];
+    ma::primitives(inflow->U, vi);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vr[k] = T(vi[k]);
+  }
+  T f[5];
+  bool sub = false;
+  if constexpr (Visc::isViscous || kWall) {
+    T vf[5], gf[5][3];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      vf[k] = T(0.5) * (vl[k] + vr[k]);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) gf[k][d] = Visc::isViscous ? gavg[k][d] : T(0);
+    }
+    if (kind == MA_BC_NOSLIP) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        vf[k] = k == 0 || k == 4 ? vl[k] : T(0);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) gf[k][d] = (vf[k] - vl[k]) * fr.nu[d] * winv;
+      }
+    }
+    sub = kind == MA_BC_NOSLIP || (Visc::isViscous && !kind);
+    if constexpr (Visc::isViscous) visc.compute_flux(gf, vf, fr.n, f);
+    else if (sub) ma::NewtonianViscousFlux{visc.prandtl}.compute_flux(gf, vf, fr.n, f);
+  }
+  ma::inviscid_flux(inv, vl, vr, F, fr);
+  if constexpr (Visc::isViscous || kWall) {
+    if (sub) {
+#pragma unroll
+      for (int k = 1; k < 5; ++k) F[k] -= f[k];  // (component 0 of a viscous flux is 0)
+    }
+  }
+}
+
 // Flux through one entry of a tile's face list along axis D (uniform over the
 // wavefront): interior_flux for an internal face (cells L and Rr), the
 // boundary policies for a boundary face (Rr < 0: ~Rr = boundary-face number
 // << 2 | kind - 1; the cell's contribution is minus the returned flux, as on
 // the left of an internal face).  kWall: the run may have no-slip faces, whose
 // viscous flux is there in inviscid runs too.  Loads and extrapolation are
-// common to the axes; only the flux arithmetic is per axis.
-template <bool SO, bool kWall, class Inv, class Visc, class T>
+// common to the axes; only the flux arithmetic is per axis.  Skew meshes: D may
+// be kSkewFace; Rr and gid carry the face's slots in the right and left cell
+// above kCellBits.
+template <bool kSkew, bool SO, bool kWall, class Inv, class Visc, class T>
 __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict__ V, const T* __restrict__ rec,
                                           const T* __restrict__ fv, const Inflow* __restrict__ inflow, int D,
                                           unsigned L, int Rr, int gid, const Inv& inv, const Visc& visc, T* F) {
@@ -493,18 +582,20 @@ __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict_
   int n = m.ns;
   asm volatile("" : "+s"(n));
   const bool bnd = Rr < 0;
-  const unsigned Rc = bnd ? L : (unsigned)Rr;
-  T vl[5], vr[5], geo[8];
+  const unsigned Rc = bnd ? L : (unsigned)(kSkew ? cell_of(Rr) : Rr);
+  constexpr int A = kAreaVals<kSkew>;
+  T vl[5], vr[5], geo[kFaceVecs<kSkew, T> * W];
   if constexpr (FV) {
     // the left cell's high face and the right cell's low face; a boundary
     // face's cell state
-    const T* lo = fv + (size_t)(10 * D) * n;
+    const T* lo = fv + (size_t)(kSkew ? 5 * slot_of(bnd ? 0 : Rr) : 10 * D) * n;
+    const T* hi = kSkew ? fv + (size_t)(5 * slot_of(gid)) * n : lo + (size_t)5 * n;
     if (bnd) {
       get_five(V, n, L, vl);
 #pragma unroll
       for (int k = 0; k < 5; ++k) vr[k] = vl[k];
     } else {
-      get_five(lo + (size_t)5 * n, n, L, vl);
+      get_five(hi, n, L, vl);
       get_five(lo, n, Rc, vr);
     }
   } else {
@@ -512,9 +603,9 @@ __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict_
     get_five(V, n, Rc, vr);
   }
 #pragma unroll
-  for (int j = 0; j < (kRecon ? 8 / W : 1); ++j)
-    get_vec(static_cast<const T*>(m.ptab), j, m.nfrec, (unsigned)gid, geo + j * W);
-  const T p = geo[0];
+  for (int j = 0; j < (kRecon ? kFaceVecs<kSkew, T> : (A + W - 1) / W); ++j)
+    get_vec(static_cast<const T*>(m.ptab), j, m.nfrec, (unsigned)(kSkew ? cell_of(gid) : gid), geo + j * W);
+  const T* q = geo + A;  // displacements
   T gf[5][3];
   if constexpr (kVisc) {
     constexpr int j0 = kRecon ? 0 : 3 / W, j1 = kRecon ? kRec / W : (15 + W - 1) / W;  // vectors used
@@ -531,12 +622,12 @@ __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict_
       for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(rl[15 + k]), "+v"(rr[15 + k]));
 #pragma unroll
       for (int d = 0; d < 3; ++d)
-        asm volatile("" : "+v"(geo[1 + d]), "+v"(geo[4 + d]), "+v"(rl[d]), "+v"(rr[d]));
+        asm volatile("" : "+v"(geo[A + d]), "+v"(geo[A + 3 + d]), "+v"(rl[d]), "+v"(rr[d]));
       if (!bnd) {
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
-          const T tl = geo[1] * rl[3 * k] + geo[2] * rl[3 * k + 1] + geo[3] * rl[3 * k + 2];
-          const T tr = geo[4] * rr[3 * k] + geo[5] * rr[3 * k + 1] + geo[6] * rr[3 * k + 2];
+          const T tl = q[0] * rl[3 * k] + q[1] * rl[3 * k + 1] + q[2] * rl[3 * k + 2];
+          const T tr = q[3] * rr[3 * k] + q[4] * rr[3 * k + 1] + q[5] * rr[3 * k + 2];
           vl[k] = vl[k] + tl * rl[15 + k];
           vr[k] = vr[k] + tr * rr[15 + k];
         }
@@ -550,9 +641,10 @@ __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict_
   const int kind = bnd ? (~Rr & 3) + 1 : 0;
   T winv = T(0);
   if (kWall && kind == MA_BC_NOSLIP) winv = T(m.fwall[m.nif + (~Rr >> 2)]);
-  if (D == 0) axis_flux<0, SO, kWall>(vl, vr, gf, p, kind, winv, inflow, inv, visc, F);
-  else if (D == 1) axis_flux<1, SO, kWall>(vl, vr, gf, p, kind, winv, inflow, inv, visc, F);
-  else axis_flux<2, SO, kWall>(vl, vr, gf, p, kind, winv, inflow, inv, visc, F);
+  if (kSkew && D == kSkewFace) skew_flux<kWall>(vl, vr, gf, geo, kind, winv, inflow, inv, visc, F);
+  else if (D == 0) axis_flux<0, SO, kWall>(vl, vr, gf, geo[0], kind, winv, inflow, inv, visc, F);
+  else if (D == 1) axis_flux<1, SO, kWall>(vl, vr, gf, geo[kSkew ? 1 : 0], kind, winv, inflow, inv, visc, F);
+  else axis_flux<2, SO, kWall>(vl, vr, gf, geo[kSkew ? 2 : 0], kind, winv, inflow, inv, visc, F);
 }
 
 // Second phase of a paired tile: every cell adds its face fluxes from LDS (5
@@ -620,7 +712,7 @@ __device__ __forceinline__ void update_tile_pair(const DevMesh& m, const TileMap
 // wavefront w takes chunks w, w + waves, ...  Slot entries are LDS index << 1 |
 // side in the reference's summation order with the boundary faces last, in
 // kind order.
-template <bool SO, bool kWall, class Inv, class Visc, class T>
+template <bool kSkew, bool SO, bool kWall, class Inv, class Visc, class T>
 __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& t, int tile, T* lds,
                                                const T* __restrict__ V, const T* __restrict__ rec,
                                                const T* __restrict__ fv, const Inflow* __restrict__ inflows,
@@ -651,7 +743,7 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
     const int D = __builtin_amdgcn_readfirstlane(c.x) >> kCellBits;  // (a chunk starts with a face)
     if (c.x < 0) continue;  // padding
     T F[5];
-    pair_flux<SO, kWall>(m, V, rec, fv, inflow, D, (unsigned)cell_of(c.x), c.y, gc, inv, visc, F);
+    pair_flux<kSkew, SO, kWall>(m, V, rec, fv, inflow, D, (unsigned)cell_of(c.x), c.y, gc, inv, visc, F);
 #pragma unroll
     for (int k = 0; k < 5; ++k) lds[k * mf + q + lane] = F[k];
   }
@@ -663,7 +755,7 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
 // otherwise one tile per workgroup, a form of its own because the walk's
 // loop-carried values cost the FP64 viscous kernel spills and the FP64 inviscid
 // one ten registers.
-template <bool SO, bool kWall, bool kWalk, class Inv, class Visc, class T>
+template <bool kSkew, bool SO, bool kWall, bool kWalk, class Inv, class Visc, class T>
 __global__ __launch_bounds__(kPairMaxThreads) __attribute__((amdgpu_waves_per_eu(kPairFluxWaves<Visc, T>)))
 void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restrict__ rec,
                  const Inflow* __restrict__ inflows, const double* Uacc_in, double* Uacc_out,
@@ -678,7 +770,7 @@ void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restr
     for (int j = blockIdx.x / kXcds; j < t.per_xcd; j += stride) {
       const int tile = xcd * t.per_xcd + j;
       if (tile >= t.ntiles) break;  // uniform over the workgroup
-      flux_tile_pair<SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
+      flux_tile_pair<kSkew, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
                                               beta, inv, visc, Un, Vnext, alpha_next, last);
       advance_time(t, tile, dt_dev, time_dev);
       __syncthreads();  // the LDS is reused by the next tile
@@ -686,7 +778,7 @@ void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restr
   } else {
     const int tile = xcd * t.per_xcd + blockIdx.x / kXcds;
     if (tile >= t.ntiles) return;  // uniform over the workgroup
-    flux_tile_pair<SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
+    flux_tile_pair<kSkew, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
                                             beta, inv, visc, Un, Vnext, alpha_next, last);
     advance_time(t, tile, dt_dev, time_dev);
   }

@@ -26,8 +26,9 @@
 //            V buffer (stage 3: the next step's, from the new U; R itself
 //            is stored on stage 3 only)
 //
-// Meshes whose faces all lie along the axes run k_grad_pair and k_flux_pair
-// instead, with their own layout and no boundary launch (pair.hpp).
+// Meshes whose cells all have six faces run k_grad_pair and k_flux_pair
+// instead, with their own layout and no boundary launch (pair.hpp); the
+// kernels above are for other meshes, mixed batches and the served form.
 //
 // Determinism and parity.  The reference scatters face results into cells
 // with atomics; with one thread the additions land in a fixed order: internal
@@ -1390,7 +1391,8 @@ __device__ __forceinline__ bool grid_sync(unsigned* gsync, unsigned& gen, long l
 template <bool kViscousSO, class T>
 constexpr int kStepsWaves = sizeof(T) == 8 ? (kViscousSO ? 1 : 2) : 1;
 
-template <bool SO, class Inv, class Visc, class Lim, class T, bool kPair>
+// kPair: 0 the general kernels' phases, 1 the paired ones, 2 those for skew meshes
+template <bool SO, class Inv, class Visc, class Lim, class T, int kPair>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(kStepsWaves<SO && Visc::isViscous, T>)))
 void k_steps(PersistArgs a, Inv inv, Visc visc) {
   // TimeSolverExplicitRK4.h:187-195: alpha = {0, 1/2, 1/2, 1}, beta = {1/6,
@@ -1428,7 +1430,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
     if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
     if (it == 0 && a.prim0) {
       for (int c = blockIdx.x * kTile + threadIdx.x; c < m.nc; c += G * kTile)
-        prim_cell_any(m, Un, a.R, 0.0, static_cast<T*>(a.V[0]), c, kPair);
+        prim_cell_any(m, Un, a.R, 0.0, static_cast<T*>(a.V[0]), c, kPair != 0);
       if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
     }
     for (int irk = 0; irk < 4; ++irk) {
@@ -1441,7 +1443,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
           if (b * kBlock >= m.nc) break;  // uniform over the workgroup
           const int c = b * kBlock + threadIdx.x;
           if constexpr (kPair) {
-            if (c < m.nc) grad_pair<SO, FV, Lim, T>(m, a.nbr, Vs, rec, static_cast<T*>(a.fv), (unsigned)c);
+            if (c < m.nc) grad_pair<kPair == 2, SO, FV, Lim, T>(m, a.nbr, Vs, rec, static_cast<T*>(a.fv), (unsigned)c);
             continue;
           }
           T out[kRec];
@@ -1465,7 +1467,8 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
         const int tile = xcd * a.t.per_xcd + j;
         if (tile >= a.t.ntiles) break;  // uniform over the workgroup
         if constexpr (kPair)
-          flux_tile_pair<SO, true, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, a.inflow, irk == 0 ? Un : Uacc,
+          flux_tile_pair<kPair == 2, SO, true, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, a.inflow,
+                                                             irk == 0 ? Un : Uacc,
                                                  Uacc, a.R, a.dt, beta(irk), inv, visc, Un, Vn, alpha_next(irk),
                                                  irk == 3 ? 1 : 0);
         else
@@ -1535,6 +1538,7 @@ struct ma_solver {
   void* fv = nullptr;  // kMaxSlots x 5 planes: extrapolated face values (inviscid second order)
   bool fp32 = false;
   bool pair = false;          // runs the paired-mesh kernels and array layouts (pair.hpp)
+  bool skew = false;          // their forms for meshes with faces along no axis
   bool wall = false;          // some boundary face is a no-slip wall
   // Cases (independent meshes stepped together; a plain run is one case).
   int ncases = 1;
@@ -1789,8 +1793,10 @@ void cell_order(const ma_mesh_data* md, const TileShape& shape, std::vector<int>
 // and tile tables; ok when the mesh is paired (find_pairs).
 struct PairPlan {
   bool ok = false;
+  bool fp32 = true;                      // in the FP32 form as well
+  bool skew = false;                     // some face is along no axis: slots in slot order, kSkewFace chunks
   int max_faces = 64;                    // longest tile list, padding included
-  std::vector<int> nbr, ent;             // kMaxSlots planes of nc: (low, high) along x, y, z
+  std::vector<int> nbr, ent;             // kMaxSlots planes of nc: (low, high) along x, y, z; skew: as L.slot
   std::vector<int> srec, frec;           // slot record -> geometry record << 1 | side; face record -> geometry record
   std::vector<int> ptr, lr, gid;         // tile lists, lr 2 per entry (see flux_tile_pair)
   std::vector<unsigned short> slot;      // kMaxSlots planes of nc: list index << 1 | side
@@ -1823,12 +1829,14 @@ ma_status validate_pairs(const Layout& L) {
   const int nc = L.nc, ntiles = L.ntiles;
   const size_t ng = L.geo.size() / kGeoVals;
   auto bad = [](const char* what) { return ma::fail(MA_ERR_INVALID, std::string("layout: paired ") + what); };
+  // skew meshes keep a slot or a side above kCellBits
+  auto low = [&](int x) { return P.skew && x >= 0 ? x & ((1 << kCellBits) - 1) : x; };
   if (P.nbr.size() != (size_t)kMaxSlots * nc || P.ent.size() != P.nbr.size() || P.slot.size() != P.nbr.size() ||
       (int)P.ptr.size() != ntiles + 1 || P.gid.size() * 2 != P.lr.size() ||
       (size_t)P.ptr[ntiles] > P.gid.size() || (size_t)P.max_faces * 5 * sizeof(double) > 65536)
     return bad("sizes");
   for (size_t i = 0; i < P.nbr.size(); ++i)
-    if (P.nbr[i] < 0 || P.nbr[i] >= nc || P.ent[i] < 0 || (size_t)P.ent[i] >= P.srec.size()) return bad("slots");
+    if (P.nbr[i] < 0 || P.nbr[i] >= nc || P.ent[i] < 0 || (size_t)low(P.ent[i]) >= P.srec.size()) return bad("slots");
   for (int x : P.srec)
     if (x < 0 || (size_t)(x >> 1) >= ng) return bad("slot records");
   for (int x : P.frec)
@@ -1838,17 +1846,20 @@ ma_status validate_pairs(const Layout& L) {
     if (n < 0 || n % 64 || n > P.max_faces) return bad("tile lists");
     for (int q = f0; q < f0 + n; ++q) {
       const int x = P.lr[2 * (size_t)q], r = P.lr[2 * (size_t)q + 1], l = x < 0 ? -1 : x & ((1 << kCellBits) - 1);
-      if (x >= 0 ? x >> kCellBits != P.lr[2 * (size_t)(q - (q - f0) % 64)] >> kCellBits || x >> kCellBits > 2
+      if (x >= 0 ? x >> kCellBits != P.lr[2 * (size_t)(q - (q - f0) % 64)] >> kCellBits || x >> kCellBits > (P.skew ? 3 : 2)
                  : (q - f0) % 64 == 0)
         return bad("tile chunks");
-      if (l >= nc || r >= nc || P.gid[q] < 0 || (size_t)P.gid[q] >= P.frec.size() || (l >= 0 && r < 0 && (~r >> 2) >= L.nbf))
+      if (l >= nc || low(r) >= nc || P.gid[q] < 0 || (size_t)low(P.gid[q]) >= P.frec.size() ||
+          (l >= 0 && r < 0 && (~r >> 2) >= L.nbf))
         return bad("tile faces");
+      if (P.skew && l >= 0 && r >= 0 && (r >> kCellBits >= kMaxSlots || P.gid[q] >> kCellBits >= kMaxSlots))
+        return bad("tile face slots");
     }
     for (int c = L.tile_cptr[b]; c < L.tile_cptr[b + 1]; ++c)
       for (int s = 0; s < kMaxSlots; ++s) {
         const int e = P.slot[(size_t)s * nc + c], j = e >> 1;
         if (j >= n || P.lr[2 * (size_t)(f0 + j)] < 0 ||
-            ((e & 1) ? P.lr[2 * (size_t)(f0 + j) + 1] : P.lr[2 * (size_t)(f0 + j)] & ((1 << kCellBits) - 1)) != c)
+            ((e & 1) ? low(P.lr[2 * (size_t)(f0 + j) + 1]) : P.lr[2 * (size_t)(f0 + j)] & ((1 << kCellBits) - 1)) != c)
           return bad("tile slots");
       }
   }
@@ -1964,9 +1975,14 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
   M.wall = false;
   for (int k = 0; k < n; ++k) {
     M.axis = M.axis && parts[k].axis;
-    M.pair.ok = M.pair.ok && parts[k].pair.ok;
+    M.pair.ok = M.pair.ok && parts[k].pair.ok && parts[k].pair.skew == parts[0].pair.skew;
+    M.pair.fp32 = M.pair.fp32 && parts[k].pair.fp32;
     M.wall = M.wall || parts[k].wall;
   }
+  M.pair.skew = parts[0].pair.skew;
+  size_t records = 0;
+  for (int k = 0; k < n; ++k) records += parts[k].pair.srec.size();
+  M.pair.ok = M.pair.ok && records < (1u << kCellBits);  // as in find_pairs
   if (M.pair.ok) {
     size_t entries = 0;
     for (int k = 0; k < n; ++k) {
@@ -2129,57 +2145,86 @@ void dedupe_geometry(Layout& L) {
   }
 }
 
-// Whether the mesh is paired -- every cell has six faces, two per axis, one on
-// its low side and one on its high side, every area vector has exactly one
-// nonzero component, positive on internal faces (left to right is up the axis)
-// -- with geometry inside the bounds under which the quotients of a tame stage
-// (pair.hpp) stay in the normal range; then the tables of the paired kernels.
-// Bounds: |area| in [2^-37, 2^100], volume in [2^-100, 2^24], displacements at
+// Whether the paired kernels take the mesh, and their tables.  Every cell must
+// have six faces, frames must follow from the area vectors, and the geometry
+// must be inside the bounds under which the quotients of a tame stage (pair.hpp)
+// stay in the normal range.  The mesh is axial if every cell has two faces per
+// axis, one on its low side and one on its high side, and every area vector
+// has exactly one nonzero component, positive on internal faces (left to right
+// is up the axis); otherwise it is skew, and its axial faces are still listed
+// by axis.
+// Bounds: largest |area| component in [2^-37, 2^100] and none but zeros below
+// 2^-37 (2^-150 in the FP64 form), volume in [2^-100, 2^24], displacements at
 // most 2^50 with squared length at least 2^-56, and largest area times largest
 // displacement at most 2^14 volumes, so that a gradient times a displacement
-// is at most 2^17 times the largest primitive: FP64 limiter terms stay below
-// 2^(3 (100 + 17) + 6), FP32 ones, scaled by 2^24, below 2^(3 (16 + 17) + 3 + 24),
-// and an FP32 limiter is at least 2^-56 / 2^(2 (16 + 17) + 2).
+// is at most 2^18 times the largest primitive: FP64 limiter terms stay below
+// 2^(3 (100 + 18) + 6), FP32 ones, scaled by 2^24, below 2^(3 (16 + 18) + 2 + 24)
+// and so in range, and an FP32 limiter is at least 2^-56 / 2^(2 (16 + 18) + 2).
 void find_pairs(Layout& L) {
   PairPlan& P = L.pair;
   P = PairPlan();
   const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
-  if (!L.axis) return;
+  if (!L.derive_frame) return;
   const size_t ng = L.geo.size() / kGeoVals;
   std::vector<signed char> axis_of(ng, -1);
   std::vector<double> amax(ng), dmax(ng);
   for (size_t r = 0; r < ng; ++r) {
     const double* q = &L.geo[r * kGeoVals];
-    for (int d = 0; d < 3; ++d)
-      if (q[d] != 0.0) axis_of[r] = (signed char)d;
-    if (axis_of[r] < 0) return;
-    amax[r] = std::fabs(q[axis_of[r]]);
+    for (int d = 0; d < 3; ++d) {
+      const double a = std::fabs(q[d]);
+      if (a != 0.0) axis_of[r] = axis_of[r] < 0 ? (signed char)d : (signed char)kSkewFace;
+      if (a != 0.0 && !(a >= 0x1p-150)) return;
+      if (a != 0.0 && !(a >= 0x1p-37)) P.fp32 = false;
+      amax[r] = std::max(amax[r], a);
+    }
     if (!(amax[r] >= 0x1p-37 && amax[r] <= 0x1p100)) return;
     for (int k = 3; k < 9; ++k) dmax[r] = std::max(dmax[r], std::fabs(q[k]));
     if (!(dmax[r] <= 0x1p50) || !(q[3] * q[3] + q[4] * q[4] + q[5] * q[5] >= 0x1p-56)) return;
   }
+  auto cls = [&](int f) -> int {  // axis, or kSkewFace
+    const int d = axis_of[L.fgeo[f]];
+    return d < kSkewFace && f < nif && L.geo[(size_t)L.fgeo[f] * kGeoVals + d] < 0.0 ? kSkewFace : d;
+  };
   for (int f = 0; f < nif; ++f) {
     const double* q = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
-    if (!(q[axis_of[L.fgeo[f]]] > 0.0) || !(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) return;
+    if (!(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) return;
   }
+  for (int f = 0; f < nf; ++f) P.skew = P.skew || cls(f) == kSkewFace;
   P.nbr.assign((size_t)kMaxSlots * nc, -1);
   P.ent.assign((size_t)kMaxSlots * nc, -1);
+  std::vector<int> fslot(2 * (size_t)nf, 0);  // a face's slot in its left and its right cell
   for (int c = 0; c < nc; ++c) {
     double am = 0.0, dm = 0.0;
     for (int q = 0; q < kMaxSlots; ++q) {
       const int e = L.slot[(size_t)q * nc + c];
-      if (e < 0) return;
+      if (e < 0) {
+        P = PairPlan();
+        return;
+      }
       const int f = e >> 1, side = e & 1, r = L.fgeo[f], d = axis_of[r];
-      const double a = L.geo[(size_t)r * kGeoVals + d];
-      const int s = 2 * d + ((side ? -a : a) > 0.0 ? 1 : 0);
-      if (P.ent[(size_t)s * nc + c] >= 0) return;
-      P.ent[(size_t)s * nc + c] = (r << 1) | side;
-      P.nbr[(size_t)s * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
       am = std::max(am, amax[r]);
       dm = std::max(dm, dmax[r]);
+      if (P.skew) continue;
+      const double a = L.geo[(size_t)r * kGeoVals + d];
+      const int s = 2 * d + ((side ? -a : a) > 0.0 ? 1 : 0);
+      // (two faces on one side: the cell's slots are not one per direction)
+      if (P.ent[(size_t)s * nc + c] >= 0) P.skew = true;
+      P.ent[(size_t)s * nc + c] = (r << 1) | side;
+      P.nbr[(size_t)s * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
     }
-    if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) return;
+    if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) {
+      P = PairPlan();
+      return;
+    }
   }
+  if (P.skew)
+    for (int c = 0; c < nc; ++c)
+      for (int q = 0; q < kMaxSlots; ++q) {
+        const int e = L.slot[(size_t)q * nc + c], f = e >> 1, side = e & 1;
+        P.ent[(size_t)q * nc + c] = (L.fgeo[f] << 1) | side;
+        P.nbr[(size_t)q * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
+        fslot[2 * (size_t)f + side] = q;
+      }
   // Tile lists in chunks of 64 entries of one axis: the faces inside the tile
   // by left cell, a chunk per axis and block of 64 cells (blocks with few
   // faces share one), then the faces shared with other tiles (low side, high
@@ -2191,15 +2236,17 @@ void find_pairs(Layout& L) {
   P.ptr.assign(1, 0);
   P.slot.assign((size_t)kMaxSlots * nc, 0);
   std::vector<int> pos(nf);  // list index of a face in the tile being built
+  std::vector<int> faces;    // the lists' faces
   using Key = std::pair<unsigned long long, int>;
-  std::vector<Key> keys[3];
-  std::vector<std::pair<int, int>> chunks[4];  // (axis, first key), by axis; shared and boundary faces
-  std::vector<int> lens[4];
+  constexpr int kClasses = kSkewFace + 1;
+  std::vector<Key> keys[kClasses];
+  std::vector<std::pair<int, int>> chunks[kClasses + 1];  // (class, first key), by class; shared and boundary faces
+  std::vector<int> lens[kClasses + 1];
   for (int b = 0; b < ntiles; ++b) {
     const int c0 = L.tile_cptr[b], c1 = L.tile_cptr[b + 1];
     for (auto& k : keys) k.clear();
-    auto add = [&](int f, int cls, int cell) {
-      keys[axis_of[L.fgeo[f]]].push_back({((unsigned long long)cls << 32) | (unsigned)cell, f});
+    auto add = [&](int f, int place, int cell) {
+      keys[cls(f)].push_back({((unsigned long long)place << 32) | (unsigned)cell, f});
     };
     for (int q = L.tptr[b]; q < L.tptr[b + 1]; ++q) {
       const int f = L.tfaces[q], l = L.fl[f], r = L.fr[f];
@@ -2211,11 +2258,11 @@ void find_pairs(Layout& L) {
         const int f = L.slot[(size_t)q * nc + c] >> 1;
         if (f >= nif) add(f, 3, c);
       }
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q <= kClasses; ++q) {
       chunks[q].clear();
       lens[q].clear();
     }
-    for (int d = 0; d < 3; ++d) {
+    for (int d = 0; d < kClasses; ++d) {
       std::vector<Key>& K = keys[d];
       std::sort(K.begin(), K.end());
       auto block = [&](int i) { return (K[i].first >> 32) ? 1 << 30 : ((int)(K[i].first & 0xffffffffu) - c0) / 64; };
@@ -2229,15 +2276,15 @@ void find_pairs(Layout& L) {
           if (e - i > 64) break;
           j = e;
         }
-        chunks[inside ? d : 3].push_back({d, i});
-        lens[inside ? d : 3].push_back(j - i);
+        chunks[inside ? d : kClasses].push_back({d, i});
+        lens[inside ? d : kClasses].push_back(j - i);
         i = j;
       }
     }
     int n = 0;
     for (size_t r = 0, left = 1; left; ++r) {
       left = 0;
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q <= kClasses; ++q) {
         if (r >= chunks[q].size()) continue;
         left = 1;
         const int d = chunks[q][r].first, i = chunks[q][r].second;
@@ -2245,13 +2292,17 @@ void find_pairs(Layout& L) {
           const int f = keys[d][k].second;
           pos[f] = n++;
           P.lr.push_back(L.fl[f] | (d << kCellBits));
-          P.lr.push_back(f < nif ? L.fr[f] : ~(((f - nif) << 2) | (L.fkind[f] - 1)));
-          P.gid.push_back(L.fgeo[f]);
+          P.lr.push_back(f >= nif  ? ~(((f - nif) << 2) | (L.fkind[f] - 1))
+                         : P.skew ? L.fr[f] | (fslot[2 * (size_t)f + 1] << kCellBits)
+                                  : L.fr[f]);
+          P.gid.push_back(L.fgeo[f]);  // (skew meshes: with the left cell's slot, below)
+          faces.push_back(f);
         }
         for (; n % 64; ++n) {
           P.lr.push_back(-1);
           P.lr.push_back(-1);
           P.gid.push_back(0);
+          faces.push_back(-1);
         }
       }
     }
@@ -2286,9 +2337,14 @@ void find_pairs(Layout& L) {
   };
   renumber(P.ent, 2 * ng, P.srec);
   renumber(P.gid, ng, P.frec);
-  if (P.srec.size() >= (1u << 28)) {  // 32-bit byte offsets into the record planes
+  if (P.srec.size() >= (1u << kCellBits)) {  // 32-bit byte offsets into the record planes
     P = PairPlan();
     return;
+  }
+  if (P.skew) {
+    for (int& x : P.ent) x |= (P.srec[x] & 1) << kCellBits;
+    for (size_t q = 0; q < faces.size(); ++q)
+      if (faces[q] >= 0) P.gid[q] |= fslot[2 * (size_t)faces[q]] << kCellBits;
   }
   P.ok = true;
 }
@@ -2777,24 +2833,26 @@ ma_status upload_pair_geo(ma_solver* s, const Layout& L) {
   const size_t ns = P.srec.size(), nf = P.frec.size();
   T *ds = nullptr, *dp = nullptr;
   ma_status st = MA_OK;
+  constexpr int W = 16 / (int)sizeof(T);  // values of a vector
+  const int A = P.skew ? 3 : 1;           // area values
+  const int SV = (A + 3 + W - 1) / W * W, FV = (A + 6 + W - 1) / W * W;
   if (s->counting) {
-    if ((st = s->alloc(&ds, 4 * ns)) || (st = s->alloc(&dp, 8 * nf))) return st;
+    if ((st = s->alloc(&ds, SV * ns)) || (st = s->alloc(&dp, FV * nf))) return st;
   } else {
-    constexpr int W = 16 / (int)sizeof(T);  // values of a vector
     auto at = [](std::vector<T>& h, size_t n, int k, size_t i) -> T& { return h[((size_t)(k / W) * n + i) * W + k % W]; };
-    auto area = [&](int r) {  // the nonzero component, exactly
+    auto area = [&](int r, int d) {  // component d, or the one that is not zero, exactly
       const double* q = &L.geo[(size_t)r * kGeoVals];
-      return q[0] + q[1] + q[2];
+      return P.skew ? q[d] : q[0] + q[1] + q[2];
     };
-    std::vector<T> hs(4 * ns, T(0)), hp(8 * nf, T(0));
+    std::vector<T> hs(SV * ns, T(0)), hp(FV * nf, T(0));
     for (size_t i = 0; i < ns; ++i) {
       const int r = P.srec[i] >> 1, side = P.srec[i] & 1;
-      at(hs, ns, 0, i) = T(side ? -area(r) : area(r));
-      for (int d = 0; d < 3; ++d) at(hs, ns, 1 + d, i) = T(L.geo[(size_t)r * kGeoVals + 3 + 3 * side + d]);
+      for (int d = 0; d < A; ++d) at(hs, ns, d, i) = T(side ? -area(r, d) : area(r, d));
+      for (int d = 0; d < 3; ++d) at(hs, ns, A + d, i) = T(L.geo[(size_t)r * kGeoVals + 3 + 3 * side + d]);
     }
     for (size_t i = 0; i < nf; ++i) {
-      at(hp, nf, 0, i) = T(area(P.frec[i]));
-      for (int d = 0; d < 6; ++d) at(hp, nf, 1 + d, i) = T(L.geo[(size_t)P.frec[i] * kGeoVals + 3 + d]);
+      for (int d = 0; d < A; ++d) at(hp, nf, d, i) = T(area(P.frec[i], d));
+      for (int d = 0; d < 6; ++d) at(hp, nf, A + d, i) = T(L.geo[(size_t)P.frec[i] * kGeoVals + 3 + d]);
     }
     if ((st = upload(s, &ds, hs)) || (st = upload(s, &dp, hp))) return st;
   }
@@ -2828,7 +2886,6 @@ ma_status upload_paired(ma_solver* s, const Layout& L) {
   }
   if (st) return st;
   s->nbr = dids;
-  s->m.axis = s->m.full = 1;
   s->t.ptr = dptr;
   s->t.lr = reinterpret_cast<const int2*>(dlr);
   s->t.fgid = dgid;
@@ -2871,7 +2928,8 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   s->org = dorg;
   m.fwall = dfw;
   s->wall = L.wall;
-  s->pair = L.pair.ok;
+  s->pair = L.pair.ok && (!s->fp32 || L.pair.fp32);
+  s->skew = L.pair.skew;
   int *dtcptr, *dtcase;
   if ((st = upload(s, &dtcptr, L.tile_cptr)) || (st = upload(s, &dtcase, tile_case))) return st;
   s->t.ntiles = L.ntiles;
@@ -2984,6 +3042,14 @@ inline int resident(const ma_solver* s, int per) {
 // threads), else 4 wavefronts walking the chunks.
 inline int pair_threads(int max_faces) { return max_faces <= kPairMaxThreads ? max_faces : kTile; }
 
+template <bool kSkew, bool SO, class Inv, class Visc, class T>
+auto pair_flux_kernel(const ma_solver* s) {
+  constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
+  if (s->wg_per_cu > 0)
+    return s->wall ? k_flux_pair<kSkew, SO, true, true, Inv, Visc, T> : k_flux_pair<kSkew, SO, VW, true, Inv, Visc, T>;
+  return s->wall ? k_flux_pair<kSkew, SO, true, false, Inv, Visc, T> : k_flux_pair<kSkew, SO, VW, false, Inv, Visc, T>;
+}
+
 template <bool SO, class Inv, class Visc, class Lim, class T>
 void run_stage(ma_solver* s, int irk) {
   // TimeSolverExplicitRK4.h:187-195
@@ -3018,16 +3084,13 @@ void run_stage(ma_solver* s, int irk) {
     if (SO || Visc::isViscous) {
       s->launch(SO ? "k_grad_limiter" : "k_grad", [&] {
         const int per = (nb + kXcds - 1) / kXcds;
-        hipLaunchKernelGGL((k_grad_pair<SO, FV, Lim, T>), dim3(per * kXcds), dim3(kBlock), 0, s->stream, m, s->nbr,
+        const auto kern = s->skew ? k_grad_pair<true, SO, FV, Lim, T> : k_grad_pair<false, SO, FV, Lim, T>;
+        hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, m, s->nbr,
                            static_cast<const T*>(Vs), FV ? nullptr : static_cast<T*>(s->grad),
                            static_cast<T*>(s->fv), per);
       });
     }
-    constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
-    const auto kern = s->wg_per_cu > 0
-                          ? (s->wall ? k_flux_pair<SO, true, true, Inv, Visc, T> : k_flux_pair<SO, VW, true, Inv, Visc, T>)
-                          : (s->wall ? k_flux_pair<SO, true, false, Inv, Visc, T>
-                                     : k_flux_pair<SO, VW, false, Inv, Visc, T>);
+    const auto kern = s->skew ? pair_flux_kernel<true, SO, Inv, Visc, T>(s) : pair_flux_kernel<false, SO, Inv, Visc, T>(s);
     s->launch("k_flux", [&] {
       hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
                          (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
@@ -3140,7 +3203,9 @@ template <bool SO, class Inv, class Visc, class Lim, class T>
 ma_status run_persistent(ma_solver* s, int nsteps) {
   if (nsteps == 0) return MA_OK;
   constexpr bool FV = SO && !Visc::isViscous;
-  const auto kern = s->pair ? k_steps<SO, Inv, Visc, Lim, T, true> : k_steps<SO, Inv, Visc, Lim, T, false>;
+  const auto kern = !s->pair  ? k_steps<SO, Inv, Visc, Lim, T, 0>
+                    : s->skew ? k_steps<SO, Inv, Visc, Lim, T, 2>
+                              : k_steps<SO, Inv, Visc, Lim, T, 1>;
   const size_t lds = std::max((size_t)s->t.max_faces * 5 * sizeof(T),
                               FV || s->pair ? (size_t)0 : (size_t)kBlock * kStageRow<T> * sizeof(T));
   int coop = 0, per_cu = 0, wall_khz = 0;
@@ -3640,7 +3705,8 @@ void stage3_gradients(ma_solver* s) {
   const int nb = nblocks(s->m.nc);
   const int per = (nb + kXcds - 1) / kXcds;
   if (s->pair) {
-    hipLaunchKernelGGL((k_grad_pair<true, true, Lim, T>), dim3(per * kXcds), dim3(kBlock), 0, s->stream, s->m, s->nbr,
+    const auto kern = s->skew ? k_grad_pair<true, true, true, Lim, T> : k_grad_pair<false, true, true, Lim, T>;
+    hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, s->m, s->nbr,
                        static_cast<const T*>(s->V2), static_cast<T*>(s->grad), static_cast<T*>(s->fv), per);
     return;
   }

@@ -1,10 +1,11 @@
-"""The paired-mesh kernels (boxes: every face along an axis) where they can go
-wrong: dimensions of one cell, tiles and 64-cell chunks with remainders, every
-boundary kind on every scheme, values outside the range of the short quotients.
+"""The paired-mesh kernels (boxes: every face along an axis; ramps: the form for
+skew meshes) where they can go wrong: dimensions of one cell, tiles and 64-cell
+chunks with remainders, every boundary kind on every scheme, values outside the
+range of the short quotients.
 
-FP64 equals the oracle bit for bit.  A batch runs the general kernels for all
-its cases when one of them is not a box, so a box batched with a ramp gives the
-general kernels' bits for the same mesh, in FP32 too: results are equal.
+FP64 equals the oracle bit for bit.  A batch of boxes and ramps together runs
+the general kernels for all its cases, so it gives the general kernels' bits
+for the meshes, in FP32 too: results are equal.
 """
 import numpy as np
 import pytest
@@ -19,11 +20,14 @@ SCHEMES = [(0, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 0)]  # second order, viscous,
 WALLS = [(1, 1, 3, 2, 4, 1), (4, 1, 2, 3, 3, 2)]
 
 
+RAMP = dict(problem_type=2, angle=20.0)
+
+
 def _kw(shape, scheme, walls=0, **more):
     nx, ny, nz = shape  # spacings that are powers of two: every area vector exactly along its axis
-    return dict(problem_type=1, lx=nx / 64, ly=ny / 128, lz=nz / 128, nx=nx, ny=ny, nz=nz, dt=1e-6,
-                ntimesteps=4, second_order_space=scheme[0], viscous=scheme[1], limiter=scheme[2], ic_kind=2,
-                perturb=0.02, seed=5, bc_kind=WALLS[walls], **more)
+    return dict(dict(problem_type=1, lx=nx / 64, ly=ny / 128, lz=nz / 128, nx=nx, ny=ny, nz=nz, dt=1e-6,
+                     ntimesteps=4, second_order_space=scheme[0], viscous=scheme[1], limiter=scheme[2], ic_kind=2,
+                     perturb=0.02, seed=5, bc_kind=WALLS[walls]), **more)
 
 
 def _same_as_oracle(p, n):
@@ -37,11 +41,12 @@ def _same_as_oracle(p, n):
             assert np.array_equal(lim, olim, equal_nan=True)
 
 
+@pytest.mark.parametrize("mesh", [{}, RAMP], ids=["box", "ramp"])
 @pytest.mark.parametrize("scheme", SCHEMES)
 @pytest.mark.parametrize("shape", SHAPES)
-def test_boxes_equal_the_oracle(shape, scheme):
+def test_equal_to_the_oracle(shape, scheme, mesh):
     for k, more in enumerate(({}, dict(workgroups_per_cu=1))):
-        p = Pair(_kw(shape, scheme, k, **more))
+        p = Pair(_kw(shape, scheme, k, **mesh, **more))
         try:
             _same_as_oracle(p, 1)
             _same_as_oracle(p, 3)
@@ -50,9 +55,10 @@ def test_boxes_equal_the_oracle(shape, scheme):
 
 
 @pytest.mark.parametrize("what", ["tiny", "huge", "nan"])
+@pytest.mark.parametrize("mesh", [{}, RAMP], ids=["box", "ramp"])
 @pytest.mark.parametrize("scheme", SCHEMES)
-def test_values_outside_the_short_quotients_range(scheme, what):
-    p = Pair(_kw((17, 9, 8), scheme))
+def test_values_outside_the_short_quotients_range(scheme, mesh, what):
+    p = Pair(_kw((17, 9, 8), scheme, **mesh))
     try:
         U = p.gpu.state().copy()
         c = np.arange(3, U.shape[0], 97)
@@ -75,24 +81,23 @@ def test_values_outside_the_short_quotients_range(scheme, what):
 
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("scheme", SCHEMES)
-def test_boxes_equal_the_general_kernels(scheme, precision):
+def test_equal_to_the_general_kernels(scheme, precision):
     for k, shape in enumerate(SHAPES):
         cases = []
-        for kw in (_kw(shape, scheme, k % 2, precision=precision),
-                   dict(_kw((6, 5, 4), scheme, precision=precision), problem_type=2, angle=20.0, lx=2.0, ly=1.0,
-                        lz=1.0)):
-            o = M.Options(**kw)
+        for mesh in ({}, RAMP):
+            o = M.Options(**_kw(shape, scheme, k % 2, precision=precision, **mesh))
             cases.append((M.Parallel3DMesh(o.nx, o.ny, o.nz, o.lx, o.ly, o.lz, o.problem_type, o.angle,
                                            options=o).fillMeshData(), o))
         _log(f"[gpu-paired] {shape} {scheme} precision {precision}")
-        solo, both = M.TimeSolverExplicitRK4(*cases[0]), M.BatchSolver(cases)
+        runs = [M.BatchSolver(cases)] + [M.TimeSolverExplicitRK4(*c) for c in cases]
         try:
-            for s in (solo, both):
+            for s in runs:
                 s.initialize()
                 s.step(4)
-            U = both.state()[both.offsets[0]:both.offsets[1]]
+            U, off = runs[0].state(), runs[0].offsets
             assert np.isfinite(U).all()
-            assert np.array_equal(solo.state(), U)
+            for j in range(2):
+                assert np.array_equal(runs[1 + j].state(), U[off[j]:off[j + 1]]), ("box", "ramp")[j]
         finally:
-            solo.close()
-            both.close()
+            for s in runs:
+                s.close()
