@@ -41,14 +41,15 @@
 //                wavefront's access is aligned.
 //
 // Measured against the general kernels, microseconds per launch (k_grad,
-// k_flux): FP64 viscous 256 x 128 x 64 plate 227 -> 155, 367 -> 338; FP32
-// viscous 211 x 127 x 45 plate 99 -> 53, 139 -> 117; 48 batched FP32 shock
+// k_flux): FP64 viscous 256 x 128 x 64 plate 227 -> 155, 367 -> 300; FP32
+// viscous 211 x 127 x 45 plate 99 -> 53, 139 -> 107; 48 batched FP32 shock
 // tubes 320 -> 194, 384 -> 318; 4096-cell FP64 plate 10.3 -> 5.3, 14.3 -> 7.3;
 // first-order 64 x 16 x 16 shock tube 14.1 with its boundary launch -> 5.2.
 // Skew: FP64 321 x 157 x 11 ramp 126 -> 74, 120 -> 97; 2240-cell ramp 13.1 -> 7.0,
 // 10.5 -> 8.0 (its boundary faces were in the gradient launch).
-// At 2.1M cells the flux kernel still has its address and data units busy 89%
-// and 92% (VALU 37%), the gradient kernel its data return 86%.
+// At 2.1M cells the flux kernel is bound by HBM and L2: 1.7 GB a launch at 5.5
+// TB/s, most of it records fetched again by the tiles around (96 tiles in flight
+// per XCD against a 4 MB L2); the gradient kernel has its data return 86% busy.
 //
 // Every value the kernels keep is formed with the general kernels' operations
 // in the same order, and the terms left out are +-0, so results are the same
@@ -647,6 +648,112 @@ __device__ __forceinline__ void pair_flux(const DevMesh& m, const T* __restrict_
   else axis_flux<2, SO, kWall>(vl, vr, gf, geo[kSkew ? 2 : 0], kind, winv, inflow, inv, visc, F);
 }
 
+// Another lane's value (byte address 4 * lane), through the LDS crossbar.
+__device__ __forceinline__ float from_lane(int addr, float x) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
+}
+__device__ __forceinline__ double from_lane(int addr, double x) {
+  return __hiloint2double(__builtin_amdgcn_ds_bpermute(addr, __double2hiint(x)),
+                          __builtin_amdgcn_ds_bpermute(addr, __double2loint(x)));
+}
+
+// Fluxes through the three high faces of cell c of an axial mesh (viscous second
+// order), list entries q0, q0 + 64 and q0 + 128: pair_flux with the cell's own
+// values and gradient record loaded once instead of once per axis.
+template <int D, bool kWall, class Inv, class Visc, class T>
+__device__ __forceinline__ void own_face(const DevMesh& m, const T* __restrict__ V, const T* __restrict__ rec,
+                                         const Inflow* __restrict__ inflow, const T* own, int mf, const T* rl, int Rr,
+                                         int gid,
+                                         unsigned c, unsigned c0, unsigned cells, const Inv& inv,
+                                         const Visc& visc, T* F) {
+  constexpr int W = kVec<T>;
+  int n = m.ns;
+  asm volatile("" : "+s"(n));  // see pair_flux
+  const bool bnd = Rr < 0;
+  const unsigned Rc = bnd ? c : (unsigned)Rr;
+  T vl[5], vr[5], rr[kRec], geo[8];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) vl[k] = own[k * mf];
+#pragma unroll
+  for (int j = 0; j < 8 / W; ++j)
+    get_vec(static_cast<const T*>(m.ptab), j, m.nfrec, (unsigned)gid, geo + j * W);
+  // a neighbour in the block (cells c0 to c0 + cells - 1) is another lane's own
+  // cell; only the block's edge loads
+  const bool near = Rc - c0 < cells;
+  if (__any(near)) {
+    const int addr = (int)(Rc - c0) * 4;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vr[k] = from_lane(addr, vl[k]);
+#pragma unroll
+    for (int k = 0; k < kRec; ++k) rr[k] = from_lane(addr, rl[k]);
+  }
+  if (!near) {
+    get_five(V, n, Rc, vr);
+#pragma unroll
+    for (int j = 0; j < kRec / W; ++j) get_vec(rec, j, n, Rc, rr + j * W);
+  }
+#pragma unroll
+  for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(rr[15 + k]));
+#pragma unroll
+  for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(geo[1 + d]), "+v"(geo[4 + d]), "+v"(rr[d]));
+  if (!bnd) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const T tl = geo[1] * rl[3 * k] + geo[2] * rl[3 * k + 1] + geo[3] * rl[3 * k + 2];
+      const T tr = geo[4] * rr[3 * k] + geo[5] * rr[3 * k + 1] + geo[6] * rr[3 * k + 2];
+      vl[k] = vl[k] + tl * rl[15 + k];
+      vr[k] = vr[k] + tr * rr[15 + k];
+    }
+  }
+  T gf[5][3];
+#pragma unroll
+  for (int k = 1; k < 5; ++k)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) gf[k][d] = T(0.5) * (rl[3 * k + d] + rr[3 * k + d]);
+  const int kind = bnd ? (~Rr & 3) + 1 : 0;
+  T winv = T(0);
+  if (kWall && kind == MA_BC_NOSLIP) winv = T(m.fwall[m.nif + (~Rr >> 2)]);
+  axis_flux<D, true, kWall>(vl, vr, gf, geo[0], kind, winv, inflow, inv, visc, F);
+}
+
+template <bool kWall, class Inv, class Visc, class T>
+__device__ __forceinline__ void own_faces(const DevMesh& m, const TileMap& t, const T* __restrict__ V,
+                                          const T* __restrict__ rec, const Inflow* __restrict__ inflow, T* lds,
+                                          int list, int q0, unsigned c, unsigned c0, unsigned cells, const Inv& inv,
+                                         const Visc& visc) {
+  const int mf = t.max_faces;
+  int R[3], g[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    R[d] = t.lr[list + q0 + 64 * d].y;
+    g[d] = t.fgid[list + q0 + 64 * d];
+  }
+  // The cell's values wait in the last face's place in LDS, its record in
+  // registers: with both in registers the FP64 kernel spills 24 bytes a lane.
+  T* own = lds + q0 + 128;
+  T rl[kRec], F[5];
+  {
+    T vc[5];
+    get_five(V, m.ns, c, vc);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) own[k * mf] = vc[k];
+  }
+#pragma unroll
+  for (int j = 0; j < kRec / kVec<T>; ++j) get_vec(rec, j, m.ns, c, rl + j * kVec<T>);
+  auto keep = [&](int d) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) lds[k * mf + q0 + 64 * d] = F[k];
+    asm volatile("" ::: "memory");  // the next axis' loads stay behind this one's arithmetic
+  };
+  asm volatile("" ::: "memory");  // (own is read back, not kept)
+  own_face<0, kWall>(m, V, rec, inflow, own, mf, rl, R[0], g[0], c, c0, cells, inv, visc, F);
+  keep(0);
+  own_face<1, kWall>(m, V, rec, inflow, own, mf, rl, R[1], g[1], c, c0, cells, inv, visc, F);
+  keep(1);
+  own_face<2, kWall>(m, V, rec, inflow, own, mf, rl, R[2], g[2], c, c0, cells, inv, visc, F);
+  keep(2);
+}
+
 // Second phase of a paired tile: every cell adds its face fluxes from LDS (5
 // planes of t.max_faces) in the reference's order and takes the RK update
 // (flux_tile's phase 2).
@@ -712,7 +819,7 @@ __device__ __forceinline__ void update_tile_pair(const DevMesh& m, const TileMap
 // wavefront w takes chunks w, w + waves, ...  Slot entries are LDS index << 1 |
 // side in the reference's summation order with the boundary faces last, in
 // kind order.
-template <bool kSkew, bool SO, bool kWall, class Inv, class Visc, class T>
+template <bool kSkew, bool kOwn, bool SO, bool kWall, class Inv, class Visc, class T>
 __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& t, int tile, T* lds,
                                                const T* __restrict__ V, const T* __restrict__ rec,
                                                const T* __restrict__ fv, const Inflow* __restrict__ inflows,
@@ -727,13 +834,22 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
   const Inflow* inflow = inflows + kcase;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), step = (int)blockDim.x;
+  int first = wave * 64;
+  if constexpr (kOwn) {
+    const int c0 = t.cptr[tile], cells = t.cptr[tile + 1] - c0;
+    for (int b = first; b < cells; b += step)
+      if (b + lane < cells)
+        own_faces<kWall>(m, t, V, rec, inflow, lds, f0, 3 * b + lane, (unsigned)(c0 + b + lane), (unsigned)(c0 + b),
+                         (unsigned)min(64, cells - b), inv, visc);
+    first += (cells + 63) / 64 * 192;
+  }
   int2 lr = make_int2(-1, -1);
   int g = 0;
-  if (wave * 64 < n) {
-    lr = t.lr[f0 + wave * 64 + lane];
-    g = t.fgid[f0 + wave * 64 + lane];
+  if (first < n) {
+    lr = t.lr[f0 + first + lane];
+    g = t.fgid[f0 + first + lane];
   }
-  for (int q = wave * 64; q < n; q += step) {
+  for (int q = first; q < n; q += step) {
     const int2 c = lr;
     const int gc = g;
     if (q + step < n) {  // the next chunk's entries are fetched while this one is evaluated
@@ -751,11 +867,19 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
   update_tile_pair(m, t, tile, kcase, lds, Uacc_in, Uacc_out, R, dt_dev, beta, Un, Vnext, alpha_next, last);
 }
 
+// kOwn: the tile lists start with their cells' high faces (PairPlan::own), whose
+// own side is loaded once for three faces.  The viscous second-order kernels
+// load 25 values a side, and a tile's records alone (41 KB in FP64) exceed the
+// 32 KB L1, so nearly every load goes to L2.  Keeping the own side, and taking a
+// neighbour of the same 64-cell block from the lane that has it, leaves a load
+// of the cell, one of its neighbour in the next block and the block's edges
+// instead of 6 (L2 reads 31 -> 23 million a launch, k_flux of the 2.1M-cell FP64
+// plate 338 -> 300 us, of the 1.2M-cell FP32 plate 117 -> 107).
 // kWalk: fewer workgroups than tiles, each walking its XCD's run (see k_flux);
 // otherwise one tile per workgroup, a form of its own because the walk's
 // loop-carried values cost the FP64 viscous kernel spills and the FP64 inviscid
 // one ten registers.
-template <bool kSkew, bool SO, bool kWall, bool kWalk, class Inv, class Visc, class T>
+template <bool kSkew, bool kOwn, bool SO, bool kWall, bool kWalk, class Inv, class Visc, class T>
 __global__ __launch_bounds__(kPairMaxThreads) __attribute__((amdgpu_waves_per_eu(kPairFluxWaves<Visc, T>)))
 void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restrict__ rec,
                  const Inflow* __restrict__ inflows, const double* Uacc_in, double* Uacc_out,
@@ -770,7 +894,7 @@ void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restr
     for (int j = blockIdx.x / kXcds; j < t.per_xcd; j += stride) {
       const int tile = xcd * t.per_xcd + j;
       if (tile >= t.ntiles) break;  // uniform over the workgroup
-      flux_tile_pair<kSkew, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
+      flux_tile_pair<kSkew, kOwn, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
                                               beta, inv, visc, Un, Vnext, alpha_next, last);
       advance_time(t, tile, dt_dev, time_dev);
       __syncthreads();  // the LDS is reused by the next tile
@@ -778,7 +902,7 @@ void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restr
   } else {
     const int tile = xcd * t.per_xcd + blockIdx.x / kXcds;
     if (tile >= t.ntiles) return;  // uniform over the workgroup
-    flux_tile_pair<kSkew, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
+    flux_tile_pair<kSkew, kOwn, SO, kWall, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, inflows, Uacc_in, Uacc_out, R, dt_dev,
                                             beta, inv, visc, Un, Vnext, alpha_next, last);
     advance_time(t, tile, dt_dev, time_dev);
   }

@@ -1467,7 +1467,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
         const int tile = xcd * a.t.per_xcd + j;
         if (tile >= a.t.ntiles) break;  // uniform over the workgroup
         if constexpr (kPair)
-          flux_tile_pair<kPair == 2, SO, true, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, a.inflow,
+          flux_tile_pair<kPair == 2, false, SO, true, Inv, Visc, T>(m, a.t, tile, lds, Vs, frec, frec, a.inflow,
                                                              irk == 0 ? Un : Uacc,
                                                  Uacc, a.R, a.dt, beta(irk), inv, visc, Un, Vn, alpha_next(irk),
                                                  irk == 3 ? 1 : 0);
@@ -1539,6 +1539,7 @@ struct ma_solver {
   bool fp32 = false;
   bool pair = false;          // runs the paired-mesh kernels and array layouts (pair.hpp)
   bool skew = false;          // their forms for meshes with faces along no axis
+  bool own = false;           // tile lists start with the cells' high faces (PairPlan)
   bool wall = false;          // some boundary face is a no-slip wall
   // Cases (independent meshes stepped together; a plain run is one case).
   int ncases = 1;
@@ -1795,6 +1796,7 @@ struct PairPlan {
   bool ok = false;
   bool fp32 = true;                      // in the FP32 form as well
   bool skew = false;                     // some face is along no axis: slots in slot order, kSkewFace chunks
+  bool own = false;                      // a tile's list starts with whole blocks, see find_pairs
   int max_faces = 64;                    // longest tile list, padding included
   std::vector<int> nbr, ent;             // kMaxSlots planes of nc: (low, high) along x, y, z; skew: as L.slot
   std::vector<int> srec, frec;           // slot record -> geometry record << 1 | side; face record -> geometry record
@@ -1855,6 +1857,12 @@ ma_status validate_pairs(const Layout& L) {
       if (P.skew && l >= 0 && r >= 0 && (r >> kCellBits >= kMaxSlots || P.gid[q] >> kCellBits >= kMaxSlots))
         return bad("tile face slots");
     }
+    const int cells = L.tile_cptr[b + 1] - L.tile_cptr[b];
+    if (P.own && (P.skew || n < (cells + 63) / 64 * 192)) return bad("own faces");
+    for (int i = 0; i < cells && P.own; ++i)
+      for (int d = 0; d < 3; ++d)
+        if (P.lr[2 * (size_t)(f0 + (i / 64 * 3 + d) * 64 + i % 64)] != ((L.tile_cptr[b] + i) | (d << kCellBits)))
+          return bad("own faces");
     for (int c = L.tile_cptr[b]; c < L.tile_cptr[b + 1]; ++c)
       for (int s = 0; s < kMaxSlots; ++s) {
         const int e = P.slot[(size_t)s * nc + c], j = e >> 1;
@@ -1971,12 +1979,13 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
   M.fgeo.assign(M.nf, 0);
   M.geo.clear();
   M.axis = true;
-  M.pair.ok = true;
+  M.pair.ok = M.pair.own = true;
   M.wall = false;
   for (int k = 0; k < n; ++k) {
     M.axis = M.axis && parts[k].axis;
     M.pair.ok = M.pair.ok && parts[k].pair.ok && parts[k].pair.skew == parts[0].pair.skew;
     M.pair.fp32 = M.pair.fp32 && parts[k].pair.fp32;
+    M.pair.own = M.pair.own && parts[k].pair.own;
     M.wall = M.wall || parts[k].wall;
   }
   M.pair.skew = parts[0].pair.skew;
@@ -2230,9 +2239,15 @@ void find_pairs(Layout& L) {
   // faces share one), then the faces shared with other tiles (low side, high
   // side, by the tile's own cell) and the boundary faces.  Chunk r of the
   // three axes and chunk r of the shared faces follow each other.
+  // own: the chunks of a block hold the high faces of its cells, one per cell in
+  // cell order, whatever is on their other side, and all blocks' chunks come
+  // before the others, so that a wavefront can keep a cell's own values over
+  // its three faces.  Tiles of at most 128 cells, which are few wavefronts'
+  // work, spread their chunks over all of them instead.
   std::vector<int> tile_of(nc);
   for (int b = 0; b < ntiles; ++b)
     for (int d = L.tile_cptr[b]; d < L.tile_cptr[b + 1]; ++d) tile_of[d] = b;
+  for (int b = 0; b < ntiles; ++b) P.own = P.own || (!P.skew && L.tile_cptr[b + 1] - L.tile_cptr[b] > 128);
   P.ptr.assign(1, 0);
   P.slot.assign((size_t)kMaxSlots * nc, 0);
   std::vector<int> pos(nf);  // list index of a face in the tile being built
@@ -2251,12 +2266,15 @@ void find_pairs(Layout& L) {
     for (int q = L.tptr[b]; q < L.tptr[b + 1]; ++q) {
       const int f = L.tfaces[q], l = L.fl[f], r = L.fr[f];
       const bool inl = tile_of[l] == b, inr = tile_of[r] == b;
-      add(f, inl && inr ? 0 : inr ? 1 : 2, inl ? l : r);
+      add(f, (inl && inr) || (P.own && inl) ? 0 : inr ? 1 : 2, inl ? l : r);
     }
     for (int c = c0; c < c1; ++c)
       for (int q = 0; q < kMaxSlots; ++q) {
         const int f = L.slot[(size_t)q * nc + c] >> 1;
-        if (f >= nif) add(f, 3, c);
+        if (f >= nif) {
+          const double* a = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
+          add(f, P.own && a[0] + a[1] + a[2] > 0.0 ? 0 : 3, c);  // (own: an axial mesh)
+        }
       }
     for (int q = 0; q <= kClasses; ++q) {
       chunks[q].clear();
@@ -2282,13 +2300,19 @@ void find_pairs(Layout& L) {
       }
     }
     int n = 0;
+    const size_t blocks = P.own ? chunks[0].size() : 0;  // (own: as many of every axis)
     for (size_t r = 0, left = 1; left; ++r) {
       left = 0;
       for (int q = 0; q <= kClasses; ++q) {
-        if (r >= chunks[q].size()) continue;
+        if (P.own && (q == kClasses) != (r >= blocks)) {
+          left |= q == kClasses;
+          continue;
+        }
+        if ((q == kClasses ? r - blocks : r) >= chunks[q].size()) continue;
         left = 1;
-        const int d = chunks[q][r].first, i = chunks[q][r].second;
-        for (int k = i; k < i + lens[q][r]; ++k) {
+        const size_t x = q == kClasses ? r - blocks : r;
+        const int d = chunks[q][x].first, i = chunks[q][x].second;
+        for (int k = i; k < i + lens[q][x]; ++k) {
           const int f = keys[d][k].second;
           pos[f] = n++;
           P.lr.push_back(L.fl[f] | (d << kCellBits));
@@ -2930,6 +2954,7 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   s->wall = L.wall;
   s->pair = L.pair.ok && (!s->fp32 || L.pair.fp32);
   s->skew = L.pair.skew;
+  s->own = L.pair.own;
   int *dtcptr, *dtcase;
   if ((st = upload(s, &dtcptr, L.tile_cptr)) || (st = upload(s, &dtcase, tile_case))) return st;
   s->t.ntiles = L.ntiles;
@@ -3042,12 +3067,14 @@ inline int resident(const ma_solver* s, int per) {
 // threads), else 4 wavefronts walking the chunks.
 inline int pair_threads(int max_faces) { return max_faces <= kPairMaxThreads ? max_faces : kTile; }
 
-template <bool kSkew, bool SO, class Inv, class Visc, class T>
+template <bool kSkew, bool kOwn, bool SO, class Inv, class Visc, class T>
 auto pair_flux_kernel(const ma_solver* s) {
   constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
   if (s->wg_per_cu > 0)
-    return s->wall ? k_flux_pair<kSkew, SO, true, true, Inv, Visc, T> : k_flux_pair<kSkew, SO, VW, true, Inv, Visc, T>;
-  return s->wall ? k_flux_pair<kSkew, SO, true, false, Inv, Visc, T> : k_flux_pair<kSkew, SO, VW, false, Inv, Visc, T>;
+    return s->wall ? k_flux_pair<kSkew, kOwn, SO, true, true, Inv, Visc, T>
+                   : k_flux_pair<kSkew, kOwn, SO, VW, true, Inv, Visc, T>;
+  return s->wall ? k_flux_pair<kSkew, kOwn, SO, true, false, Inv, Visc, T>
+                 : k_flux_pair<kSkew, kOwn, SO, VW, false, Inv, Visc, T>;
 }
 
 template <bool SO, class Inv, class Visc, class Lim, class T>
@@ -3090,7 +3117,10 @@ void run_stage(ma_solver* s, int irk) {
                            static_cast<T*>(s->fv), per);
       });
     }
-    const auto kern = s->skew ? pair_flux_kernel<true, SO, Inv, Visc, T>(s) : pair_flux_kernel<false, SO, Inv, Visc, T>(s);
+    constexpr bool kOwn = SO && Visc::isViscous;
+    const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Inv, Visc, T>(s)
+                      : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Inv, Visc, T>(s)
+                                       : pair_flux_kernel<false, false, SO, Inv, Visc, T>(s);
     s->launch("k_flux", [&] {
       hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
                          (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
