@@ -24,9 +24,11 @@ ma_status plan_layout_shared(const ma_mesh_data* md, const ma_options* opt, std:
 ma_status plan_case_with(const std::shared_ptr<const LayoutPlan>& lp, const ma_options* opt, PlannedCase** out,
                          size_t* bytes);
 void destroy_plan(PlannedCase* pc);
-// Builds the planned case inside [region, region + region_bytes) on its own
-// stream (no device allocation); the plan is only read.
-ma_status create_from_plan(PlannedCase* pc, void* region, size_t region_bytes, ma_solver** out);
+// Builds the planned case inside [region, region + region_bytes) on the
+// caller's stream, which outlives it (no device allocation); the plan is only
+// read.  solver_set_stream: the stream of its later copies.
+ma_status create_from_plan(PlannedCase* pc, void* region, size_t region_bytes, hipStream_t stream, ma_solver** out);
+void solver_set_stream(ma_solver* s, hipStream_t stream);
 // Which of the case's two state buffers holds sol_n (0 or 1).
 int solver_cur(const ma_solver* s);
 // Records that `steps` steps ran outside the solver's own launches (in a

@@ -242,6 +242,10 @@ struct ma_server {
   long long finished = 0;
   bool stop = false;
   std::vector<std::thread> setup;
+  // one per setup thread and one for the finisher, kept while the server runs: a
+  // stream made and destroyed for every request is two runtime calls on the
+  // request's way and leaves the runtime thousands of dead streams to tidy up
+  std::vector<hipStream_t> streams;
   std::thread sched, finish;
 
   double now() const { return std::chrono::duration<double>(Clock::now() - t0).count(); }
@@ -280,7 +284,7 @@ void retire(ma_server* S, Request* r) {
   }
 }
 
-void setup_worker(ma_server* S) {
+void setup_worker(ma_server* S, hipStream_t stream) {
   (void)hipSetDevice(S->device);
   for (;;) {
     Request* r = nullptr;
@@ -348,7 +352,7 @@ void setup_worker(ma_server* S) {
     }
     // build inside the region, outside the lock
     ma_solver* s = nullptr;
-    st = ma::create_from_plan(pc, S->base + r->offset, r->bytes, &s);
+    st = ma::create_from_plan(pc, S->base + r->offset, r->bytes, stream, &s);
     ma::destroy_plan(pc);
     r->solver = s;
     if (!st) st = ma_solver_initialize(s);
@@ -401,7 +405,7 @@ void hand_off(ma_server* S, Request* r) {
   S->cv_complete.notify_one();
 }
 
-void finisher(ma_server* S) {
+void finisher(ma_server* S, hipStream_t stream) {
   (void)hipSetDevice(S->device);
   for (;;) {
     Request* r = nullptr;
@@ -412,6 +416,7 @@ void finisher(ma_server* S) {
       r = S->completing.front();
       S->completing.pop_front();
     }
+    if (r->solver) ma::solver_set_stream(r->solver, stream);  // (its build ended with a wait)
     complete(S, r);
   }
 }
@@ -626,9 +631,15 @@ extern "C" ma_status ma_server_create(const ma_server_config* cfg, ma_server** o
   S->region.reset(size);
   S->t0 = Clock::now();
   try {
-    for (int i = 0; i < c.setup_threads; ++i) S->setup.emplace_back(setup_worker, S);
+    S->streams.assign((size_t)c.setup_threads + 1, nullptr);
+    for (hipStream_t& st : S->streams)
+      if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
+        ma_server_destroy(S);
+        return ma::fail(MA_ERR_DEVICE, "ma_server_create: hipStreamCreate failed");
+      }
+    for (int i = 0; i < c.setup_threads; ++i) S->setup.emplace_back(setup_worker, S, S->streams[i]);
     S->sched = std::thread(scheduler, S);
-    S->finish = std::thread(finisher, S);
+    S->finish = std::thread(finisher, S, S->streams.back());
   } catch (const std::exception&) {
     ma_server_destroy(S);
     return ma::fail(MA_ERR_DEVICE, "ma_server_create: could not start threads");
@@ -751,6 +762,8 @@ extern "C" void ma_server_destroy(ma_server* S) {
   // built after the scheduler stopped
   for (Request* r : S->incoming) retire(S, r);
   S->incoming.clear();
+  for (hipStream_t st : S->streams)
+    if (st) (void)hipStreamDestroy(st);
   if (S->base) (void)hipFree(S->base);
   delete S;
 }

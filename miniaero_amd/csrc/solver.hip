@@ -1565,6 +1565,7 @@ struct Timing {
 struct ma_solver {
   ma_options opt;
   int device = 0;
+  bool own_stream = true;  // false: a server's, which outlives the solver
   hipStream_t stream = nullptr;
   DevMesh m{};
   TileMap t{};
@@ -4050,7 +4051,7 @@ extern "C" void ma_solver_destroy(ma_solver* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   drop_graphs(s);
   for (void* p : s->allocs) (void)hipFree(p);
-  if (s->stream) (void)hipStreamDestroy(s->stream);
+  if (s->stream && s->own_stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
 
@@ -4149,7 +4150,7 @@ ma_status plan_case(const ma_mesh_data* md, const ma_options* opt, PlannedCase**
 
 void destroy_plan(PlannedCase* pc) { delete pc; }
 
-ma_status create_from_plan(PlannedCase* pc, void* region, size_t region_bytes, ma_solver** out) {
+ma_status create_from_plan(PlannedCase* pc, void* region, size_t region_bytes, hipStream_t stream, ma_solver** out) {
   *out = nullptr;
   ma_solver* s = new (std::nothrow) ma_solver();
   if (!s) return ma::fail(MA_ERR_NOMEM, "serve: out of host memory");
@@ -4165,10 +4166,9 @@ ma_status create_from_plan(PlannedCase* pc, void* region, size_t region_bytes, m
     s->arena_size = region_bytes;
     (void)hipGetDevice(&s->device);
     (void)hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, s->device);
-    if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
-      st = ma::fail(MA_ERR_DEVICE, "hipStreamCreate failed");
-    else
-      st = build_planned(s, pc->lp->P);
+    s->stream = stream;
+    s->own_stream = false;
+    st = build_planned(s, pc->lp->P);
   } catch (const std::bad_alloc&) {
     st = ma::fail(MA_ERR_NOMEM, "serve: out of host memory");
   }
@@ -4379,5 +4379,7 @@ void solver_set_progress(ma_solver* s, int steps) {
 }
 
 int solver_cur(const ma_solver* s) { return s->cur; }
+
+void solver_set_stream(ma_solver* s, hipStream_t stream) { s->stream = stream; }
 
 }  // namespace ma
