@@ -1539,12 +1539,17 @@ struct TileShape {
   int b[3];
 };
 constexpr TileShape kDefaultShape = {{4, 8, 8}};
-// The default for a run with fewer cells than one default tile per CU: with
-// so few tiles a step's time is each tile's latency, and a quarter of the
-// faces per 256-thread workgroup shortens it (64x16x16 first-order Sod,
-// 16k cells: 77 -> 53 us per step as one graph, 81 -> 58 with a launch per
-// kernel; 2x4x4 and 2x2x4 tiles 56 us, 2x2x2 93 us)
+// The defaults for runs with fewer cells than one default tile per CU.  Up to
+// two 64-cell tiles per CU a step's time is each tile's latency, which a
+// quarter of the faces per workgroup shortens; the FP64 viscous flux kernel
+// holds two of their 384-thread workgroups per CU, and with more of them the
+// last ones wait for a second round, so the tiles then hold 128 cells.  k_flux
+// us, 4x4x4 / 4x4x8 / 4x8x8 tiles: FP64 viscous plates of 28k cells 14.0 / 15.1
+// / 15.6, 38k 19.0 / 16.4 / 16.5, 60k 23.6 / 16.9 / 16.4; second-order shock
+// tubes 9.2 / 10.7 / 11.5, 12.3 / 11.8 / 11.9, 15.5 / 12.5 / 12.4; ramps 12.2 /
+// 13.1 / 16.0, 15.3 / 13.7 / 17.1, 18.1 / 16.2 / 17.8.
 constexpr TileShape kSmallRunShape = {{4, 4, 4}};
+constexpr TileShape kMediumRunShape = {{4, 4, 8}};
 
 bool valid_shape(const TileShape& t) {
   if (t.b[0] == 0 && t.b[1] == 0 && t.b[2] == 0) return true;
@@ -3630,7 +3635,7 @@ ma_status create_run(int ncases, const ma_mesh_data* const* mds, const ma_option
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
         cells < (long long)cus * kTile)
-      tune.shape = kSmallRunShape;
+      tune.shape = cells <= (long long)cus * 128 ? kSmallRunShape : kMediumRunShape;
   }
   double tuned_ms = 0.0;
   if (!force && o0.autotune) {
