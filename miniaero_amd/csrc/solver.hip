@@ -959,10 +959,14 @@ __device__ __forceinline__ void flux_tile(const DevMesh& m, const TileMap& t, in
 template <class T>
 constexpr int kFluxWaves = sizeof(T) == 8 ? 3 : 5;
 
-// A step with fixed time steps has nothing to reduce before it, so no kernel of
-// its own advances the time: the last stage's flux workgroup of each case's
-// first tile does, from the same dt (a launch less per step, 3 of 24 us on a
-// 16k-cell shock tube).
+// A paired run's step with fixed time steps has nothing to reduce before it, so
+// no kernel of its own advances the time: the last stage's flux workgroup of
+// each case's first tile does, from the same dt (a launch less per step, 3 of
+// 24 us on a 16k-cell shock tube).  k_flux does not: with the table and the two
+// pointers live over its tile it keeps 10 to 20 more values of the scalar
+// registers in vector lanes, and its FP32 viscous forms wait for their loads in
+// more places (10k-cell FP32 viscous ramp 75.7 -> 84.1 us a step, launch saved
+// included).
 __device__ __forceinline__ void advance_time(const TileMap& t, int tile, const double* __restrict__ dt_dev,
                                              double* __restrict__ time_dev) {
   if (!time_dev || threadIdx.x != 0) return;
@@ -979,7 +983,7 @@ void k_flux(DevMesh m, TileMap t, const T* __restrict__ V,
             double* Uacc_out, double* __restrict__ R,
             const double* __restrict__ dt_dev, double beta,
             Inv inv, Visc visc, const double* __restrict__ Un, T* Vnext,
-            double alpha_next, int last, double* __restrict__ time_dev) {
+            double alpha_next, int last) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T* lds = reinterpret_cast<T*>(lds_raw);  // 5 planes of t.max_faces
   // XCD-aware order: the workgroups an XCD receives (every kXcds-th) take a
@@ -994,7 +998,6 @@ void k_flux(DevMesh m, TileMap t, const T* __restrict__ V,
     // the face-value scheme reads no gradients: its face values come in rec
     flux_tile<kSecondOrder, Inv, Visc, T>(m, t, tile, lds, V, rec, rec, bc, Uacc_in, Uacc_out, R, dt_dev, beta,
                                           inv, visc, Un, Vnext, alpha_next, last);
-    advance_time(t, tile, dt_dev, time_dev);
     __syncthreads();  // the LDS is reused by the next tile
   }
 }
@@ -3134,8 +3137,7 @@ void run_stage(ma_solver* s, int irk) {
   const int nb = nblocks(m.nc);
   double* Un = s->U[s->cur];
   double* Uacc = s->U[1 - s->cur];
-  double* time_dev = irk == 3 && !s->any_cfl ? s->time_dev : nullptr;  // see advance_time
-  // the stage's primitives: V for stages 0 and 2, V2 for 1 and 3; stage 0's
+    // the stage's primitives: V for stages 0 and 2, V2 for 1 and 3; stage 0's
   // come from k_prim, the others from the previous stage's flux kernel
   // (stage 3 writes the next step's stage-0 primitives into V, so k_prim
   // runs only when V does not hold them yet)
@@ -3166,6 +3168,7 @@ void run_stage(ma_solver* s, int irk) {
       });
     }
     constexpr bool kOwn = SO && Visc::isViscous;
+    double* time_dev = irk == 3 && !s->any_cfl ? s->time_dev : nullptr;  // see advance_time
     const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Inv, Visc, T>(s)
                       : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Inv, Visc, T>(s)
                                        : pair_flux_kernel<false, false, SO, Inv, Visc, T>(s);
@@ -3216,7 +3219,7 @@ void run_stage(ma_solver* s, int irk) {
                        s->stream, m, s->t, static_cast<const T*>(Vs), static_cast<const T*>(FV ? s->fv : s->grad),
                        static_cast<const T*>(s->bc), acc_in, Uacc, s->R,
                        s->dt_dev, beta[irk], inv, visc, Un, Vn, irk < 3 ? alpha[irk + 1] : alpha[0],
-                       irk == 3 ? 1 : 0, time_dev);
+                       irk == 3 ? 1 : 0);
   });
   if (irk == 3) s->v0_valid = true;  // V now holds the next step's stage-0 primitives
 }
@@ -3224,13 +3227,15 @@ void run_stage(ma_solver* s, int irk) {
 template <bool SO, class Inv, class Visc, class Lim, class T>
 void run_steps(ma_solver* s, int nsteps) {
   for (int it = 0; it < nsteps; ++it) {
-    // per-case dt (CFL minimum or fixed) and time += dt; without a CFL number
-    // dt stays as it is and the last stage advances the time
+    // per-case dt (CFL minimum or fixed) and time += dt; in paired runs without
+    // a CFL number dt stays as it is and the last stage advances the time
     if (s->any_cfl) {
       s->launch("k_dt_partial", [&] {
         hipLaunchKernelGGL(k_dt_partial, dim3(s->t.ntiles), dim3(kTile), 0, s->stream, s->m, s->t,
                            s->U[s->cur], s->opt.viscous, effective_prandtl(s->opt), s->partial);
       });
+    }
+    if (s->any_cfl || !s->pair) {
       s->launch("k_dt_final", [&] {
         hipLaunchKernelGGL(k_dt_final, dim3(s->ncases), dim3(kBlock), 0, s->stream, s->partial, s->case_tiles,
                            s->cfl_dev, s->dt_dev, s->time_dev);
