@@ -2342,7 +2342,11 @@ void find_pairs(Layout& L) {
         while (j < nk && j - i < 64 && inside == !(K[j].first >> 32)) {
           int e = j;  // whole blocks inside the tile, single faces otherwise
           while (e < nk && (e == j || (inside && block(e) == block(j)))) ++e;
-          if (e - i > 64) break;
+          if (e - i > 64) {
+            // a block has up to 192 faces of class kSkewFace: they fill chunks of their own
+            if (j == i) j = i + 64;
+            break;
+          }
           j = e;
         }
         chunks[inside ? d : kClasses].push_back({d, i});
