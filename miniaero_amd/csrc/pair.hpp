@@ -57,9 +57,14 @@
 
 // Waves per SIMD the paired flux kernels are register-budgeted for: the FP64
 // inviscid forms need a few more than the 128 registers that allow 4 unless
-// told to fit.
-template <class Visc, class T>
-constexpr int kPairFluxWaves = sizeof(T) == 4 ? 5 : Visc::isViscous ? 3 : 4;
+// told to fit.  Two for the FP64 viscous skew and first-order forms, which hold
+// averaged gradients over a whole face frame or without the second order's
+// ordered loads: at the 168 registers of three they spill 22 to 66 of them
+// (k_flux us at 590k cells, general kernel / three waves / two: rotated box
+// second order 123 / 183 / 130, first order 117 / 187 / 109; ramp 122 / 138 /
+// 118, 116 / 144 / 96; plate first order 90 / 90 / 73).
+template <bool kSkew, bool SO, class Visc, class T>
+constexpr int kPairFluxWaves = sizeof(T) == 4 ? 5 : Visc::isViscous ? (kSkew || !SO ? 2 : 3) : 4;
 
 constexpr int kSkewFace = 3;  // class of a tile's chunk of faces that are along no axis
 
@@ -880,7 +885,7 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
 // loop-carried values cost the FP64 viscous kernel spills and the FP64 inviscid
 // one ten registers.
 template <bool kSkew, bool kOwn, bool SO, bool kWall, bool kWalk, class Inv, class Visc, class T>
-__global__ __launch_bounds__(kPairMaxThreads) __attribute__((amdgpu_waves_per_eu(kPairFluxWaves<Visc, T>)))
+__global__ __launch_bounds__(kPairMaxThreads) __attribute__((amdgpu_waves_per_eu(kPairFluxWaves<kSkew, SO, Visc, T>)))
 void k_flux_pair(DevMesh m, TileMap t, const T* __restrict__ V, const T* __restrict__ rec,
                  const Inflow* __restrict__ inflows, const double* Uacc_in, double* Uacc_out,
                  double* __restrict__ R, const double* __restrict__ dt_dev, double beta, Inv inv, Visc visc,
