@@ -66,11 +66,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
+#include <iterator>
 #include <map>
 #include <limits>
 #include <memory>
@@ -78,7 +79,6 @@
 #include <new>
 #include <string>
 #include <thread>
-#include <unordered_map>
 #include <vector>
 
 #include "../../include/miniaero.h"
@@ -1721,8 +1721,8 @@ std::vector<int> processing_order(const ma_faces& F, int nc) {
   return perm;
 }
 
-template <class T>
-ma_status upload(ma_solver* s, T** dst, const std::vector<T>& h) {
+template <class T, class A>
+ma_status upload(ma_solver* s, T** dst, const std::vector<T, A>& h) {
   ma_status st = s->alloc(dst, h.size());
   if (st || s->counting) return st;
   MA_HIP(hipMemcpyAsync(*dst, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, s->stream));
@@ -1841,6 +1841,26 @@ void cell_order(const ma_mesh_data* md, const TileShape& shape, std::vector<int>
   }
 }
 
+// A vector whose new elements are left as they are, for tables that several
+// threads fill: filling them with a value first would touch every page on one.
+template <class T>
+struct RawAlloc : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = RawAlloc<U>;
+  };
+  template <class U>
+  void construct(U* p) {
+    ::new ((void*)p) U;
+  }
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new ((void*)p) U(std::forward<A>(a)...);
+  }
+};
+template <class T>
+using RawVector = std::vector<T, RawAlloc<T>>;
+
 // What the paired-mesh kernels (pair.hpp) read instead of the general slot
 // and tile tables; ok when the mesh is paired (find_pairs).
 struct PairPlan {
@@ -1849,10 +1869,12 @@ struct PairPlan {
   bool skew = false;                     // some face is along no axis: slots in slot order, kSkewFace chunks
   bool own = false;                      // a tile's list starts with whole blocks, see find_pairs
   int max_faces = 64;                    // longest tile list, padding included
-  std::vector<int> nbr, ent;             // kMaxSlots planes of nc: (low, high) along x, y, z; skew: as L.slot
+  std::vector<signed char> axis_of;      // while planning: axis of a geometry record's area vector, or kSkewFace
+  RawVector<int> nbr, ent;               // kMaxSlots planes of nc: (low, high) along x, y, z; skew: as L.slot
   std::vector<int> srec, frec;           // slot record -> geometry record << 1 | side; face record -> geometry record
-  std::vector<int> ptr, lr, gid;         // tile lists, lr 2 per entry (see flux_tile_pair)
-  std::vector<unsigned short> slot;      // kMaxSlots planes of nc: list index << 1 | side
+  std::vector<int> ptr;                  // tile lists
+  RawVector<int> lr, gid;                // their entries, lr 2 each (see flux_tile_pair)
+  RawVector<unsigned short> slot;        // kMaxSlots planes of nc: list index << 1 | side
 };
 
 // Everything the device needs, computed on the host (no GPU involved).
@@ -1876,8 +1898,59 @@ struct Layout {
   PairPlan pair;
 };
 
+// Host threads for planning one mesh of nc cells (cases of a batch are planned
+// side by side instead, one thread each).
+int plan_threads(int nc) {
+  return std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), 1 + nc / 8192}));
+}
+
+// fn(begin, end) for [0, n) in runs of `grain`, spread over up to `threads` host
+// threads; returns when all have run.  Where no more threads can be started the
+// ones there are do the work; an exception of fn is passed on.
+template <class F>
+void for_runs(int threads, int n, int grain, F&& fn) {
+  std::atomic<long long> next{0};
+  std::exception_ptr failed;
+  std::mutex mu;
+  auto work = [&] {
+    try {
+      for (long long i; (i = next.fetch_add(grain)) < n;) fn((int)i, (int)std::min<long long>(n, i + grain));
+    } catch (...) {
+      next = n;
+      std::lock_guard<std::mutex> lock(mu);
+      if (!failed) failed = std::current_exception();
+    }
+  };
+  std::vector<std::thread> pool;
+  try {
+    const int most = std::min(threads, (n + grain - 1) / grain);
+    pool.reserve((size_t)std::max(0, most));
+    for (int i = 1; i < most; ++i) pool.emplace_back(work);
+  } catch (const std::exception&) {
+  }
+  work();
+  for (auto& t : pool) t.join();
+  if (failed) std::rethrow_exception(failed);
+}
+
+// Class of a face in the tiles' lists: its axis, or kSkewFace where it is along
+// none or is an internal face pointing down its axis.
+inline int face_class(const Layout& L, int f) {
+  const int r = L.fgeo[f], d = L.pair.axis_of[r];
+  return d < kSkewFace && f < L.nif && L.geo[(size_t)r * kGeoVals + d] < 0.0 ? kSkewFace : d;
+}
+
+// The side of its left (side 0) or right cell that an axial face is on: twice
+// the axis, + 1 for the high side (2 * kSkewFace otherwise).
+inline int cell_side(const Layout& L, int f, int side) {
+  const int r = L.fgeo[f], d = L.pair.axis_of[r];
+  if (d == kSkewFace) return 2 * kSkewFace;
+  const double a = L.geo[(size_t)r * kGeoVals + d];
+  return 2 * d + ((side ? -a : a) > 0.0 ? 1 : 0);
+}
+
 // Every index the paired kernels will use, checked on the host before any upload.
-ma_status validate_pairs(const Layout& L) {
+ma_status validate_pairs(const Layout& L, int threads) {
   const PairPlan& P = L.pair;
   const int nc = L.nc, ntiles = L.ntiles;
   const size_t ng = L.geo.size() / kGeoVals;
@@ -1888,45 +1961,56 @@ ma_status validate_pairs(const Layout& L) {
       (int)P.ptr.size() != ntiles + 1 || P.gid.size() * 2 != P.lr.size() ||
       (size_t)P.ptr[ntiles] > P.gid.size() || (size_t)P.max_faces * 5 * sizeof(double) > 65536)
     return bad("sizes");
-  for (size_t i = 0; i < P.nbr.size(); ++i)
-    if (P.nbr[i] < 0 || P.nbr[i] >= nc || P.ent[i] < 0 || (size_t)low(P.ent[i]) >= P.srec.size()) return bad("slots");
   for (int x : P.srec)
     if (x < 0 || (size_t)(x >> 1) >= ng) return bad("slot records");
   for (int x : P.frec)
     if (x < 0 || (size_t)x >= ng) return bad("face records");
-  for (int b = 0; b < ntiles; ++b) {
+  std::atomic<const char*> wrong{nullptr};
+  for_runs(threads, nc, 4096, [&](int c0, int c1) {
+    for (int s = 0; s < kMaxSlots; ++s)
+      for (int c = c0; c < c1; ++c) {
+        const size_t i = (size_t)s * nc + c;
+        if (P.nbr[i] < 0 || P.nbr[i] >= nc || P.ent[i] < 0 || (size_t)low(P.ent[i]) >= P.srec.size()) wrong = "slots";
+      }
+  });
+  auto tile = [&](int b) -> const char* {
     const int f0 = P.ptr[b], n = P.ptr[b + 1] - f0;
-    if (n < 0 || n % 64 || n > P.max_faces) return bad("tile lists");
+    if (n < 0 || n % 64 || n > P.max_faces) return "tile lists";
     for (int q = f0; q < f0 + n; ++q) {
       const int x = P.lr[2 * (size_t)q], r = P.lr[2 * (size_t)q + 1], l = x < 0 ? -1 : x & ((1 << kCellBits) - 1);
       if (x >= 0 ? x >> kCellBits != P.lr[2 * (size_t)(q - (q - f0) % 64)] >> kCellBits || x >> kCellBits > (P.skew ? 3 : 2)
                  : (q - f0) % 64 == 0)
-        return bad("tile chunks");
+        return "tile chunks";
       if (l >= nc || low(r) >= nc || P.gid[q] < 0 || (size_t)low(P.gid[q]) >= P.frec.size() ||
           (l >= 0 && r < 0 && (~r >> 2) >= L.nbf))
-        return bad("tile faces");
+        return "tile faces";
       if (P.skew && l >= 0 && r >= 0 && (r >> kCellBits >= kMaxSlots || P.gid[q] >> kCellBits >= kMaxSlots))
-        return bad("tile face slots");
+        return "tile face slots";
     }
     const int cells = L.tile_cptr[b + 1] - L.tile_cptr[b];
-    if (P.own && (P.skew || n < (cells + 63) / 64 * 192)) return bad("own faces");
+    if (P.own && (P.skew || n < (cells + 63) / 64 * 192)) return "own faces";
     for (int i = 0; i < cells && P.own; ++i)
       for (int d = 0; d < 3; ++d)
         if (P.lr[2 * (size_t)(f0 + (i / 64 * 3 + d) * 64 + i % 64)] != ((L.tile_cptr[b] + i) | (d << kCellBits)))
-          return bad("own faces");
+          return "own faces";
     for (int c = L.tile_cptr[b]; c < L.tile_cptr[b + 1]; ++c)
       for (int s = 0; s < kMaxSlots; ++s) {
         const int e = P.slot[(size_t)s * nc + c], j = e >> 1;
         if (j >= n || P.lr[2 * (size_t)(f0 + j)] < 0 ||
             ((e & 1) ? low(P.lr[2 * (size_t)(f0 + j) + 1]) : P.lr[2 * (size_t)(f0 + j)] & ((1 << kCellBits) - 1)) != c)
-          return bad("tile slots");
+          return "tile slots";
       }
-  }
-  return MA_OK;
+    return nullptr;
+  };
+  for_runs(threads, ntiles, 32, [&](int b0, int b1) {
+    for (int b = b0; b < b1; ++b)
+      if (const char* w = tile(b)) wrong = w;
+  });
+  return wrong ? bad(wrong) : MA_OK;
 }
 
 // Every index a kernel will use, checked on the host before any upload.
-ma_status validate_layout(const Layout& L) {
+ma_status validate_layout(const Layout& L, int threads) {
   const int nc = L.nc, nif = L.nif, nf = L.nf, nbf = L.nbf, ntiles = L.ntiles;
   const std::vector<int>& dev_of = L.dev_of;
   const std::vector<int>& tile_cptr = L.tile_cptr;
@@ -1983,14 +2067,14 @@ ma_status validate_layout(const Layout& L) {
     }
   }
   }
-  return L.pair.ok ? validate_pairs(L) : MA_OK;
+  return L.pair.ok ? validate_pairs(L, threads) : MA_OK;
 }
 
 // Concatenation of independent cases' layouts into one: cells, internal faces,
 // boundary faces and tiles of case k follow those of case k-1; tiles never
 // span two cases.  Internal faces of all cases come before all boundary faces.
 void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile_case,
-                   std::vector<int>& case_tiles, std::vector<int>& bc_case, std::vector<int>& cell_case) {
+                   std::vector<int>& case_tiles, std::vector<int>& bc_case, std::vector<int>& cell_case, int threads) {
   const int n = (int)parts.size();
   std::vector<int> co(n + 1, 0), io(n + 1, 0), bo(n + 1, 0), to(n + 1, 0), qo(n + 1, 0);
   M.derive_frame = true;
@@ -2035,31 +2119,37 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
   for (int k = 0; k < n; ++k) {
     M.axis = M.axis && parts[k].axis;
     M.pair.ok = M.pair.ok && parts[k].pair.ok && parts[k].pair.skew == parts[0].pair.skew;
-    M.pair.fp32 = M.pair.fp32 && parts[k].pair.fp32;
     M.pair.own = M.pair.own && parts[k].pair.own;
     M.wall = M.wall || parts[k].wall;
   }
   M.pair.skew = parts[0].pair.skew;
-  size_t records = 0;
-  for (int k = 0; k < n; ++k) records += parts[k].pair.srec.size();
-  M.pair.ok = M.pair.ok && records < (1u << kCellBits);  // as in find_pairs
+  // where each part's geometry records, and its records and entries of the
+  // paired kernels' tables, start
+  std::vector<size_t> go(n + 1, 0), so(n + 1, 0), po(n + 1, 0), eo(n + 1, 0);
+  for (int k = 0; k < n; ++k) {
+    const PairPlan& P = parts[k].pair;
+    go[k + 1] = go[k] + parts[k].geo.size() / kGeoVals;
+    so[k + 1] = so[k] + P.srec.size();
+    po[k + 1] = po[k] + P.frec.size();
+    eo[k + 1] = eo[k] + P.gid.size();
+    M.pair.max_faces = std::max(M.pair.max_faces, P.max_faces);
+  }
+  M.geo.resize(go[n] * kGeoVals);
+  M.pair.ok = M.pair.ok && so[n] < (1u << kCellBits);  // as in list_pairs
   if (M.pair.ok) {
-    size_t entries = 0;
-    for (int k = 0; k < n; ++k) {
-      entries += parts[k].pair.gid.size();
-      M.pair.max_faces = std::max(M.pair.max_faces, parts[k].pair.max_faces);
-    }
-    for (auto* v : {&M.pair.nbr, &M.pair.ent}) v->assign((size_t)kMaxSlots * nc, 0);
-    M.pair.slot.assign((size_t)kMaxSlots * nc, 0);
-    M.pair.ptr.assign(1, 0);
-    M.pair.lr.reserve(2 * entries);
-    M.pair.gid.reserve(entries);
+    for (auto* v : {&M.pair.nbr, &M.pair.ent}) v->resize((size_t)kMaxSlots * nc);
+    M.pair.slot.resize((size_t)kMaxSlots * nc);
+    M.pair.ptr.assign((size_t)M.ntiles + 1, 0);
+    M.pair.lr.resize(2 * eo[n]);
+    M.pair.gid.resize(eo[n]);
+    M.pair.srec.resize(so[n]);
+    M.pair.frec.resize(po[n]);
   }
   tile_case.assign(M.ntiles, 0);
   case_tiles.assign(n + 1, 0);
   bc_case.assign(std::max(1, M.nbf), 0);
   cell_case.assign(nc, 0);
-  for (int k = 0; k < n; ++k) {
+  for_runs(threads, n, 1, [&](int k, int) {  // every part has places of its own
     Layout& L = parts[k];
     const int lnc = L.nc, lnif = L.nif, lnf = L.nf;
     auto gf = [&](int f) { return f < lnif ? io[k] + f : M.nif + bo[k] + (f - lnif); };
@@ -2109,34 +2199,33 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
       }
       if (f >= lnif) bc_case[bo[k] + (f - lnif)] = k;
     }
-    {  // this part's geometry records follow the earlier parts'
-      const int r0 = (int)(M.geo.size() / kGeoVals);
-      if (M.pair.ok) {
-        const PairPlan& P = L.pair;
-        const int s0 = (int)M.pair.srec.size(), p0 = (int)M.pair.frec.size();
-        for (int q = 0; q < kMaxSlots; ++q)
-          for (int c = 0; c < lnc; ++c) {
-            const size_t to_ = (size_t)q * nc + co[k] + c, from = (size_t)q * lnc + c;
-            M.pair.nbr[to_] = co[k] + P.nbr[from];
-            M.pair.ent[to_] = s0 + P.ent[from];
-            M.pair.slot[to_] = P.slot[from];
-          }
-        const int e0 = M.pair.ptr.back();
-        for (int b = 0; b < L.ntiles; ++b) M.pair.ptr.push_back(e0 + P.ptr[b + 1]);
-        for (size_t q = 0; q < P.gid.size(); ++q) {
-          const int l = P.lr[2 * q], r = P.lr[2 * q + 1];
-          M.pair.lr.push_back(l < 0 ? l : co[k] + l);
-          M.pair.lr.push_back(l < 0 ? r : r >= 0 ? co[k] + r : ~(~r + (bo[k] << 2)));
-          M.pair.gid.push_back(p0 + P.gid[q]);
+    const int r0 = (int)go[k];
+    for (int f = 0; f < lnf; ++f) M.fgeo[gf(f)] = r0 + L.fgeo[f];
+    std::copy(L.geo.begin(), L.geo.end(), M.geo.begin() + go[k] * kGeoVals);
+    if (M.pair.ok) {
+      const PairPlan& P = L.pair;
+      PairPlan& T = M.pair;
+      const int s0 = (int)so[k], p0 = (int)po[k];
+      const size_t e0 = eo[k];
+      for (int q = 0; q < kMaxSlots; ++q)
+        for (int c = 0; c < lnc; ++c) {
+          const size_t to_ = (size_t)q * nc + co[k] + c, from = (size_t)q * lnc + c;
+          T.nbr[to_] = co[k] + P.nbr[from];
+          T.ent[to_] = s0 + P.ent[from];
+          T.slot[to_] = P.slot[from];
         }
-        for (int x : P.srec) M.pair.srec.push_back(x + 2 * r0);
-        for (int x : P.frec) M.pair.frec.push_back(x + r0);
+      for (int b = 0; b < L.ntiles; ++b) T.ptr[to[k] + b + 1] = (int)e0 + P.ptr[b + 1];
+      for (size_t q = 0; q < P.gid.size(); ++q) {
+        const int l = P.lr[2 * q], r = P.lr[2 * q + 1];
+        T.lr[2 * (e0 + q)] = l < 0 ? l : co[k] + l;
+        T.lr[2 * (e0 + q) + 1] = l < 0 ? r : r >= 0 ? co[k] + r : ~(~r + (bo[k] << 2));
+        T.gid[e0 + q] = p0 + P.gid[q];
       }
-      for (int f = 0; f < lnf; ++f) M.fgeo[gf(f)] = r0 + L.fgeo[f];
-      M.geo.insert(M.geo.end(), L.geo.begin(), L.geo.end());
+      for (size_t x = 0; x < P.srec.size(); ++x) T.srec[so[k] + x] = P.srec[x] + 2 * r0;
+      for (size_t x = 0; x < P.frec.size(); ++x) T.frec[po[k] + x] = P.frec[x] + r0;
     }
     Layout().swap_out(L);  // release the part as soon as it is merged
-  }
+  });
 }
 
 // Geometry records of the faces, which the flux and gradient kernels read:
@@ -2152,19 +2241,46 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
 // its own record (record f for face f).
 constexpr int kGeoReuse = 8;
 
-struct GeoKeyHash {
-  size_t operator()(const std::array<unsigned long long, kGeoVals>& k) const {
-    unsigned long long h = 1469598103934665603ull;
-    for (unsigned long long x : k) {
-      h ^= x;
-      h *= 1099511628211ull;
+// Records by their bits: open addressing, at most half full (an
+// std::unordered_map of the nine values took over half of a mesh's planning).
+class GeoTable {
+ public:
+  // Number of the record r, appended to geo when it is new.
+  int find(const double* r, std::vector<double>& geo) {
+    if (2 * count_ >= slots_.size()) grow(geo);
+    for (size_t i = hash(r) & (slots_.size() - 1);; i = (i + 1) & (slots_.size() - 1)) {
+      if (slots_[i] < 0) {
+        geo.insert(geo.end(), r, r + kGeoVals);
+        return slots_[i] = (int)count_++;
+      }
+      if (!std::memcmp(&geo[(size_t)slots_[i] * kGeoVals], r, kGeoVals * sizeof(double))) return slots_[i];
+    }
+  }
+  size_t size() const { return count_; }
+
+ private:
+  static size_t hash(const double* r) {
+    unsigned long long x[kGeoVals], h = 1469598103934665603ull;
+    std::memcpy(x, r, sizeof x);
+    for (unsigned long long v : x) {
+      h = (h ^ v) * 1099511628211ull;
       h ^= h >> 29;
     }
-    return (size_t)h;
+    return (size_t)(h ^ (h >> 32));
   }
+  void grow(const std::vector<double>& geo) {
+    slots_.assign(std::max<size_t>(1024, 4 * slots_.size()), -1);
+    for (size_t k = 0; k < count_; ++k) {
+      size_t i = hash(&geo[k * kGeoVals]) & (slots_.size() - 1);
+      while (slots_[i] >= 0) i = (i + 1) & (slots_.size() - 1);
+      slots_[i] = (int)k;
+    }
+  }
+  std::vector<int> slots_;
+  size_t count_ = 0;
 };
 
-void dedupe_geometry(Layout& L) {
+void dedupe_geometry(Layout& L, int threads) {
   const int nf = L.nf, nc = L.nc;
   L.axis = true;
   for (int f = 0; f < nf && L.axis; ++f)
@@ -2182,37 +2298,31 @@ void dedupe_geometry(Layout& L) {
   L.fgeo.assign((size_t)nf, 0);
   L.geo.clear();
   const size_t cap = std::min<size_t>((size_t)nf / kGeoReuse, size_t(1) << 20);
-  std::unordered_map<std::array<unsigned long long, kGeoVals>, int, GeoKeyHash> ids;
-  ids.reserve(std::min<size_t>(cap, 1 << 16) * 2);
+  GeoTable ids;
   bool shared = nf >= kGeoReuse;
   for (int f = 0; shared && f < nf; ++f) {
     double r[kGeoVals];
     record(f, r);
-    std::array<unsigned long long, kGeoVals> key;
-    std::memcpy(key.data(), r, sizeof r);
-    const auto it = ids.emplace(key, (int)ids.size());
-    if (it.second) {
-      if (ids.size() > cap) shared = false;  // too few repeats
-      L.geo.insert(L.geo.end(), r, r + kGeoVals);
-    }
-    L.fgeo[f] = it.first->second;
+    L.fgeo[f] = ids.find(r, L.geo);
+    shared = ids.size() <= cap;  // (else: too few repeats)
   }
   if (shared) return;
-  L.geo.assign((size_t)kGeoVals * nf, 0.0);
-  for (int f = 0; f < nf; ++f) {
-    record(f, &L.geo[(size_t)kGeoVals * f]);
-    L.fgeo[f] = f;
-  }
+  L.geo.resize((size_t)kGeoVals * nf);
+  for_runs(threads, nf, 16384, [&](int f0, int f1) {
+    for (int f = f0; f < f1; ++f) {
+      record(f, &L.geo[(size_t)kGeoVals * f]);
+      L.fgeo[f] = f;
+    }
+  });
 }
 
-// Whether the paired kernels take the mesh, and their tables.  Every cell must
-// have six faces, frames must follow from the area vectors, and the geometry
-// must be inside the bounds under which the quotients of a tame stage (pair.hpp)
-// stay in the normal range.  The mesh is axial if every cell has two faces per
-// axis, one on its low side and one on its high side, and every area vector
-// has exactly one nonzero component, positive on internal faces (left to right
-// is up the axis); otherwise it is skew, and its axial faces are still listed
-// by axis.
+// Whether the paired kernels take the mesh.  Every cell must have six faces,
+// frames must follow from the area vectors, and the geometry must be inside the
+// bounds under which the quotients of a tame stage (pair.hpp) stay in the normal
+// range.  The mesh is axial if every cell has two faces per axis, one on its low
+// side and one on its high side, and every area vector has exactly one nonzero
+// component, positive on internal faces (left to right is up the axis);
+// otherwise it is skew, and its axial faces are still listed by axis.
 // Bounds: largest |area| component in [2^-37, 2^100] and none but zeros below
 // 2^-37 (2^-150 in the FP64 form), volume in [2^-100, 2^24], displacements at
 // most 2^50 with squared length at least 2^-56, and largest area times largest
@@ -2220,71 +2330,95 @@ void dedupe_geometry(Layout& L) {
 // is at most 2^18 times the largest primitive: FP64 limiter terms stay below
 // 2^(3 (100 + 18) + 6), FP32 ones, scaled by 2^24, below 2^(3 (16 + 18) + 2 + 24)
 // and so in range, and an FP32 limiter is at least 2^-56 / 2^(2 (16 + 18) + 2).
-void find_pairs(Layout& L) {
+// The runs of the loops are spread over host threads: on one, planning a mesh
+// cost up to half as much again as without the paired kernels' tables.
+void find_pairs(Layout& L, int threads) {
   PairPlan& P = L.pair;
   P = PairPlan();
-  const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
+  const int nc = L.nc, nif = L.nif, nf = L.nf;
   if (!L.derive_frame) return;
   const size_t ng = L.geo.size() / kGeoVals;
-  std::vector<signed char> axis_of(ng, -1);
-  std::vector<double> amax(ng), dmax(ng);
-  for (size_t r = 0; r < ng; ++r) {
-    const double* q = &L.geo[r * kGeoVals];
-    for (int d = 0; d < 3; ++d) {
-      const double a = std::fabs(q[d]);
-      if (a != 0.0) axis_of[r] = axis_of[r] < 0 ? (signed char)d : (signed char)kSkewFace;
-      if (a != 0.0 && !(a >= 0x1p-150)) return;
-      if (a != 0.0 && !(a >= 0x1p-37)) P.fp32 = false;
-      amax[r] = std::max(amax[r], a);
-    }
-    if (!(amax[r] >= 0x1p-37 && amax[r] <= 0x1p100)) return;
-    for (int k = 3; k < 9; ++k) dmax[r] = std::max(dmax[r], std::fabs(q[k]));
-    if (!(dmax[r] <= 0x1p50) || !(q[3] * q[3] + q[4] * q[4] + q[5] * q[5] >= 0x1p-56)) return;
-  }
-  auto cls = [&](int f) -> int {  // axis, or kSkewFace
-    const int d = axis_of[L.fgeo[f]];
-    return d < kSkewFace && f < nif && L.geo[(size_t)L.fgeo[f] * kGeoVals + d] < 0.0 ? kSkewFace : d;
-  };
-  for (int f = 0; f < nif; ++f) {
-    const double* q = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
-    if (!(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) return;
-  }
-  for (int f = 0; f < nf; ++f) P.skew = P.skew || cls(f) == kSkewFace;
-  P.nbr.assign((size_t)kMaxSlots * nc, -1);
-  P.ent.assign((size_t)kMaxSlots * nc, -1);
-  std::vector<int> fslot(2 * (size_t)nf, 0);  // a face's slot in its left and its right cell
-  for (int c = 0; c < nc; ++c) {
-    double am = 0.0, dm = 0.0;
-    for (int q = 0; q < kMaxSlots; ++q) {
-      const int e = L.slot[(size_t)q * nc + c];
-      if (e < 0) {
-        P = PairPlan();
-        return;
+  P.axis_of.assign(ng, -1);
+  std::vector<double> amax(ng, 0.0), dmax(ng, 0.0);
+  std::atomic<bool> out{false}, skew{false}, fp32{true};  // out: outside the bounds
+  for_runs(threads, (int)ng, 4096, [&](int r0, int r1) {
+    for (int r = r0; r < r1 && !out; ++r) {
+      const double* q = &L.geo[(size_t)r * kGeoVals];
+      for (int d = 0; d < 3; ++d) {
+        const double a = std::fabs(q[d]);
+        if (a != 0.0) P.axis_of[r] = P.axis_of[r] < 0 ? (signed char)d : (signed char)kSkewFace;
+        if (a != 0.0 && !(a >= 0x1p-150)) out = true;
+        if (a != 0.0 && !(a >= 0x1p-37)) fp32 = false;
+        amax[r] = std::max(amax[r], a);
       }
-      const int f = e >> 1, side = e & 1, r = L.fgeo[f], d = axis_of[r];
-      am = std::max(am, amax[r]);
-      dm = std::max(dm, dmax[r]);
-      if (P.skew) continue;
-      const double a = L.geo[(size_t)r * kGeoVals + d];
-      const int s = 2 * d + ((side ? -a : a) > 0.0 ? 1 : 0);
-      // (two faces on one side: the cell's slots are not one per direction)
-      if (P.ent[(size_t)s * nc + c] >= 0) P.skew = true;
-      P.ent[(size_t)s * nc + c] = (r << 1) | side;
-      P.nbr[(size_t)s * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
+      if (!(amax[r] >= 0x1p-37 && amax[r] <= 0x1p100)) out = true;
+      for (int k = 3; k < 9; ++k) dmax[r] = std::max(dmax[r], std::fabs(q[k]));
+      if (!(dmax[r] <= 0x1p50) || !(q[3] * q[3] + q[4] * q[4] + q[5] * q[5] >= 0x1p-56)) out = true;
     }
-    if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) {
-      P = PairPlan();
-      return;
+  });
+  if (out) return;
+  for_runs(threads, nf, 16384, [&](int f0, int f1) {
+    for (int f = f0; f < f1 && !out; ++f) {
+      const double* q = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
+      if (f < nif && !(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) out = true;
+      if (face_class(L, f) == kSkewFace) skew = true;
     }
-  }
-  if (P.skew)
-    for (int c = 0; c < nc; ++c)
+  });
+  if (out) return;
+  for_runs(threads, nc, 4096, [&](int c0, int c1) {
+    for (int c = c0; c < c1 && !out; ++c) {
+      double am = 0.0, dm = 0.0;
+      unsigned sides = 0;
       for (int q = 0; q < kMaxSlots; ++q) {
-        const int e = L.slot[(size_t)q * nc + c], f = e >> 1, side = e & 1;
-        P.ent[(size_t)q * nc + c] = (L.fgeo[f] << 1) | side;
-        P.nbr[(size_t)q * nc + c] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
-        fslot[2 * (size_t)f + side] = q;
+        const int e = L.slot[(size_t)q * nc + c];
+        if (e < 0) {
+          out = true;
+          return;
+        }
+        const int f = e >> 1, r = L.fgeo[f];
+        am = std::max(am, amax[r]);
+        dm = std::max(dm, dmax[r]);
+        if (!skew) sides |= 1u << cell_side(L, f, e & 1);
       }
+      if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) out = true;
+      if (sides != 0x3f) skew = true;  // (two faces on one side: the cell's slots are not one per direction)
+    }
+  });
+  if (out) return;
+  P.fp32 = fp32;
+  P.skew = skew;
+  P.ok = true;
+}
+
+// The paired kernels' tables of a mesh that find_pairs took (P.ok is cleared if
+// a list is too long).
+void list_pairs(Layout& L, int threads) {
+  PairPlan& P = L.pair;
+  const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
+  const size_t ng = L.geo.size() / kGeoVals;
+  const int* fslot = nullptr;  // skew: a face's slot in its left and its right cell
+  std::vector<int> fslots;
+  if (P.skew) {
+    fslots.assign(2 * (size_t)nf, 0);
+    fslot = fslots.data();
+  }
+  P.nbr.resize((size_t)kMaxSlots * nc);
+  P.ent.resize((size_t)kMaxSlots * nc);
+  std::vector<int> tile_of(nc);
+  for_runs(threads, nc, 4096, [&](int c0, int c1) {
+    for (int q = 0; q < kMaxSlots; ++q)
+      for (int c = c0; c < c1; ++c) {
+        const int e = L.slot[(size_t)q * nc + c], f = e >> 1, side = e & 1;
+        const size_t at = (size_t)(P.skew ? q : cell_side(L, f, side)) * nc + c;
+        P.ent[at] = (L.fgeo[f] << 1) | side;
+        P.nbr[at] = f < nif ? (side ? L.fl[f] : L.fr[f]) : c;
+        if (P.skew) fslots[2 * (size_t)f + side] = q;
+      }
+  });
+  for (int b = 0; b < ntiles; ++b) {
+    std::fill(tile_of.begin() + L.tile_cptr[b], tile_of.begin() + L.tile_cptr[b + 1], b);
+    P.own = P.own || (!P.skew && L.tile_cptr[b + 1] - L.tile_cptr[b] > 128);
+  }
   // Tile lists in chunks of 64 entries of one axis: the faces inside the tile
   // by left cell, a chunk per axis and block of 64 cells (blocks with few
   // faces share one), then the faces shared with other tiles (low side, high
@@ -2295,140 +2429,170 @@ void find_pairs(Layout& L) {
   // before the others, so that a wavefront can keep a cell's own values over
   // its three faces.  Tiles of at most 128 cells, which are few wavefronts'
   // work, spread their chunks over all of them instead.
-  std::vector<int> tile_of(nc);
-  for (int b = 0; b < ntiles; ++b)
-    for (int d = L.tile_cptr[b]; d < L.tile_cptr[b + 1]; ++d) tile_of[d] = b;
-  for (int b = 0; b < ntiles; ++b) P.own = P.own || (!P.skew && L.tile_cptr[b + 1] - L.tile_cptr[b] > 128);
-  P.ptr.assign(1, 0);
-  P.slot.assign((size_t)kMaxSlots * nc, 0);
-  std::vector<int> pos(nf);  // list index of a face in the tile being built
-  std::vector<int> faces;    // the lists' faces
-  using Key = std::pair<unsigned long long, int>;
   constexpr int kClasses = kSkewFace + 1;
-  std::vector<Key> keys[kClasses];
-  std::vector<std::pair<int, int>> chunks[kClasses + 1];  // (class, first key), by class; shared and boundary faces
-  std::vector<int> lens[kClasses + 1];
-  for (int b = 0; b < ntiles; ++b) {
-    const int c0 = L.tile_cptr[b], c1 = L.tile_cptr[b + 1];
-    for (auto& k : keys) k.clear();
-    auto add = [&](int f, int place, int cell) {
-      keys[cls(f)].push_back({((unsigned long long)place << 32) | (unsigned)cell, f});
-    };
-    for (int q = L.tptr[b]; q < L.tptr[b + 1]; ++q) {
-      const int f = L.tfaces[q], l = L.fl[f], r = L.fr[f];
-      const bool inl = tile_of[l] == b, inr = tile_of[r] == b;
-      add(f, (inl && inr) || (P.own && inl) ? 0 : inr ? 1 : 2, inl ? l : r);
-    }
-    for (int c = c0; c < c1; ++c)
-      for (int q = 0; q < kMaxSlots; ++q) {
-        const int f = L.slot[(size_t)q * nc + c] >> 1;
-        if (f >= nif) {
-          const double* a = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
-          add(f, P.own && a[0] + a[1] + a[2] > 0.0 ? 0 : 3, c);  // (own: an axial mesh)
-        }
+  struct Item {
+    int cell, f, loc;  // loc: the face's place in L.tfaces of the tile, ~its boundary number
+    bool operator<(const Item& o) const { return cell != o.cell ? cell < o.cell : f < o.f; }
+  };
+  struct Chunk {
+    const std::vector<Item>* from;
+    int cls, first, len;
+  };
+  constexpr int kTileRun = 32;  // tiles of a run
+  struct Run {
+    std::vector<int> lr, gid, len;
+  };
+  std::vector<Run> runs((ntiles + kTileRun - 1) / kTileRun);
+  std::vector<int> bpos(nf - nif);  // list index of a boundary face in its tile
+  P.slot.resize((size_t)kMaxSlots * nc);
+  std::atomic<bool> too_long{false};
+  for_runs(threads, ntiles, kTileRun, [&](int b0, int b1) {
+    Run& R = runs[b0 / kTileRun];
+    // by class: faces inside the tile (own: every high face of its cells), the
+    // boundary faces among them, faces with only their right cell in the tile,
+    // with only their left one, other boundary faces
+    std::vector<Item> inside[kClasses], inside_b[kClasses], low[kClasses], high[kClasses], outer[kClasses],
+        merged[kClasses];
+    std::vector<Chunk> chunks[kClasses + 1];
+    std::vector<int> pos;  // list index of an internal face, by its place in L.tfaces
+    for (int b = b0; b < b1 && !too_long; ++b) {
+      const int c0 = L.tile_cptr[b], c1 = L.tile_cptr[b + 1];
+      for (int d = 0; d < kClasses; ++d)
+        for (auto* v : {&inside[d], &inside_b[d], &low[d], &high[d], &outer[d], &merged[d]}) v->clear();
+      // internal faces come in the order of their left cells, boundary faces in
+      // that of their cells; only the low ones need sorting
+      for (int q = L.tptr[b]; q < L.tptr[b + 1]; ++q) {
+        const int f = L.tfaces[q], l = L.fl[f], d = face_class(L, f);
+        const bool inl = tile_of[l] == b, inr = tile_of[L.fr[f]] == b;
+        auto& to = (inl && inr) || (P.own && inl) ? inside[d] : inr ? low[d] : high[d];
+        to.push_back({inl ? l : L.fr[f], f, q - L.tptr[b]});
       }
-    for (int q = 0; q <= kClasses; ++q) {
-      chunks[q].clear();
-      lens[q].clear();
-    }
-    for (int d = 0; d < kClasses; ++d) {
-      std::vector<Key>& K = keys[d];
-      std::sort(K.begin(), K.end());
-      auto block = [&](int i) { return (K[i].first >> 32) ? 1 << 30 : ((int)(K[i].first & 0xffffffffu) - c0) / 64; };
-      const int nk = (int)K.size();
-      for (int i = 0; i < nk;) {
-        int j = i;
-        const bool inside = !(K[i].first >> 32);
-        while (j < nk && j - i < 64 && inside == !(K[j].first >> 32)) {
-          int e = j;  // whole blocks inside the tile, single faces otherwise
-          while (e < nk && (e == j || (inside && block(e) == block(j)))) ++e;
-          if (e - i > 64) {
-            // a block has up to 192 faces of class kSkewFace: they fill chunks of their own
-            if (j == i) j = i + 64;
-            break;
+      for (int c = c0; c < c1; ++c)
+        for (int q = 0; q < kMaxSlots; ++q) {
+          const int f = L.slot[(size_t)q * nc + c] >> 1;
+          if (f < nif) continue;
+          const int d = face_class(L, f);
+          auto& to = P.own && (cell_side(L, f, 0) & 1) ? inside_b[d] : outer[d];
+          to.push_back({c, f, ~(f - nif)});
+        }
+      for (auto& v : chunks) v.clear();
+      for (int d = 0; d < kClasses; ++d) {
+        if (!inside_b[d].empty())
+          std::merge(inside[d].begin(), inside[d].end(), inside_b[d].begin(), inside_b[d].end(),
+                     std::back_inserter(merged[d]));
+        std::sort(low[d].begin(), low[d].end());
+        for (auto* v : {&high[d], &outer[d]}) low[d].insert(low[d].end(), v->begin(), v->end());
+        const std::vector<Item>&K = inside_b[d].empty() ? inside[d] : merged[d], &S = low[d];
+        const int nk = (int)K.size(), nsh = (int)S.size();
+        for (int i = 0; i < nk;) {
+          int j = i;
+          while (j < nk && j - i < 64) {  // whole blocks of 64 cells
+            int e = j;
+            while (e < nk && (K[e].cell - c0) / 64 == (K[j].cell - c0) / 64) ++e;
+            if (e - i > 64) {
+              if (j == i) j = i + 64;  // (a block with more faces of one class than a chunk holds)
+              break;
+            }
+            j = e;
           }
-          j = e;
+          chunks[d].push_back({&K, d, i, j - i});
+          i = j;
         }
-        chunks[inside ? d : kClasses].push_back({d, i});
-        lens[inside ? d : kClasses].push_back(j - i);
-        i = j;
+        for (int i = 0; i < nsh; i += 64) chunks[kClasses].push_back({&S, d, i, std::min(64, nsh - i)});
       }
-    }
-    int n = 0;
-    const size_t blocks = P.own ? chunks[0].size() : 0;  // (own: as many of every axis)
-    for (size_t r = 0, left = 1; left; ++r) {
-      left = 0;
-      for (int q = 0; q <= kClasses; ++q) {
-        if (P.own && (q == kClasses) != (r >= blocks)) {
-          left |= q == kClasses;
-          continue;
-        }
-        if ((q == kClasses ? r - blocks : r) >= chunks[q].size()) continue;
-        left = 1;
-        const size_t x = q == kClasses ? r - blocks : r;
-        const int d = chunks[q][x].first, i = chunks[q][x].second;
-        for (int k = i; k < i + lens[q][x]; ++k) {
-          const int f = keys[d][k].second;
-          pos[f] = n++;
-          P.lr.push_back(L.fl[f] | (d << kCellBits));
-          P.lr.push_back(f >= nif  ? ~(((f - nif) << 2) | (L.fkind[f] - 1))
+      pos.assign((size_t)(L.tptr[b + 1] - L.tptr[b]), 0);
+      int n = 0;
+      auto put = [&](const Chunk& k) {
+        for (int i = k.first; i < k.first + k.len; ++i) {
+          const Item& x = (*k.from)[i];
+          const int f = x.f;
+          (x.loc < 0 ? bpos[~x.loc] : pos[x.loc]) = n++;
+          R.lr.push_back(L.fl[f] | (k.cls << kCellBits));
+          R.lr.push_back(f >= nif  ? ~(((f - nif) << 2) | (L.fkind[f] - 1))
                          : P.skew ? L.fr[f] | (fslot[2 * (size_t)f + 1] << kCellBits)
                                   : L.fr[f]);
-          P.gid.push_back(L.fgeo[f]);  // (skew meshes: with the left cell's slot, below)
-          faces.push_back(f);
+          R.gid.push_back(L.fgeo[f] | (P.skew ? fslot[2 * (size_t)f] << kCellBits : 0));
         }
         for (; n % 64; ++n) {
-          P.lr.push_back(-1);
-          P.lr.push_back(-1);
-          P.gid.push_back(0);
-          faces.push_back(-1);
+          R.lr.push_back(-1);
+          R.lr.push_back(-1);
+          R.gid.push_back(0);
         }
+      };
+      size_t most = 0;
+      for (const auto& v : chunks) most = std::max(most, v.size());
+      for (size_t r = 0; r < most; ++r)
+        for (int q = 0; q < kClasses + (P.own ? 0 : 1); ++q)
+          if (r < chunks[q].size()) put(chunks[q][r]);
+      if (P.own)
+        for (const Chunk& k : chunks[kClasses]) put(k);
+      R.len.push_back(n);
+      if ((size_t)n * 5 * sizeof(double) > 65536) too_long = true;  // e.g. long thin tiles of consecutive cells
+      // summation order: internal faces in slot order, then the boundary faces
+      // by kind (in slot order within a kind), the order of TimeSolverExplicitRK4.h:428-475
+      for (int c = c0; c < c1; ++c) {
+        int w = 0;
+        auto add = [&](int at, int side) { P.slot[(size_t)w++ * nc + c] = (unsigned short)((at << 1) | side); };
+        int q = 0;
+        for (; q < kMaxSlots; ++q) {  // (the boundary faces follow the internal ones)
+          const int e = L.slot[(size_t)q * nc + c];
+          if (e >> 1 >= nif) break;
+          add(pos[L.tslot[(size_t)q * nc + c] >> 3], e & 1);
+        }
+        const int q0 = q;
+        for (int kind = 1; kind <= MA_BC_INFLOW && w < kMaxSlots; ++kind)
+          for (q = q0; q < kMaxSlots; ++q) {
+            const int f = L.slot[(size_t)q * nc + c] >> 1;
+            if (L.fkind[f] == kind) add(bpos[f - nif], 0);
+          }
       }
     }
-    P.ptr.push_back(P.ptr.back() + n);
-    P.max_faces = std::max(P.max_faces, n);
-    if ((size_t)P.max_faces * 5 * sizeof(double) > 65536) {  // e.g. long thin tiles of consecutive cells
-      P = PairPlan();
-      return;
-    }
-    // summation order: internal faces in slot order, then the boundary faces
-    // by kind (in slot order within a kind), the order of TimeSolverExplicitRK4.h:428-475
-    for (int c = c0; c < c1; ++c) {
-      int w = 0;
-      for (int kind = 0; kind <= MA_BC_INFLOW; ++kind)
-        for (int q = 0; q < kMaxSlots; ++q) {
-          const int e = L.slot[(size_t)q * nc + c], f = e >> 1;
-          if ((f < nif ? 0 : L.fkind[f]) != kind) continue;
-          P.slot[(size_t)w++ * nc + c] = (unsigned short)((pos[f] << 1) | (e & 1));
-        }
-    }
+  });
+  if (too_long) {
+    P = PairPlan();
+    return;
   }
-  // records renumbered in the order the kernels meet them
-  auto renumber = [](std::vector<int>& ids, size_t most, std::vector<int>& rec) {
+  P.ptr.assign(1, 0);
+  for (const Run& R : runs)
+    for (int n : R.len) {
+      P.ptr.push_back(P.ptr.back() + n);
+      P.max_faces = std::max(P.max_faces, n);
+    }
+  P.lr.resize(2 * (size_t)P.ptr.back());
+  P.gid.resize((size_t)P.ptr.back());
+  for_runs(threads, (int)runs.size(), 1, [&](int r0, int r1) {
+    for (int r = r0; r < r1; ++r) {
+      const size_t to = (size_t)P.ptr[(size_t)r * kTileRun];
+      std::copy(runs[r].lr.begin(), runs[r].lr.end(), P.lr.begin() + 2 * to);
+      std::copy(runs[r].gid.begin(), runs[r].gid.end(), P.gid.begin() + to);
+      runs[r] = Run();
+    }
+  });
+  // records renumbered in the order the kernels meet them (above kCellBits a
+  // skew mesh's gid has the face's slot in its left cell, ent the cell's side)
+  auto renumber = [](RawVector<int>& ids, size_t most, int mask, std::vector<int>& rec) {
     std::vector<int> now(most, -1);
     for (int& x : ids) {
-      if (now[x] < 0) {
-        now[x] = (int)rec.size();
-        rec.push_back(x);
+      const int k = x & mask;
+      if (now[k] < 0) {
+        now[k] = (int)rec.size();
+        rec.push_back(k);
       }
-      x = now[x];
+      x = now[k] | (x & ~mask);
     }
   };
-  renumber(P.ent, 2 * ng, P.srec);
-  renumber(P.gid, ng, P.frec);
+  renumber(P.ent, 2 * ng, -1, P.srec);
+  renumber(P.gid, ng, (1 << kCellBits) - 1, P.frec);
   if (P.srec.size() >= (1u << kCellBits)) {  // 32-bit byte offsets into the record planes
     P = PairPlan();
     return;
   }
-  if (P.skew) {
+  if (P.skew)
     for (int& x : P.ent) x |= (P.srec[x] & 1) << kCellBits;
-    for (size_t q = 0; q < faces.size(); ++q)
-      if (faces[q] >= 0) P.gid[q] |= fslot[2 * (size_t)faces[q]] << kCellBits;
-  }
-  P.ok = true;
+  std::vector<signed char>().swap(P.axis_of);
 }
 
-ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, bool pairs, Layout& L) {
+ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, int threads, Layout& L) {
   const int nc = md->num_owned_cells;
   L.nc = nc;
   const ma_faces& I = md->internal_faces;
@@ -2493,17 +2657,20 @@ ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, bool pairs
   // Area vector and centroid of every face; whether every stored tangent
   // and binormal follow from the area vector as Face.C builds them (then the
   // kernels rebuild the frame and no frame array is stored).
-  auto derivable = [](const ma_faces& F) {  // in the caller's order (sequential reads)
-    for (int i = 0; i < F.nfaces; ++i) {
-      double t[3], b[3];
-      ma::tangent_binormal(&F.face_normal[3 * i], t, b);
-      for (int d = 0; d < 3; ++d)
-        if (t[d] != F.face_tangent[3 * i + d] || b[d] != F.face_binormal[3 * i + d] ||
-            std::signbit(t[d]) != std::signbit(F.face_tangent[3 * i + d]) ||
-            std::signbit(b[d]) != std::signbit(F.face_binormal[3 * i + d]))
-          return false;
-    }
-    return true;
+  auto derivable = [&](const ma_faces& F) {  // in the caller's order (sequential reads)
+    std::atomic<bool> all{true};
+    for_runs(threads, F.nfaces, 16384, [&](int i0, int i1) {
+      for (int i = i0; i < i1 && all; ++i) {
+        double t[3], b[3];
+        ma::tangent_binormal(&F.face_normal[3 * i], t, b);
+        for (int d = 0; d < 3; ++d)
+          if (t[d] != F.face_tangent[3 * i + d] || b[d] != F.face_binormal[3 * i + d] ||
+              std::signbit(t[d]) != std::signbit(F.face_tangent[3 * i + d]) ||
+              std::signbit(b[d]) != std::signbit(F.face_binormal[3 * i + d]))
+            all = false;
+      }
+    });
+    return all.load();
   };
   L.derive_frame = derivable(I);
   for (int g = 0; g < md->num_boundary_groups && L.derive_frame; ++g)
@@ -2520,12 +2687,14 @@ ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, bool pairs
       ffr[(size_t)(3 + d) * nf + f] = F.face_binormal[3 * i + d];
     }
   };
-  for (int g = 0; g < nif; ++g) {
-    const int i = dface[g];
-    put(g, I, i);
-    fl[g] = dev_of[I.face_cell_conn[2 * i]];
-    fr[g] = dev_of[I.face_cell_conn[2 * i + 1]];
-  }
+  for_runs(threads, nif, 8192, [&](int g0, int g1) {
+    for (int g = g0; g < g1; ++g) {
+      const int i = dface[g];
+      put(g, I, i);
+      fl[g] = dev_of[I.face_cell_conn[2 * i]];
+      fr[g] = dev_of[I.face_cell_conn[2 * i + 1]];
+    }
+  });
   {
     int f = nif;
     for (int g = 0; g < md->num_boundary_groups; ++g) {
@@ -2611,27 +2780,27 @@ ma_status plan_layout(const ma_mesh_data* md, const TileShape& shape, bool pairs
     return ma::fail(MA_ERR_UNSUPPORTED, "too many faces per cell tile for the flux kernel's LDS");
   std::vector<int>& tslot = L.tslot;
   tslot.assign((size_t)kMaxSlots * nc, -1);
-  for (int c = 0; c < nc; ++c)
-    for (int q = 0; q < kMaxSlots; ++q) {
-      const int e = slot[(size_t)q * nc + c];
-      if (e < 0) break;
-      const int g = e >> 1, side = e & 1;
-      tslot[(size_t)q * nc + c] =
-          g < nif ? (((side ? locr[g] : locl[g]) << 3) | side) : (((g - nif) << 3) | (3 + fkind[g]));
-    }
-
   L.vol.assign(nc, 0.0);
   L.xc.assign((size_t)3 * nc, 0.0);
-  for (int c = 0; c < nc; ++c) {
-    const int d = dev_of[c];
-    L.vol[d] = md->cell_volumes[c];
-    for (int k = 0; k < 3; ++k) L.xc[(size_t)k * nc + d] = md->cell_coordinates[3 * c + k];
-  }
+  for_runs(threads, nc, 8192, [&](int c0, int c1) {
+    for (int c = c0; c < c1; ++c)
+      for (int q = 0; q < kMaxSlots; ++q) {
+        const int e = slot[(size_t)q * nc + c];
+        if (e < 0) break;
+        const int g = e >> 1, side = e & 1;
+        tslot[(size_t)q * nc + c] =
+            g < nif ? (((side ? locr[g] : locl[g]) << 3) | side) : (((g - nif) << 3) | (3 + fkind[g]));
+      }
+    for (int d = c0; d < c1; ++d) {
+      const int c = org_of[d];
+      L.vol[d] = md->cell_volumes[c];
+      for (int k = 0; k < 3; ++k) L.xc[(size_t)k * nc + d] = md->cell_coordinates[3 * c + k];
+    }
+  });
   L.ntiles = ntiles;
   L.max_faces = max_faces;
-  dedupe_geometry(L);
+  dedupe_geometry(L, threads);
   for (int f = nif; f < nf; ++f) L.wall = L.wall || fkind[f] == MA_BC_NOSLIP;
-  if (pairs) find_pairs(L);
   return MA_OK;
 }
 
@@ -2717,10 +2886,11 @@ struct RunPlan {
   std::vector<int> tile_case, case_tiles, bc_case, cell_case, case_cell_off;
 };
 
-// pairs: meshes that qualify get the paired kernels' tables (find_pairs).  The
-// served form plans without: there, where cases come and go in launches of
-// many, the paired kernels are not used.
-ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, bool pairs, RunPlan& P) {
+// Which runs' meshes get the paired kernels' tables where they qualify
+// (find_pairs).  The served form plans without: there, where cases come and go
+// in launches of many, the paired kernels are not used.
+enum class Pairs { none, fp64, fp32 };
+ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, Pairs pairs, RunPlan& P) {
   if (!valid_shape(shape)) return ma::fail(MA_ERR_INVALID, "tile shape: extents >= 1 with product <= 256, or all 0");
   P.case_cell_off.assign(ncases + 1, 0);
   long long total_cells = 0, total_faces = 0;
@@ -2736,8 +2906,13 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
   }
   ma_status st = MA_OK;
   Layout& L = P.L;
+  auto usable = [&](const Layout& x) { return x.pair.ok && (pairs == Pairs::fp64 || x.pair.fp32); };
+  const int threads = ncases == 1 ? plan_threads(mds[0]->num_owned_cells) : 16;
   if (ncases == 1) {
-    if ((st = plan_layout(mds[0], shape, pairs, L))) return st;
+    if ((st = plan_layout(mds[0], shape, threads, L))) return st;
+    if (pairs != Pairs::none) find_pairs(L, threads);
+    if (usable(L)) list_pairs(L, threads);
+    else L.pair = PairPlan();
     P.all_lattice = L.dims[0] > 0;
     P.tile_case.assign(L.ntiles, 0);
     P.case_tiles = {0, L.ntiles};
@@ -2748,30 +2923,30 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
     std::vector<Layout> parts(ncases);
     std::vector<ma_status> status(ncases, MA_OK);
     std::vector<std::string> message(ncases);
-    std::atomic<int> next{0};
-    auto worker = [&] {
-      for (int k = next++; k < ncases; k = next++) {
-        try {
-          status[k] = plan_layout(mds[k], shape, pairs, parts[k]);
-          if (status[k]) message[k] = ma::last_error();
-        } catch (const std::bad_alloc&) {
-          status[k] = MA_ERR_NOMEM;
-          message[k] = "plan: out of host memory";
-        }
+    const int nthreads = std::min(16, (int)std::thread::hardware_concurrency());
+    for_runs(nthreads, ncases, 1, [&](int k, int) {
+      try {
+        status[k] = plan_layout(mds[k], shape, 1, parts[k]);
+        if (status[k]) message[k] = ma::last_error();
+        else if (pairs != Pairs::none) find_pairs(parts[k], 1);
+      } catch (const std::bad_alloc&) {
+        status[k] = MA_ERR_NOMEM;
+        message[k] = "plan: out of host memory";
       }
-    };
-    const int nthreads = std::max(1, std::min({ncases, 16, (int)std::thread::hardware_concurrency()}));
-    std::vector<std::thread> pool;
-    for (int i = 1; i < nthreads; ++i) pool.emplace_back(worker);
-    worker();
-    for (auto& th : pool) th.join();
+    });
     for (int k = 0; k < ncases; ++k) {
       if (status[k]) return ma::fail(status[k], "case " + std::to_string(k) + ": " + message[k]);
       P.all_lattice = P.all_lattice && parts[k].dims[0] > 0;
     }
-    merge_layouts(parts, L, P.tile_case, P.case_tiles, P.bc_case, P.cell_case);
+    // the paired kernels take the batch if they take every case, in one form
+    bool all = true;
+    for (const Layout& x : parts) all = all && usable(x) && x.pair.skew == parts[0].pair.skew;
+    if (all) for_runs(nthreads, ncases, 1, [&](int k, int) { list_pairs(parts[k], 1); });
+    else
+      for (Layout& x : parts) x.pair = PairPlan();
+    merge_layouts(parts, L, P.tile_case, P.case_tiles, P.bc_case, P.cell_case, nthreads);
   }
-  return validate_layout(L);
+  return validate_layout(L, threads);
 }
 
 void plan_stats(const Layout& L, long long* stats) {
@@ -2905,7 +3080,8 @@ ma_status upload_general(ma_solver* s, const Layout& L) {
 }
 
 // Geometry tables of the paired kernels in the arithmetic type (DevMesh::stab,
-// ptab), the values general records hold.
+// ptab), the values general records hold.  (Paired runs are never only counted:
+// the served form, which is, plans without pairs.)
 template <class T>
 ma_status upload_pair_geo(ma_solver* s, const Layout& L) {
   const PairPlan& P = L.pair;
@@ -2915,26 +3091,29 @@ ma_status upload_pair_geo(ma_solver* s, const Layout& L) {
   constexpr int W = 16 / (int)sizeof(T);  // values of a vector
   const int A = P.skew ? 3 : 1;           // area values
   const int SV = (A + 3 + W - 1) / W * W, FV = (A + 6 + W - 1) / W * W;
-  if (s->counting) {
-    if ((st = s->alloc(&ds, SV * ns)) || (st = s->alloc(&dp, FV * nf))) return st;
-  } else {
-    auto at = [](std::vector<T>& h, size_t n, int k, size_t i) -> T& { return h[((size_t)(k / W) * n + i) * W + k % W]; };
-    auto area = [&](int r, int d) {  // component d, or the one that is not zero, exactly
-      const double* q = &L.geo[(size_t)r * kGeoVals];
-      return P.skew ? q[d] : q[0] + q[1] + q[2];
-    };
-    std::vector<T> hs(SV * ns, T(0)), hp(FV * nf, T(0));
-    for (size_t i = 0; i < ns; ++i) {
+  const int threads = plan_threads(L.nc);
+  auto at = [](RawVector<T>& h, size_t n, int k, size_t i) -> T& { return h[((size_t)(k / W) * n + i) * W + k % W]; };
+  auto area = [&](int r, int d) {  // component d, or the one that is not zero, exactly
+    const double* q = &L.geo[(size_t)r * kGeoVals];
+    return P.skew ? q[d] : q[0] + q[1] + q[2];
+  };
+  RawVector<T> hs(SV * ns), hp(FV * nf);
+  for_runs(threads, (int)ns, 8192, [&](int i0, int i1) {
+    for (size_t i = i0; i < (size_t)i1; ++i) {
       const int r = P.srec[i] >> 1, side = P.srec[i] & 1;
       for (int d = 0; d < A; ++d) at(hs, ns, d, i) = T(side ? -area(r, d) : area(r, d));
       for (int d = 0; d < 3; ++d) at(hs, ns, A + d, i) = T(L.geo[(size_t)r * kGeoVals + 3 + 3 * side + d]);
+      for (int k = A + 3; k < SV; ++k) at(hs, ns, k, i) = T(0);
     }
-    for (size_t i = 0; i < nf; ++i) {
+  });
+  for_runs(threads, (int)nf, 8192, [&](int i0, int i1) {
+    for (size_t i = i0; i < (size_t)i1; ++i) {
       for (int d = 0; d < A; ++d) at(hp, nf, d, i) = T(area(P.frec[i], d));
       for (int d = 0; d < 6; ++d) at(hp, nf, A + d, i) = T(L.geo[(size_t)P.frec[i] * kGeoVals + 3 + d]);
+      for (int k = A + 6; k < FV; ++k) at(hp, nf, k, i) = T(0);
     }
-    if ((st = upload(s, &ds, hs)) || (st = upload(s, &dp, hp))) return st;
-  }
+  });
+  if ((st = upload(s, &ds, hs)) || (st = upload(s, &dp, hp))) return st;
   s->m.stab = ds;
   s->m.ptab = dp;
   s->m.nsrec = (int)ns;
@@ -2953,17 +3132,14 @@ ma_status upload_paired(ma_solver* s, const Layout& L) {
   if ((st = upload(s, &dptr, P.ptr)) || (st = upload(s, &dlr, P.lr)) || (st = upload(s, &dgid, P.gid)) ||
       (st = upload(s, &dslot, P.slot)) || (st = s->fp32 ? upload_pair_geo<float>(s, L) : upload_pair_geo<double>(s, L)))
     return st;
-  if (s->counting) {
-    st = s->alloc(&dids, (size_t)12 * ns);
-  } else {  // see slot_ids
-    std::vector<int> h((size_t)12 * ns, 0);
+  RawVector<int> h((size_t)12 * ns);  // see slot_ids
+  for_runs(plan_threads(nc), ns, 8192, [&](int c0, int c1) {
     for (int k = 0; k < 12; ++k) {
       const int* from = k < 6 ? &P.nbr[(size_t)k * nc] : &P.ent[(size_t)(k - 6) * nc];
-      for (int c = 0; c < nc; ++c) h[((size_t)(k / 4) * ns + c) * 4 + k % 4] = from[c];
+      for (int c = c0; c < c1; ++c) h[((size_t)(k / 4) * ns + c) * 4 + k % 4] = c < nc ? from[c] : 0;
     }
-    st = upload(s, &dids, h);
-  }
-  if (st) return st;
+  });
+  if ((st = upload(s, &dids, h))) return st;
   s->nbr = dids;
   s->t.ptr = dptr;
   s->t.lr = reinterpret_cast<const int2*>(dlr);
@@ -3007,7 +3183,7 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   s->org = dorg;
   m.fwall = dfw;
   s->wall = L.wall;
-  s->pair = L.pair.ok && (!s->fp32 || L.pair.fp32);
+  s->pair = L.pair.ok;
   s->skew = L.pair.skew;
   s->own = L.pair.own;
   int *dtcptr, *dtcase;
@@ -3105,7 +3281,7 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
 
 ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds) {
   RunPlan P;
-  ma_status st = plan_run(ncases, mds, s->shape, true, P);
+  ma_status st = plan_run(ncases, mds, s->shape, s->fp32 ? Pairs::fp32 : Pairs::fp64, P);
   if (st) return st;
   return build_planned(s, P);
 }
@@ -3495,7 +3671,7 @@ extern "C" ma_status ma_batch_plan(int ncases, const ma_mesh_data* const* meshes
   RunPlan P;
   ma_status st = MA_OK;
   try {
-    st = plan_run(ncases, meshes, kDefaultShape, true, P);
+    st = plan_run(ncases, meshes, kDefaultShape, Pairs::fp64, P);
   } catch (const std::bad_alloc&) {
     st = ma::fail(MA_ERR_NOMEM, "plan: out of host memory");
   }
@@ -4105,7 +4281,7 @@ ma_status plan_layout_shared(const ma_mesh_data* md, const ma_options* opt, std:
   try {
     std::shared_ptr<LayoutPlan> lp = std::make_shared<LayoutPlan>();
     lp->shape = shape;
-    if ((st = plan_run(1, &md, shape, false, lp->P))) return st;
+    if ((st = plan_run(1, &md, shape, Pairs::none, lp->P))) return st;
     const Layout& L = lp->P.L;
     lp->host_bytes = vbytes(L.dev_of) + vbytes(L.org_of) + vbytes(L.tile_cptr) + vbytes(L.tptr) +
                      vbytes(L.tfaces) + vbytes(L.slot) + vbytes(L.tslot) + vbytes(L.fl) + vbytes(L.fr) +

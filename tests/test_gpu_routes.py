@@ -74,3 +74,27 @@ def test_rotated_boxes(scheme, precision, tile):
     """Meshes with no face along an axis: up to three chunks of a block's faces."""
     box, o = _case((21, 13, 10), scheme, precision=precision, tile_shape=tile)
     _solo_equals_batched((rotated_mesh(o), o), _case((6, 5, 4), scheme, precision=precision, tile_shape=tile))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("scheme", [(0, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 0)])
+def test_batch_of_skew_meshes(scheme, precision):
+    """Meshes of different sizes merged in the skew form, their tables' side and
+    slot bits above cell and record numbers that follow another mesh's: the bits
+    of each one alone."""
+    cases = []
+    for shape, angles in (((21, 13, 10), (0.4, 0.3, 0.2)), ((1, 3, 17), (0.1, 0.7, 0.3)), ((9, 8, 7), (0.2, 0.2, 1.0))):
+        o = _case(shape, scheme, precision=precision)[1]
+        cases.append((rotated_mesh(o, angles), o))
+    if not precision:  # (a ramp's area vectors carry noise too small for the FP32 form)
+        cases.append(_case((17, 9, 8), scheme, **RAMP))
+    runs = [M.BatchSolver(cases)] + [M.TimeSolverExplicitRK4(*c) for c in cases]
+    try:
+        for s in runs:
+            s.initialize()
+            s.step(4)
+        for k in range(len(cases)):
+            assert np.array_equal(runs[0].case_state(k), runs[1 + k].state())
+    finally:
+        for s in runs:
+            s.close()
