@@ -1863,6 +1863,7 @@ using RawVector = std::vector<T, RawAlloc<T>>;
 
 // What the paired-mesh kernels (pair.hpp) read instead of the general slot
 // and tile tables; ok when the mesh is paired (find_pairs).
+constexpr long long kMaxEntries = 1ll << 30;  // of a run's tile lists
 struct PairPlan {
   bool ok = false;
   bool fp32 = true;                      // in the FP32 form as well
@@ -2135,7 +2136,7 @@ void merge_layouts(std::vector<Layout>& parts, Layout& M, std::vector<int>& tile
     M.pair.max_faces = std::max(M.pair.max_faces, P.max_faces);
   }
   M.geo.resize(go[n] * kGeoVals);
-  M.pair.ok = M.pair.ok && so[n] < (1u << kCellBits);  // as in list_pairs
+  M.pair.ok = M.pair.ok && so[n] < (1u << kCellBits) && eo[n] <= (size_t)kMaxEntries;  // as in list_pairs
   if (M.pair.ok) {
     for (auto* v : {&M.pair.nbr, &M.pair.ent}) v->resize((size_t)kMaxSlots * nc);
     M.pair.slot.resize((size_t)kMaxSlots * nc);
@@ -2391,7 +2392,7 @@ void find_pairs(Layout& L, int threads) {
 }
 
 // The paired kernels' tables of a mesh that find_pairs took (P.ok is cleared if
-// a list is too long).
+// a list is too long, or the lists are).
 void list_pairs(Layout& L, int threads) {
   PairPlan& P = L.pair;
   const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
@@ -2423,7 +2424,12 @@ void list_pairs(Layout& L, int threads) {
   // by left cell, a chunk per axis and block of 64 cells (blocks with few
   // faces share one), then the faces shared with other tiles (low side, high
   // side, by the tile's own cell) and the boundary faces.  Chunk r of the
-  // three axes and chunk r of the shared faces follow each other.
+  // three axes and chunk r of the shared faces follow each other.  Where one
+  // chunk holds all faces of a class, a small or flat tile's, it does: two mostly
+  // empty ones made 384 threads of the 100 faces of an 8-cell tile, and two
+  // workgroups a CU instead of four (second-order viscous 64 x 48 x 32 plate, us a
+  // step, general kernels / two chunks a class / one: 2x2x2 tiles 720 / 934 / 304,
+  // 1x4x4 ones 376 / 460 / 188; 512 x 512 x 1 plate, 32-cell tiles 671 / 587 / 261).
   // own: the chunks of a block hold the high faces of its cells, one per cell in
   // cell order, whatever is on their other side, and all blocks' chunks come
   // before the others, so that a wavefront can keep a cell's own values over
@@ -2446,6 +2452,12 @@ void list_pairs(Layout& L, int threads) {
   std::vector<int> bpos(nf - nif);  // list index of a boundary face in its tile
   P.slot.resize((size_t)kMaxSlots * nc);
   std::atomic<bool> too_long{false};
+  // Lists that are mostly padding (tiles of few cells: 192 entries for one cell)
+  // are not worth their memory where they are large, 12 bytes an entry here and
+  // on the device: beyond 2^26 of them at most 16 a cell (4 x 8 x 8 tiles have 4,
+  // 4 x 4 x 4 ones 6, 4 x 8 x 1 ones 6), and places in the lists are 32-bit.
+  const long long most_entries = std::min<long long>(kMaxEntries, std::max<long long>(1ll << 26, 16ll * nc));
+  std::atomic<long long> entries{0};
   for_runs(threads, ntiles, kTileRun, [&](int b0, int b1) {
     Run& R = runs[b0 / kTileRun];
     // by class: faces inside the tile (own: every high face of its cells), the
@@ -2482,6 +2494,11 @@ void list_pairs(Layout& L, int threads) {
                      std::back_inserter(merged[d]));
         std::sort(low[d].begin(), low[d].end());
         for (auto* v : {&high[d], &outer[d]}) low[d].insert(low[d].end(), v->begin(), v->end());
+        if (!P.own && inside[d].size() + low[d].size() <= 64 && !low[d].empty()) {
+          chunks[d].push_back({&low[d], d, 0, (int)(inside[d].size() + low[d].size())});
+          low[d].insert(low[d].begin(), inside[d].begin(), inside[d].end());
+          continue;
+        }
         const std::vector<Item>&K = inside_b[d].empty() ? inside[d] : merged[d], &S = low[d];
         const int nk = (int)K.size(), nsh = (int)S.size();
         for (int i = 0; i < nk;) {
@@ -2528,6 +2545,7 @@ void list_pairs(Layout& L, int threads) {
         for (const Chunk& k : chunks[kClasses]) put(k);
       R.len.push_back(n);
       if ((size_t)n * 5 * sizeof(double) > 65536) too_long = true;  // e.g. long thin tiles of consecutive cells
+      if ((entries += n) > most_entries) too_long = true;
       // summation order: internal faces in slot order, then the boundary faces
       // by kind (in slot order within a kind), the order of TimeSolverExplicitRK4.h:428-475
       for (int c = c0; c < c1; ++c) {

@@ -98,3 +98,31 @@ def test_batch_of_skew_meshes(scheme, precision):
     finally:
         for s in runs:
             s.close()
+
+
+@pytest.mark.parametrize("scheme", [(0, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 0)])
+@pytest.mark.parametrize("tile", [(1, 1, 1), (2, 2, 2), (1, 4, 4), (4, 8, 1), (1, 1, 21), (1, 1, 22)])
+def test_tiles_of_few_cells(scheme, tile):
+    """Tiles whose faces of a class fill one chunk of 64, and (1 x 1 x 22: 67
+    faces across) tiles where one class does not."""
+    box = _case((13, 11, 23), scheme, tile_shape=tile)
+    other = _case((6, 5, 4), scheme, tile_shape=tile, **RAMP)
+    _solo_equals_batched(box, other)
+    _solo_equals_batched((rotated_mesh(box[1]), box[1]), _case((6, 5, 4), scheme, tile_shape=tile))
+
+
+def test_lists_of_mostly_padding_are_not_made():
+    """373k tiles of one cell: 72 million list entries for the paired kernels."""
+    md, o = _case((72, 72, 72))
+    U = []
+    for tile in ((1, 1, 1), (0, 0, 0)):
+        s = M.TimeSolverExplicitRK4(md, o.replace(tile_shape=tile))
+        try:
+            s.initialize()
+            s.step(2)
+            U.append(s.state())
+            if tile[0]:
+                assert s.sizes()["device_bytes"] < 1500 * 72 ** 3
+        finally:
+            s.close()
+    assert np.array_equal(*U)
