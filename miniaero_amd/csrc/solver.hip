@@ -1217,6 +1217,23 @@ __global__ __launch_bounds__(kBlock) void k_state_out(int nc, const int* __restr
   for (int k = 0; k < 5; ++k) p[k] = src[(size_t)k * nc + d];
 }
 
+// Values j0 to j0 + nj - 1 of the gradient records of the caller's cells c0 to
+// c0 + n - 1, nj a cell.  np: 0 where a cell's record is a block, else the planes
+// of vectors of paired runs (rec_at).  A host loop over the records, ten lines of
+// memory a cell from the planes, took 55 ms for 983k cells, 28 in FP32 (blocks
+// 50 and 16); permuted here 14 and 9.
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_records_out(int nc, const int* __restrict__ org,
+                                                        const S* __restrict__ rec, int np, int j0, int nj, int c0,
+                                                        int n, double* __restrict__ raw) {
+  const int d = blockIdx.x * blockDim.x + threadIdx.x;
+  if (d >= nc) return;
+  const int c = org[d] - c0;
+  if (c < 0 || c >= n) return;
+  double* p = raw + (size_t)c * nj;
+  for (int j = 0; j < nj; ++j) p[j] = double(rec[np ? rec_at<S>(j0 + j, np, (unsigned)d) : (size_t)d * kRec + j0 + j]);
+}
+
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_prim(DevMesh m, const double* __restrict__ Un,
                                                  const double* __restrict__ R, double alpha,
@@ -3279,7 +3296,8 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   const size_t n5 = (size_t)5 * nc;
   const size_t tsize = s->fp32 ? sizeof(float) : sizeof(double);
   const size_t np = s->pair ? (size_t)s->m.ns : (size_t)nc;  // plane length of V, grad and fv
-  if ((st = s->alloc(&s->U[0], n5)) || (st = s->alloc(&s->U[1], n5)) || (st = s->alloc(&s->R, n5)) ||
+  const size_t nu = std::max<size_t>(n5, 15);  // (download_records)
+  if ((st = s->alloc(&s->U[0], nu)) || (st = s->alloc(&s->U[1], nu)) || (st = s->alloc(&s->R, n5)) ||
       (st = s->alloc_bytes(&s->V, 5 * np * tsize)) || (st = s->alloc_bytes(&s->V2, 5 * np * tsize)) ||
       (st = s->alloc_bytes(&s->grad, (size_t)kRec * np * tsize)) ||
       (s->opt.second_order_space && !s->opt.viscous &&
@@ -3660,23 +3678,26 @@ ma_status download_state(ma_solver* s, const double* src, double* host) {
 
 // Gradient records (kRec values per device cell) to the caller's order:
 // grad (n x 5 x 3) and lim (n x 5), either may be null.
+// Gradients and limiters to the caller's order, through the same buffer: all
+// limiters, or the gradients of a third of the cells at a time.
 template <class S>
-ma_status download_records(ma_solver* s, const S* dsrc, double* grad, double* lim) {
-  const int nc = s->m.nc;
-  const size_t np = s->pair ? (size_t)s->m.ns : (size_t)nc;
-  constexpr int W = 16 / (int)sizeof(S);
-  std::vector<S> tmp((size_t)kRec * np);
-  MA_HIP(hipMemcpyAsync(tmp.data(), dsrc, tmp.size() * sizeof(S), hipMemcpyDeviceToHost, s->stream));
+ma_status download_records(ma_solver* s, const S* rec, double* grad, double* lim) {
+  const int nc = s->m.nc, np = s->pair ? s->m.ns : 0;
+  double* raw = s->U[1 - s->cur];
+  auto part = [&](int j0, int nj, int c0, int n, double* host) -> ma_status {
+    hipLaunchKernelGGL(k_records_out<S>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, s->org, rec, np, j0, nj,
+                       c0, n, raw);
+    MA_HIP(hipGetLastError());
+    MA_HIP(hipMemcpyAsync(host + (size_t)c0 * nj, raw, (size_t)n * nj * sizeof(double), hipMemcpyDeviceToHost,
+                          s->stream));
+    return MA_OK;
+  };
+  ma_status st = MA_OK;
+  if (lim && (st = part(15, 5, 0, nc, lim))) return st;
+  const int third = std::max(1, nc / 3);  // (U holds at least 15 values)
+  for (int c0 = 0; grad && c0 < nc; c0 += third)
+    if ((st = part(0, 15, c0, std::min(third, nc - c0), grad))) return st;
   MA_HIP(hipStreamSynchronize(s->stream));
-  for (int c = 0; c < nc; ++c) {
-    const size_t d = s->dev_of[c];
-    // a block per cell, or planes of vectors on paired meshes
-    auto at = [&](int j) { return s->pair ? tmp[((size_t)(j / W) * np + d) * W + j % W] : tmp[d * kRec + j]; };
-    if (grad)
-      for (int j = 0; j < 15; ++j) grad[(size_t)c * 15 + j] = at(j);
-    if (lim)
-      for (int k = 0; k < 5; ++k) lim[(size_t)c * 5 + k] = at(15 + k);
-  }
   return MA_OK;
 }
 
@@ -4022,6 +4043,7 @@ extern "C" ma_status ma_solver_get_gradients(ma_solver* s, double* grad, double*
   if (!s) return ma::fail(MA_ERR_INVALID, "null solver");
   ma_status st = fill_gradients(s);
   if (st) return st;
+  std::lock_guard<std::mutex> lock(s->transfer);
   return s->fp32 ? download_records(s, static_cast<const float*>(s->grad), grad, lim)
                  : download_records(s, static_cast<const double*>(s->grad), grad, lim);
 }

@@ -126,3 +126,34 @@ def test_lists_of_mostly_padding_are_not_made():
         finally:
             s.close()
     assert np.array_equal(*U)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 1, 1), (1, 2, 2), (7, 1, 1), (13, 11, 7)])
+def test_gradients_read_in_parts(shape, precision):
+    """Gradients come back a third of the cells at a time: meshes of one to a few
+    cells and counts that three does not divide, together and one at a time."""
+    from miniaero_amd import _lib
+    case = _case(shape, precision=precision)
+    _solo_equals_batched(case, _case((3, 2, 2), precision=precision, **RAMP))
+    s = M.TimeSolverExplicitRK4(*case)
+    try:
+        s.initialize()
+        s.step(2)
+        U, (g, lim) = s.state(), s.gradients()
+        assert np.isfinite(g).all() and np.isfinite(lim).all()
+        g1, l1 = np.empty_like(g), np.empty_like(lim)
+        _lib.check(s._L.ma_solver_get_gradients(s._h, g1.ctypes.data_as(_lib._D), None))
+        _lib.check(s._L.ma_solver_get_gradients(s._h, None, l1.ctypes.data_as(_lib._D)))
+        assert np.array_equal(g, g1) and np.array_equal(lim, l1)
+        assert np.array_equal(s.state(), U)
+        s.step(2)
+        t = M.TimeSolverExplicitRK4(*case)
+        try:
+            t.initialize()
+            t.step(4)
+            assert np.array_equal(s.state(), t.state())
+        finally:
+            t.close()
+    finally:
+        s.close()
