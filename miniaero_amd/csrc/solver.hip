@@ -1561,13 +1561,18 @@ struct TileShape {
 constexpr TileShape kDefaultShape = {{4, 8, 8}};
 // The defaults for runs with fewer cells than one default tile per CU.  Up to
 // two 64-cell tiles per CU a step's time is each tile's latency, which a
-// quarter of the faces per workgroup shortens; the FP64 viscous flux kernel
-// holds two of their 384-thread workgroups per CU, and with more of them the
-// last ones wait for a second round, so the tiles then hold 128 cells.  k_flux
-// us, 4x4x4 / 4x4x8 / 4x8x8 tiles: FP64 viscous plates of 28k cells 14.0 / 15.1
-// / 15.6, 38k 19.0 / 16.4 / 16.5, 60k 23.6 / 16.9 / 16.4; second-order shock
-// tubes 9.2 / 10.7 / 11.5, 12.3 / 11.8 / 11.9, 15.5 / 12.5 / 12.4; ramps 12.2 /
-// 13.1 / 16.0, 15.3 / 13.7 / 17.1, 18.1 / 16.2 / 17.8.
+// quarter of the faces per workgroup shortens; the paired FP64 viscous flux
+// kernel holds two of their 384-thread workgroups per CU, and with more of them
+// the last ones wait for a second round, so a paired run's tiles then hold 128
+// cells.  k_flux us, 4x4x4 / 4x4x8 / 4x8x8 tiles: FP64 viscous plates of 28k
+// cells 14.0 / 15.1 / 15.6, 38k 19.0 / 16.4 / 16.5, 60k 23.6 / 16.9 / 16.4;
+// second-order shock tubes 9.2 / 10.7 / 11.5, 12.3 / 11.8 / 11.9, 15.5 / 12.5 /
+// 12.4; ramps 12.2 / 13.1 / 16.0, 15.3 / 13.7 / 17.1, 18.1 / 16.2 / 17.8.  Runs on
+// the general kernels, whose workgroups have 256 threads, keep 64 cells: us a step
+// with 4x4x4 / 4x4x8 tiles, 41k cells: FP64 second-order viscous 118 / 123,
+// inviscid 102 / 111, FP32 86 / 94, 90 / 92, first-order viscous FP32 69 / 75; 61k
+// cells: FP32 78 / 84, 97 / 99, 95 / 104, FP64 inviscid 114 / 120, and only FP64
+// viscous ones the other way, 157 / 133 and 134 / 114.
 constexpr TileShape kSmallRunShape = {{4, 4, 4}};
 constexpr TileShape kMediumRunShape = {{4, 4, 8}};
 
@@ -2348,6 +2353,31 @@ void dedupe_geometry(Layout& L, int threads) {
 // is at most 2^18 times the largest primitive: FP64 limiter terms stay below
 // 2^(3 (100 + 18) + 6), FP32 ones, scaled by 2^24, below 2^(3 (16 + 18) + 2 + 24)
 // and so in range, and an FP32 limiter is at least 2^-56 / 2^(2 (16 + 18) + 2).
+struct FaceBounds {
+  double area = 0.0, disp = 0.0;  // largest components
+  int axis = -1;                  // the area vector's, or kSkewFace
+  bool in = true, fp32 = true;    // inside the bounds of the FP64 form, and of the FP32 form
+};
+inline bool apart(const double* d) { return d[0] * d[0] + d[1] * d[1] + d[2] * d[2] >= 0x1p-56; }
+// q: a geometry record; internal: with the right cell's displacement.
+inline FaceBounds face_bounds(const double* q, bool internal) {
+  FaceBounds b;
+  for (int d = 0; d < 3; ++d) {
+    const double a = std::fabs(q[d]);
+    if (a != 0.0) b.axis = b.axis < 0 ? d : kSkewFace;
+    if (a != 0.0 && !(a >= 0x1p-150)) b.in = false;
+    if (a != 0.0 && !(a >= 0x1p-37)) b.fp32 = false;
+    b.area = std::max(b.area, a);
+  }
+  for (int k = 3; k < 9; ++k) b.disp = std::max(b.disp, std::fabs(q[k]));
+  b.in = b.in && b.area >= 0x1p-37 && b.area <= 0x1p100 && b.disp <= 0x1p50 && apart(q + 3) &&
+         (!internal || apart(q + 6));
+  return b;
+}
+inline bool cell_in_bounds(double vol, double area, double disp) {
+  return vol >= 0x1p-100 && vol <= 0x1p24 && area * disp <= vol * 0x1p14;
+}
+
 // The runs of the loops are spread over host threads: on one, planning a mesh
 // cost up to half as much again as without the paired kernels' tables.
 void find_pairs(Layout& L, int threads) {
@@ -2361,24 +2391,18 @@ void find_pairs(Layout& L, int threads) {
   std::atomic<bool> out{false}, skew{false}, fp32{true};  // out: outside the bounds
   for_runs(threads, (int)ng, 4096, [&](int r0, int r1) {
     for (int r = r0; r < r1 && !out; ++r) {
-      const double* q = &L.geo[(size_t)r * kGeoVals];
-      for (int d = 0; d < 3; ++d) {
-        const double a = std::fabs(q[d]);
-        if (a != 0.0) P.axis_of[r] = P.axis_of[r] < 0 ? (signed char)d : (signed char)kSkewFace;
-        if (a != 0.0 && !(a >= 0x1p-150)) out = true;
-        if (a != 0.0 && !(a >= 0x1p-37)) fp32 = false;
-        amax[r] = std::max(amax[r], a);
-      }
-      if (!(amax[r] >= 0x1p-37 && amax[r] <= 0x1p100)) out = true;
-      for (int k = 3; k < 9; ++k) dmax[r] = std::max(dmax[r], std::fabs(q[k]));
-      if (!(dmax[r] <= 0x1p50) || !(q[3] * q[3] + q[4] * q[4] + q[5] * q[5] >= 0x1p-56)) out = true;
+      const FaceBounds b = face_bounds(&L.geo[(size_t)r * kGeoVals], false);
+      P.axis_of[r] = (signed char)b.axis;
+      amax[r] = b.area;
+      dmax[r] = b.disp;
+      if (!b.in) out = true;
+      if (!b.fp32) fp32 = false;
     }
   });
   if (out) return;
   for_runs(threads, nf, 16384, [&](int f0, int f1) {
     for (int f = f0; f < f1 && !out; ++f) {
-      const double* q = &L.geo[(size_t)L.fgeo[f] * kGeoVals];
-      if (f < nif && !(q[6] * q[6] + q[7] * q[7] + q[8] * q[8] >= 0x1p-56)) out = true;
+      if (f < nif && !apart(&L.geo[(size_t)L.fgeo[f] * kGeoVals + 6])) out = true;
       if (face_class(L, f) == kSkewFace) skew = true;
     }
   });
@@ -2398,7 +2422,7 @@ void find_pairs(Layout& L, int threads) {
         dm = std::max(dm, dmax[r]);
         if (!skew) sides |= 1u << cell_side(L, f, e & 1);
       }
-      if (!(L.vol[c] >= 0x1p-100 && L.vol[c] <= 0x1p24) || !(am * dm <= L.vol[c] * 0x1p14)) out = true;
+      if (!cell_in_bounds(L.vol[c], am, dm)) out = true;
       if (sides != 0x3f) skew = true;  // (two faces on one side: the cell's slots are not one per direction)
     }
   });
@@ -2925,6 +2949,51 @@ struct RunPlan {
 // (find_pairs).  The served form plans without: there, where cases come and go
 // in launches of many, the paired kernels are not used.
 enum class Pairs { none, fp64, fp32 };
+// Whether the run is likely to get the paired kernels: what find_pairs and
+// plan_run ask, of the faces of the first 64 cells and every 16th, before the
+// tile shape gives the cells an order (0.5 ms for 46k cells; asking all of them,
+// whose faces come in random order, 3).
+bool expects_pairs(int ncases, const ma_mesh_data* const* mds, Pairs pairs) {
+  int skew0 = -1;
+  for (int k = 0; k < ncases; ++k) {
+    const ma_mesh_data* md = mds[k];
+    const int nc = md->num_owned_cells;
+    bool fp32 = true;
+    int skew = 0;
+    std::vector<double> area(nc, 0.0), disp(nc, 0.0);
+    auto picked = [&](int c) { return c >= 0 && c < nc && (c < 64 || c % 16 == 0); };
+    for (int g = -1; g < md->num_boundary_groups; ++g) {
+      const ma_faces& F = g < 0 ? md->internal_faces : md->boundary_faces[g].faces;
+      if (F.nfaces > 0 && (!F.coordinates || !F.face_normal || !F.face_cell_conn)) return false;
+      for (int i = 0; i < F.nfaces; ++i) {
+        const int c[2] = {F.face_cell_conn[2 * i], g < 0 ? F.face_cell_conn[2 * i + 1] : -1};
+        if (!picked(c[0]) && !picked(c[1])) continue;
+        double q[kGeoVals] = {};
+        for (int d = 0; d < 3; ++d) {
+          q[d] = F.face_normal[3 * (size_t)i + d];
+          for (int s = 0; s < 2; ++s)
+            if (c[s] >= 0 && c[s] < nc)
+              q[3 + 3 * s + d] = F.coordinates[3 * (size_t)i + d] - md->cell_coordinates[3 * (size_t)c[s] + d];
+        }
+        const FaceBounds b = face_bounds(q, g < 0);
+        if (!b.in) return false;
+        fp32 = fp32 && b.fp32;
+        if (b.axis == kSkewFace || (g < 0 && q[b.axis] < 0.0)) skew = 1;
+        for (int x : c)
+          if (picked(x)) {
+            area[x] = std::max(area[x], b.area);
+            disp[x] = std::max(disp[x], b.disp);
+          }
+      }
+    }
+    for (int c = 0; c < nc; ++c)
+      if (picked(c) && !cell_in_bounds(md->cell_volumes[c], area[c], disp[c])) return false;
+    if ((pairs == Pairs::fp32 && !fp32) || (skew0 >= 0 && skew != skew0)) return false;
+    skew0 = skew;
+  }
+  return true;
+}
+
 ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, Pairs pairs, RunPlan& P) {
   if (!valid_shape(shape)) return ma::fail(MA_ERR_INVALID, "tile shape: extents >= 1 with product <= 256, or all 0");
   P.case_cell_off.assign(ncases + 1, 0);
@@ -3315,9 +3384,16 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   return MA_OK;
 }
 
-ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds) {
+// otherwise: the tile shape to plan with again when the run does not get the
+// paired kernels (null: none).
+ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds, const TileShape* otherwise) {
   RunPlan P;
   ma_status st = plan_run(ncases, mds, s->shape, s->fp32 ? Pairs::fp32 : Pairs::fp64, P);
+  if (!st && otherwise && !P.L.pair.ok) {
+    s->shape = *otherwise;
+    P = RunPlan();
+    st = plan_run(ncases, mds, s->shape, Pairs::none, P);
+  }
   if (st) return st;
   return build_planned(s, P);
 }
@@ -3852,14 +3928,25 @@ ma_status create_run(int ncases, const ma_mesh_data* const* mds, const ma_option
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0)
     return ma::fail(MA_ERR_DEVICE, "no HIP device available");
+  const TileShape* otherwise = nullptr;  // see kMediumRunShape
   if (!force && !o0.autotune && o0.tile_shape[0] == 0 && o0.tile_shape[1] == 0 && o0.tile_shape[2] == 0) {
     long long cells = 0;
     for (int k = 0; k < ncases; ++k) cells += mds[k]->num_owned_cells;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        cells < (long long)cus * kTile)
-      tune.shape = cells <= (long long)cus * 128 ? kSmallRunShape : kMediumRunShape;
+        cells < (long long)cus * kTile) {
+      tune.shape = kSmallRunShape;
+      try {
+        if (cells > (long long)cus * 128 &&
+            expects_pairs(ncases, mds, o0.precision == MA_PRECISION_FP32 ? Pairs::fp32 : Pairs::fp64)) {
+          tune.shape = kMediumRunShape;
+          otherwise = &kSmallRunShape;
+        }
+      } catch (const std::bad_alloc&) {
+        return ma::fail(MA_ERR_NOMEM, "create: out of host memory");
+      }
+    }
   }
   double tuned_ms = 0.0;
   if (!force && o0.autotune) {
@@ -3887,7 +3974,7 @@ ma_status create_run(int ncases, const ma_mesh_data* const* mds, const ma_option
     if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
       st = ma::fail(MA_ERR_DEVICE, "hipStreamCreate failed");
     else
-      st = build(s, ncases, mds);
+      st = build(s, ncases, mds, otherwise);
   } catch (const std::bad_alloc&) {
     st = ma::fail(MA_ERR_NOMEM, "create: out of host memory");
   }

@@ -40,7 +40,7 @@ class Options:
     seed: int = 0
     precision: int = 0        # 0 FP64, 1 FP32 flux/gradient/limiter arithmetic
     tile_shape: tuple = (0, 0, 0)   # flux tile brick (i, j, k); zeros = 4x8x8 (below 256 cells per
-                                    # CU 4x4x8, up to 128 4x4x4), (-1, ..) = consecutive
+                                    # CU 4x4x4, above 128 4x4x8 if paired), (-1, ..) = consecutive
     autotune: int = 0         # 1: pick the fastest tile shape / resident workgroups at creation
     workgroups_per_cu: int = 0  # flux kernel: resident workgroups per CU (0: one per tile)
 

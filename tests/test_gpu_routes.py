@@ -157,3 +157,35 @@ def test_gradients_read_in_parts(shape, precision):
             t.close()
     finally:
         s.close()
+
+
+def test_default_tiles():
+    """4x4x4 up to 128 cells per CU, 4x4x8 above for runs on the paired kernels
+    (4x4x4 for others: stretched beyond their bounds, a FP32 ramp whose area
+    vectors carry noise, a box and a ramp as one batch), 4x8x8 from 256 on; the same bits with each."""
+    cus = 256
+    kw = dict(lx=1.0, ly=0.05, lz=0.025, dt=1e-14)
+    small, medium, large = (4, 4, 4), (4, 4, 8), (4, 8, 8)
+    cases = [((cus // 2, 16, 16), {}, small), ((cus // 2 + 1, 16, 16), {}, medium), ((cus, 16, 16), {}, large),
+             ((cus // 2 + 1, 16, 16), dict(precision=1), medium),
+             ((64, 40, 16), dict(precision=1, lx=2.0, ly=2.0, lz=1.0, problem_type=2, angle=30.0), small),
+             ((65, 40, 16), dict(y_stretch=1.45), small), ((65, 40, 16), dict(y_stretch=1.05), medium)]
+    for shape, more, tile in cases:
+        md, o = _case(shape, **dict(kw, **more))
+        U = []
+        for t in ((0, 0, 0), (4, 4, 4), (4, 4, 8), (4, 8, 8)):
+            s = M.TimeSolverExplicitRK4(md, o.replace(tile_shape=t))
+            try:
+                assert s.tile_shape()[0] == (t if t[0] else tile), (shape, more)
+                s.initialize()
+                s.step(1)
+                U.append(s.state())
+            finally:
+                s.close()
+        assert all(np.array_equal(U[0], x, equal_nan=True) for x in U[1:])
+    n = cus * 128 // 2 // 256 + 1
+    both = M.BatchSolver([_case((n, 16, 16)), _case((n, 16, 16), ly=1.0, lz=1.0, **RAMP)])
+    try:
+        assert both.tile_shape()[0] == small
+    finally:
+        both.close()
