@@ -767,4 +767,33 @@ struct VanAlbadaLimiter {
   }
 };
 
+// What the paired kernels (pair.hpp) need of the policies beyond the shapes that
+// the other kernels take them in: limit() with the short divisions (kTame), the
+// viscous flux along an axis, and boundary treatments that are the ones written
+// into their face lists.  A run with a policy that has none of that stays on the
+// general kernels.
+template <class Lim, class T, class = void>
+struct takes_tame : std::false_type {};
+template <class Lim, class T>
+struct takes_tame<Lim, T, decltype(Lim::template limit<T, true>(T(), T(), T(), T()), void())> : std::true_type {};
+
+template <class Visc, class T, class = void>
+struct takes_viscous_axis : std::false_type {};
+template <class Visc, class T>
+struct takes_viscous_axis<Visc, T,
+                          decltype(std::declval<const Visc&>().template compute_flux_axis<0, T>(
+                                       std::declval<const T(*)[3]>(), std::declval<const T*>(), T(),
+                                       std::declval<T*>()),
+                                   void())> : std::true_type {};
+
+template <class BCs>
+constexpr bool are_reference_boundaries =
+    std::is_same<typename BCs::Extrapolate, ExtrapolateBC>::value &&
+    std::is_same<typename BCs::Tangent, TangentBC>::value && std::is_same<typename BCs::NoSlip, NoSlipBC>::value &&
+    std::is_same<typename BCs::Inflow, InflowBC>::value;
+
+template <class Visc, class Lim, class BCs>
+constexpr bool pair_policies =
+    takes_tame<Lim, double>::value && takes_viscous_axis<Visc, double>::value && are_reference_boundaries<BCs>;
+
 }  // namespace ma

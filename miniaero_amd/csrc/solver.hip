@@ -758,6 +758,11 @@ __device__ __forceinline__ void interior_flux(const DevMesh& m, const T* __restr
   }
 }
 
+// The policies of the runs; the viscous flux and the limiter follow the options
+// (dispatch).
+using Inviscid = ma::RoeFlux;
+using Boundaries = ma::ReferenceBoundaries;
+
 // Boundary faces, one thread each: the contribution each adds to its cell's
 // flux sum, from the boundary policy of the face's kind (BCs::Extrapolate,
 // Tangent, NoSlip, Inflow; the reference's functors Extrapolate_BC.h:69-101,
@@ -800,7 +805,7 @@ __global__ __launch_bounds__(kBlock) void k_bc(DevMesh m, const T* __restrict__ 
                                                const Inflow* __restrict__ inflows,
                                                const int* __restrict__ bc_case, T* __restrict__ bc) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m.nf - m.nif) bc_face<Inv, ma::ReferenceBoundaries>(m, V, inv, prandtl, inflows, bc_case, bc, i);
+  if (i < m.nf - m.nif) bc_face<Inv, Boundaries>(m, V, inv, prandtl, inflows, bc_case, bc, i);
 }
 
 // Workgroups past the per_xcd * kXcds cell blocks take the boundary faces,
@@ -814,7 +819,7 @@ void k_grad(DevMesh m, const int* __restrict__ nbr, const T* __restrict__ V, T* 
   const int ncb = per_xcd * kXcds;
   if ((int)blockIdx.x >= ncb) {  // a boundary-face block (uniform over the workgroup)
     const int i = ((int)blockIdx.x - ncb) * kBlock + threadIdx.x;
-    if (i < m.nf - m.nif) bc_face<Inv, ma::ReferenceBoundaries>(m, V, inv, prandtl, inflows, bc_case, bc, i);
+    if (i < m.nf - m.nif) bc_face<Inv, Boundaries>(m, V, inv, prandtl, inflows, bc_case, bc, i);
     return;
   }
   // XCD-aware: each XCD takes a contiguous run of blocks (see k_flux)
@@ -1299,7 +1304,7 @@ __device__ __forceinline__ void bc_block(const CaseView* __restrict__ cv, const 
   const CaseView& v = cv[k];
   const int i = (g - start[k]) * kBlock + threadIdx.x;
   if (i < v.m.nf - v.m.nif)
-    bc_face<Inv, ma::ReferenceBoundaries>(v.m, static_cast<const T*>(v.V[vsel]), inv, prandtl, v.inflow,
+    bc_face<Inv, Boundaries>(v.m, static_cast<const T*>(v.V[vsel]), inv, prandtl, v.inflow,
                                           v.bc_case, static_cast<T*>(v.bc), i);
 }
 
@@ -1519,7 +1524,7 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
       }
       if (!kPair && nbf > 0) {  // (paired meshes: boundary faces are in the tiles' lists)
         for (int i = blockIdx.x * kTile + threadIdx.x; i < nbf; i += G * kTile)
-          bc_face<Inv, ma::ReferenceBoundaries>(m, Vs, inv, visc.prandtl, a.inflow, a.bc_case,
+          bc_face<Inv, Boundaries>(m, Vs, inv, visc.prandtl, a.inflow, a.bc_case,
                                                 static_cast<T*>(a.bc), i);
         if (!grid_sync(a.gsync, gen, a.wait_ticks, &stop)) return;
       }
@@ -2937,6 +2942,17 @@ ma_status upload_geo(ma_solver* s, const Layout& L, void** out) {
   return st;
 }
 
+// Whether the policies that the options select are ones the paired kernels can
+// be made with.
+template <class Visc>
+bool paired_limiter(const ma_options& o) {
+  return o.limiter == MA_LIMITER_VANALBADA ? ma::pair_policies<Visc, ma::VanAlbadaLimiter, Boundaries>
+                                           : ma::pair_policies<Visc, ma::VenkatLimiter, Boundaries>;
+}
+bool paired_policies(const ma_options& o) {
+  return o.viscous ? paired_limiter<ma::NewtonianViscousFlux>(o) : paired_limiter<ma::NoViscousFlux>(o);
+}
+
 // Layout of a run over ncases meshes (concatenated when there are several),
 // checked, with the case of every tile, boundary face and device cell.
 struct RunPlan {
@@ -2949,11 +2965,16 @@ struct RunPlan {
 // (find_pairs).  The served form plans without: there, where cases come and go
 // in launches of many, the paired kernels are not used.
 enum class Pairs { none, fp64, fp32 };
+Pairs pairs_of(const ma_options& o) {
+  if (!paired_policies(o)) return Pairs::none;
+  return o.precision == MA_PRECISION_FP32 ? Pairs::fp32 : Pairs::fp64;
+}
 // Whether the run is likely to get the paired kernels: what find_pairs and
 // plan_run ask, of the faces of the first 64 cells and every 16th, before the
 // tile shape gives the cells an order (0.5 ms for 46k cells; asking all of them,
 // whose faces come in random order, 3).
 bool expects_pairs(int ncases, const ma_mesh_data* const* mds, Pairs pairs) {
+  if (pairs == Pairs::none) return false;
   int skew0 = -1;
   for (int k = 0; k < ncases; ++k) {
     const ma_mesh_data* md = mds[k];
@@ -3388,7 +3409,7 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
 // paired kernels (null: none).
 ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds, const TileShape* otherwise) {
   RunPlan P;
-  ma_status st = plan_run(ncases, mds, s->shape, s->fp32 ? Pairs::fp32 : Pairs::fp64, P);
+  ma_status st = plan_run(ncases, mds, s->shape, pairs_of(s->opt), P);
   if (!st && otherwise && !P.L.pair.ok) {
     s->shape = *otherwise;
     P = RunPlan();
@@ -3448,31 +3469,33 @@ void run_stage(ma_solver* s, int irk) {
   Visc visc{effective_prandtl(s->opt)};
   const Inv inv{};
   const int nbf = m.nf - m.nif;
-  if (s->pair) {
-    // paired mesh: gradients, then the flux tiles with the boundary faces in them
-    if (SO || Visc::isViscous) {
-      s->launch(SO ? "k_grad_limiter" : "k_grad", [&] {
-        const int per = (nb + kXcds - 1) / kXcds;
-        const auto kern = s->skew ? k_grad_pair<true, SO, FV, Lim, T> : k_grad_pair<false, SO, FV, Lim, T>;
-        hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, m, s->nbr,
-                           static_cast<const T*>(Vs), FV ? nullptr : static_cast<T*>(s->grad),
-                           static_cast<T*>(s->fv), per);
+  if constexpr (ma::pair_policies<Visc, Lim, Boundaries>) {
+    if (s->pair) {
+      // paired mesh: gradients, then the flux tiles with the boundary faces in them
+      if (SO || Visc::isViscous) {
+        s->launch(SO ? "k_grad_limiter" : "k_grad", [&] {
+          const int per = (nb + kXcds - 1) / kXcds;
+          const auto kern = s->skew ? k_grad_pair<true, SO, FV, Lim, T> : k_grad_pair<false, SO, FV, Lim, T>;
+          hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, m, s->nbr,
+                             static_cast<const T*>(Vs), FV ? nullptr : static_cast<T*>(s->grad),
+                             static_cast<T*>(s->fv), per);
+        });
+      }
+      constexpr bool kOwn = SO && Visc::isViscous;
+      double* time_dev = irk == 3 && !s->any_cfl ? s->time_dev : nullptr;  // see advance_time
+      const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Inv, Visc, T>(s)
+                        : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Inv, Visc, T>(s)
+                                         : pair_flux_kernel<false, false, SO, Inv, Visc, T>(s);
+      s->launch("k_flux", [&] {
+        hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
+                           (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
+                           static_cast<const T*>(FV ? s->fv : s->grad), s->inflow_dev, irk == 0 ? Un : Uacc, Uacc,
+                           s->R, s->dt_dev, beta[irk], inv, visc, Un, Vn, irk < 3 ? alpha[irk + 1] : alpha[0],
+                           irk == 3 ? 1 : 0, time_dev);
       });
+      if (irk == 3) s->v0_valid = true;  // V now holds the next step's stage-0 primitives
+      return;
     }
-    constexpr bool kOwn = SO && Visc::isViscous;
-    double* time_dev = irk == 3 && !s->any_cfl ? s->time_dev : nullptr;  // see advance_time
-    const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Inv, Visc, T>(s)
-                      : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Inv, Visc, T>(s)
-                                       : pair_flux_kernel<false, false, SO, Inv, Visc, T>(s);
-    s->launch("k_flux", [&] {
-      hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
-                         (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
-                         static_cast<const T*>(FV ? s->fv : s->grad), s->inflow_dev, irk == 0 ? Un : Uacc, Uacc,
-                         s->R, s->dt_dev, beta[irk], inv, visc, Un, Vn, irk < 3 ? alpha[irk + 1] : alpha[0],
-                         irk == 3 ? 1 : 0, time_dev);
-    });
-    if (irk == 3) s->v0_valid = true;  // V now holds the next step's stage-0 primitives
-    return;
   }
   if (SO || Visc::isViscous) {
     // the gradient kernel; its workgroups past the cell blocks compute the
@@ -3543,7 +3566,6 @@ void run_steps(ma_solver* s, int nsteps) {
 // one this library instantiates), viscous flux and limiter selected from the
 // options, as TimeSolverExplicitRK4 instantiates compute_face_flux and the
 // limiter (TimeSolverExplicitRK4.h:388-486, StencilLimiter.h:455).
-using Inviscid = ma::RoeFlux;
 
 template <bool SO, class Visc, class T>
 void dispatch_lim(ma_solver* s, int n) {
@@ -3578,9 +3600,10 @@ template <bool SO, class Inv, class Visc, class Lim, class T>
 ma_status run_persistent(ma_solver* s, int nsteps) {
   if (nsteps == 0) return MA_OK;
   constexpr bool FV = SO && !Visc::isViscous;
-  const auto kern = !s->pair  ? k_steps<SO, Inv, Visc, Lim, T, 0>
-                    : s->skew ? k_steps<SO, Inv, Visc, Lim, T, 2>
-                              : k_steps<SO, Inv, Visc, Lim, T, 1>;
+  auto kern = k_steps<SO, Inv, Visc, Lim, T, 0>;
+  if constexpr (ma::pair_policies<Visc, Lim, Boundaries>) {
+    if (s->pair) kern = s->skew ? k_steps<SO, Inv, Visc, Lim, T, 2> : k_steps<SO, Inv, Visc, Lim, T, 1>;
+  }
   const size_t lds = std::max((size_t)s->t.max_faces * 5 * sizeof(T),
                               FV || s->pair ? (size_t)0 : (size_t)kBlock * kStageRow<T> * sizeof(T));
   int coop = 0, per_cu = 0, wall_khz = 0;
@@ -3939,7 +3962,7 @@ ma_status create_run(int ncases, const ma_mesh_data* const* mds, const ma_option
       tune.shape = kSmallRunShape;
       try {
         if (cells > (long long)cus * 128 &&
-            expects_pairs(ncases, mds, o0.precision == MA_PRECISION_FP32 ? Pairs::fp32 : Pairs::fp64)) {
+            expects_pairs(ncases, mds, pairs_of(o0))) {
           tune.shape = kMediumRunShape;
           otherwise = &kSmallRunShape;
         }
@@ -4093,11 +4116,13 @@ template <class Lim, class T>
 void stage3_gradients(ma_solver* s) {
   const int nb = nblocks(s->m.nc);
   const int per = (nb + kXcds - 1) / kXcds;
-  if (s->pair) {
-    const auto kern = s->skew ? k_grad_pair<true, true, true, Lim, T> : k_grad_pair<false, true, true, Lim, T>;
-    hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, s->m, s->nbr,
-                       static_cast<const T*>(s->V2), static_cast<T*>(s->grad), static_cast<T*>(s->fv), per);
-    return;
+  if constexpr (ma::pair_policies<ma::NoViscousFlux, Lim, Boundaries>) {
+    if (s->pair) {
+      const auto kern = s->skew ? k_grad_pair<true, true, true, Lim, T> : k_grad_pair<false, true, true, Lim, T>;
+      hipLaunchKernelGGL(kern, dim3(per * kXcds), dim3(kBlock), 0, s->stream, s->m, s->nbr,
+                         static_cast<const T*>(s->V2), static_cast<T*>(s->grad), static_cast<T*>(s->fv), per);
+      return;
+    }
   }
   // no boundary-face blocks: the grid is the cell blocks alone
   hipLaunchKernelGGL((k_grad<true, true, Lim, T, 0, Inviscid>), dim3(per * kXcds), dim3(kBlock), 0, s->stream,
