@@ -1633,7 +1633,10 @@ struct ma_solver {
   bool persistent = false;    // ma_solver_step runs its steps as one k_steps launch
   double *norm_partial = nullptr, *norm_out = nullptr;  // per tile x 5, per case x 5
   const double* xc = nullptr;  // cell centroids (3 planes), for the initial condition
-  std::mutex transfer;         // U[1 - cur] as the staging of a state copy
+  // Held while a call queues its work: a copy of the state goes through U[1 - cur],
+  // which a step accumulates in, so it must not come between another thread's
+  // launches of a step (the monitor of a run, say).
+  std::mutex queueing;
   const int* org = nullptr;    // device cell -> caller's cell index
   const int* nbr = nullptr;    // kMaxSlots planes of nc: the cell across each slot (grad_cell)
   int cur = 0;  // U[cur] holds sol_n
@@ -3762,11 +3765,12 @@ ma_status advance(ma_solver* s, int nsteps) {
   return MA_OK;
 }
 
-// Five planes to the caller's order, through the state buffer that is free
-// between steps (the lock keeps calls from several threads off each other's).
-ma_status download_state(ma_solver* s, const double* src, double* host) {
+// The state or the residual to the caller's order, through the state buffer that
+// is free between steps.
+ma_status download_state(ma_solver* s, bool residual, double* host) {
   const int nc = s->m.nc;
-  std::lock_guard<std::mutex> lock(s->transfer);
+  std::lock_guard<std::mutex> lock(s->queueing);
+  const double* src = residual ? s->R : s->U[s->cur];
   double* raw = s->U[1 - s->cur];
   hipLaunchKernelGGL(k_state_out, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, s->org, src, raw);
   MA_HIP(hipGetLastError());
@@ -3775,10 +3779,9 @@ ma_status download_state(ma_solver* s, const double* src, double* host) {
   return MA_OK;
 }
 
-// Gradient records (kRec values per device cell) to the caller's order:
-// grad (n x 5 x 3) and lim (n x 5), either may be null.
-// Gradients and limiters to the caller's order, through the same buffer: all
-// limiters, or the gradients of a third of the cells at a time.
+// Gradient records to the caller's order, grad (n x 5 x 3) and lim (n x 5),
+// either may be null, through the same buffer: all limiters, or the gradients of
+// a third of the cells at a time.
 template <class S>
 ma_status download_records(ma_solver* s, const S* rec, double* grad, double* lim) {
   const int nc = s->m.nc, np = s->pair ? s->m.ns : 0;
@@ -4026,6 +4029,7 @@ extern "C" ma_status ma_batch_create(int ncases, const ma_mesh_data* const* mesh
 
 extern "C" ma_status ma_solver_initialize(ma_solver* s) {
   if (!s) return ma::fail(MA_ERR_INVALID, "null solver");
+  std::lock_guard<std::mutex> lock(s->queueing);
   s->cur = 0;
   hipLaunchKernelGGL(k_init, dim3(nblocks(s->m.nc)), dim3(kBlock), 0, s->stream, s->m, s->xc, s->org, s->ic_dev,
                      s->cell_case, s->U[0]);
@@ -4042,7 +4046,7 @@ extern "C" ma_status ma_solver_initialize(ma_solver* s) {
 extern "C" ma_status ma_solver_set_state(ma_solver* s, const double* U) {
   if (!s || !U) return ma::fail(MA_ERR_INVALID, "null argument");
   const int nc = s->m.nc;
-  std::lock_guard<std::mutex> lock(s->transfer);
+  std::lock_guard<std::mutex> lock(s->queueing);
   s->cur = 0;
   double* raw = s->U[1];
   MA_HIP(hipMemcpyAsync(raw, U, (size_t)5 * nc * sizeof(double), hipMemcpyHostToDevice, s->stream));
@@ -4056,6 +4060,7 @@ extern "C" ma_status ma_solver_set_state(ma_solver* s, const double* U) {
 extern "C" ma_status ma_solver_step(ma_solver* s, int nsteps) {
   if (!s) return ma::fail(MA_ERR_INVALID, "null solver");
   if (nsteps < 0) return ma::fail(MA_ERR_INVALID, "negative step count");
+  std::lock_guard<std::mutex> lock(s->queueing);
   ma_status st = advance(s, nsteps);
   if (st) return st;
   MA_HIP(hipGetLastError());
@@ -4102,12 +4107,12 @@ extern "C" ma_status ma_solver_synchronize(ma_solver* s) {
 
 extern "C" ma_status ma_solver_get_state(ma_solver* s, double* U) {
   if (!s || !U) return ma::fail(MA_ERR_INVALID, "null argument");
-  return download_state(s, s->U[s->cur], U);
+  return download_state(s, false, U);
 }
 
 extern "C" ma_status ma_solver_get_residual(ma_solver* s, double* R) {
   if (!s || !R) return ma::fail(MA_ERR_INVALID, "null argument");
-  return download_state(s, s->R, R);
+  return download_state(s, true, R);
 }
 
 namespace {
@@ -4153,9 +4158,9 @@ ma_status fill_gradients(ma_solver* s) {
 
 extern "C" ma_status ma_solver_get_gradients(ma_solver* s, double* grad, double* lim) {
   if (!s) return ma::fail(MA_ERR_INVALID, "null solver");
+  std::lock_guard<std::mutex> lock(s->queueing);
   ma_status st = fill_gradients(s);
   if (st) return st;
-  std::lock_guard<std::mutex> lock(s->transfer);
   return s->fp32 ? download_records(s, static_cast<const float*>(s->grad), grad, lim)
                  : download_records(s, static_cast<const double*>(s->grad), grad, lim);
 }
@@ -4317,6 +4322,7 @@ extern "C" int ma_solver_profile(ma_solver* s, int nsteps, const char** names, i
     ma::fail(MA_ERR_INVALID, "ma_solver_profile: bad argument");
     return -1;
   }
+  std::lock_guard<std::mutex> lock(s->queueing);
   (void)hipStreamSynchronize(s->stream);
   s->timing.on = true;
   s->timing.recs.clear();

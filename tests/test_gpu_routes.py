@@ -189,3 +189,38 @@ def test_default_tiles():
         assert both.tile_shape()[0] == small
     finally:
         both.close()
+
+
+@pytest.mark.parametrize("graph", [0, 2])
+def test_state_read_while_another_thread_steps(graph):
+    """A monitor thread's reads go through the buffer that a step accumulates in:
+    they come between steps, and the run ends with an undisturbed run's bits."""
+    import threading
+    case = _case((24, 20, 16))
+    states = []
+    for watch in (False, True):
+        s = M.TimeSolverExplicitRK4(*case)
+        try:
+            s.set_graph(graph)
+            s.initialize()
+            done = threading.Event()
+            seen = []
+
+            def read():
+                while not done.is_set():
+                    seen.append(np.isfinite(s.state()).all() and np.isfinite(s.residual()).all())
+
+            t = threading.Thread(target=read)
+            if watch:
+                t.start()
+            for _ in range(60):
+                s.step(3 if not graph else 4)
+            done.set()
+            if watch:
+                t.join()
+                assert seen and all(seen)
+            states.append(s.state())
+        finally:
+            done.set()
+            s.close()
+    assert np.array_equal(*states)
