@@ -302,6 +302,12 @@ double ma_server_now(ma_server* srv);
 /* Requests whose layout came from the plan cache (*hits) and those that
  * generated and planned their mesh (*misses). */
 ma_status ma_server_plan_cache(ma_server* srv, long long* hits, long long* misses);
+/* The longest a wait on the device may take (building a case, a step, copying a
+ * result back; 120 s unless set here).  When one takes longer and nothing else
+ * ends meanwhile, every unfinished request finishes with MA_ERR_DEVICE and
+ * ma_server_submit fails with it; destroying the server then frees nothing that
+ * the device may still write to.  Looked at by submit, poll and destroy. */
+ma_status ma_server_set_wait_limit(ma_server* srv, double seconds);
 /* Cancels cases not yet admitted, waits for the active ones to finish their
  * launched steps, frees everything. */
 void ma_server_destroy(ma_server* srv);

@@ -35,7 +35,7 @@ EXPORTS = (
     "ma_batch_get_case_time", "ma_batch_plan", "ma_solver_set_graph", "ma_solver_set_persistent",
     "ma_solver_tuning", "ma_solver_residual_norms", "ma_solver_residual_norms_noalloc", "ma_server_create", "ma_server_submit", "ma_server_poll",
     "ma_server_get_state", "ma_server_release", "ma_server_stats", "ma_server_now", "ma_server_destroy",
-    "ma_server_plan_cache",
+    "ma_server_plan_cache", "ma_server_set_wait_limit",
 )
 
 
@@ -174,6 +174,7 @@ def load() -> ctypes.CDLL:
     L.ma_server_now.restype = ctypes.c_double
     L.ma_server_now.argtypes = [P]
     L.ma_server_plan_cache.argtypes = [P, ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(ctypes.c_longlong)]
+    L.ma_server_set_wait_limit.argtypes = [P, ctypes.c_double]
     L.ma_server_destroy.argtypes = [P]
     L.ma_server_destroy.restype = None
     L.ma_batch_sizes.argtypes = [P, _I, _I]

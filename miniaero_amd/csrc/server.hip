@@ -134,6 +134,7 @@ struct Group {
     std::vector<Request*> finishing;  // cases whose last step this is
   };
   std::deque<Step> inflight;
+  double since = 0.0;  // when the front one was queued or became the front
   std::vector<hipEvent_t> spare;
 };
 
@@ -247,6 +248,19 @@ struct ma_server {
   // request's way and leaves the runtime thousands of dead streams to tidy up
   std::vector<hipStream_t> streams;
   std::thread sched, finish;
+  // Waits on the device, so that one that never ends is an error and not a server
+  // that hangs (check_waits): when each setup thread and the finisher (last) began
+  // theirs, since when the scheduler's oldest step in flight is the next to end,
+  // and when it began its current round; negative: none.
+  std::vector<double> busy;
+  double step_wait = -1.0, round = -1.0;
+  double progress = 0.0;       // last time that a wait or a round ended
+  double wait_limit = 120.0;   // ma_server_set_wait_limit
+  bool lost = false;           // a wait did not end: every request has failed, no thread touches the device
+  std::string lost_why;
+  std::vector<std::unique_ptr<Request>> released;  // after that: released requests a thread may still hold
+  int live = 0;                // threads running
+  std::condition_variable cv_exit;
 
   double now() const { return std::chrono::duration<double>(Clock::now() - t0).count(); }
 };
@@ -256,6 +270,7 @@ namespace {
 // Under the lock: the request is done (successfully or not).  A case that
 // held a slot finished when it gave the slot back.
 void mark_finished(ma_server* S, Request* r) {
+  if (r->finished) return;  // (failed by check_waits)
   r->finished = true;
   if (r->t_finish == 0.0) r->t_finish = S->now();
   S->done_unpolled.push_back(r);
@@ -265,16 +280,84 @@ void mark_finished(ma_server* S, Request* r) {
 
 void fail_request(ma_server* S, Request* r, ma_status st, const std::string& err) {
   std::lock_guard<std::mutex> lk(S->mu);
+  if (r->finished) return;
   r->status = st;
   r->error = err;
   mark_finished(S, r);
 }
 
+// Under the lock: fails everything when a wait on the device is older than the
+// limit and nothing else has ended meanwhile either (ten times the limit whatever
+// has).  The threads that can still leave do, without touching the device.
+void check_waits(ma_server* S) {
+  if (S->lost) return;
+  const double t = S->now();
+  double oldest = 0.0;
+  const char* what = nullptr;
+  auto look = [&](double since, const char* name) {
+    if (since >= 0.0 && t - since > oldest) {
+      oldest = t - since;
+      what = name;
+    }
+  };
+  for (size_t i = 0; i < S->busy.size(); ++i)
+    look(S->busy[i], i + 1 < S->busy.size() ? "building a case" : "copying a result back");
+  look(S->step_wait, "a step");
+  look(S->round, "queueing steps");
+  if (!(oldest > S->wait_limit) || !(t - S->progress > S->wait_limit || oldest > 10.0 * S->wait_limit)) return;
+  S->lost = true;
+  S->lost_why = std::string("server: ") + what + " has not ended for " + std::to_string((int)oldest) +
+                " s; its device work is given up";
+  S->queue.clear();
+  S->incoming.clear();
+  S->completing.clear();
+  for (auto& e : S->all) {
+    Request* r = e.second.get();
+    if (r->finished) continue;
+    r->status = MA_ERR_DEVICE;
+    r->error = S->lost_why;
+    mark_finished(S, r);
+  }
+  S->waiting = 0;
+  S->active = 0;
+  for (auto* cv : {&S->cv_work, &S->cv_admit, &S->cv_sched, &S->cv_complete, &S->cv_exit}) cv->notify_all();
+}
+
+// A wait of thread i on the device, from construction to destruction.
+struct Wait {
+  ma_server* S;
+  size_t i;
+  Wait(ma_server* server, size_t thread) : S(server), i(thread) {
+    std::lock_guard<std::mutex> lk(S->mu);
+    S->busy[i] = S->now();
+  }
+  ~Wait() {
+    std::lock_guard<std::mutex> lk(S->mu);
+    S->busy[i] = -1.0;
+    S->progress = S->now();
+  }
+};
+
+// Counts a thread out as it ends.
+struct Leaving {
+  ma_server* S;
+  ~Leaving() {
+    std::lock_guard<std::mutex> lk(S->mu);
+    --S->live;
+    S->cv_exit.notify_all();  // (under the lock: the server may be deleted once it is gone)
+  }
+};
+
 // Frees a built case's device resources and returns its region block.
 void retire(ma_server* S, Request* r) {
+  {
+    std::lock_guard<std::mutex> lk(S->mu);
+    if (S->lost) return;  // (its waits might not end either)
+  }
   if (r->solver) ma_solver_destroy(r->solver);
   r->solver = nullptr;
   std::lock_guard<std::mutex> lk(S->mu);
+  if (S->lost) return;
   if (r->has_region) {
     S->region.release(r->offset, r->bytes);
     r->has_region = false;
@@ -284,14 +367,16 @@ void retire(ma_server* S, Request* r) {
   }
 }
 
-void setup_worker(ma_server* S, hipStream_t stream) {
+void setup_worker(ma_server* S, int index) {
+  Leaving leaving{S};
+  const hipStream_t stream = S->streams[index];
   (void)hipSetDevice(S->device);
   for (;;) {
     Request* r = nullptr;
     {
       std::unique_lock<std::mutex> lk(S->mu);
-      S->cv_work.wait(lk, [&] { return S->stop || !S->queue.empty(); });
-      if (S->stop) return;  // queued requests are cancelled by ma_server_destroy
+      S->cv_work.wait(lk, [&] { return S->stop || S->lost || !S->queue.empty(); });
+      if (S->stop || S->lost) return;  // queued requests are cancelled by ma_server_destroy
       r = S->queue.front();
       S->queue.pop_front();
     }
@@ -322,15 +407,19 @@ void setup_worker(ma_server* S, hipStream_t stream) {
 
     {
       std::unique_lock<std::mutex> lk(S->mu);
-      S->cv_admit.wait(lk, [&] { return S->stop || S->admit_next == r->id; });
+      S->cv_admit.wait(lk, [&] { return S->stop || S->lost || S->admit_next == r->id; });
       if (!st && !S->stop && Region::granule(bytes) > S->region.size()) {
         st = MA_ERR_NOMEM;
         err = "case needs " + std::to_string(bytes) + " device bytes, more than the server's region";
       }
       if (!st)
         S->cv_admit.wait(lk, [&] {
-          return S->stop || (S->active < S->cfg.max_active && S->region.reserve(bytes, &r->offset));
+          return S->stop || S->lost || (S->active < S->cfg.max_active && S->region.reserve(bytes, &r->offset));
         });
+      if (S->lost) {
+        ma::destroy_plan(pc);
+        return;
+      }
       if (!st && S->stop) {
         st = MA_ERR_INVALID;
         err = "server stopped before the case was admitted";
@@ -352,12 +441,15 @@ void setup_worker(ma_server* S, hipStream_t stream) {
     }
     // build inside the region, outside the lock
     ma_solver* s = nullptr;
-    st = ma::create_from_plan(pc, S->base + r->offset, r->bytes, stream, &s);
-    ma::destroy_plan(pc);
-    r->solver = s;
-    if (!st) st = ma_solver_initialize(s);
+    {
+      Wait wait(S, (size_t)index);
+      st = ma::create_from_plan(pc, S->base + r->offset, r->bytes, stream, &s);
+      ma::destroy_plan(pc);
+      r->solver = s;
+      if (!st) st = ma_solver_initialize(s);
+      if (st) err = ma::last_error();
+    }
     if (st) {
-      err = ma::last_error();
       retire(S, r);
       fail_request(S, r, st, err);
       continue;
@@ -365,32 +457,40 @@ void setup_worker(ma_server* S, hipStream_t stream) {
     r->total = r->opt.ntimesteps;
     {
       std::lock_guard<std::mutex> lk(S->mu);
+      if (S->lost) return;
       S->incoming.push_back(r);
     }
     S->cv_sched.notify_one();
   }
 }
 
-// Copies the final state to the host, frees the case's device resources.
-void complete(ma_server* S, Request* r) {
-  if (r->status == MA_OK) {
-    r->U.resize((size_t)r->cells * 5);
-    ma_status st = ma_solver_get_state(r->solver, r->U.data());
+// Copies the final state to the host, frees the case's device resources.  st:
+// how the case ended.
+void complete(ma_server* S, Request* r, ma_status st) {
+  std::vector<double> U;
+  std::string error;
+  if (st == MA_OK) {
+    U.resize((size_t)r->cells * 5);
+    Wait wait(S, S->busy.size() - 1);
+    st = ma_solver_get_state(r->solver, U.data());
     if (st) {
-      r->status = st;
-      r->error = ma::last_error();
-      r->U.clear();
+      error = ma::last_error();
+      U.clear();
     } else {
       long long bad = 0;
-      for (double x : r->U) bad += !std::isfinite(x);
+      for (double x : U) bad += !std::isfinite(x);
       if (bad) {  // the state is kept for inspection
-        r->status = MA_ERR_NONFINITE;
-        r->error = std::to_string(bad) + " non-finite values in the final state";
+        st = MA_ERR_NONFINITE;
+        error = std::to_string(bad) + " non-finite values in the final state";
       }
     }
   }
   retire(S, r);
   std::lock_guard<std::mutex> lk(S->mu);
+  if (r->finished) return;
+  r->status = st;
+  if (!error.empty()) r->error = error;
+  r->U = std::move(U);
   mark_finished(S, r);
 }
 
@@ -400,24 +500,29 @@ void complete(ma_server* S, Request* r) {
 void hand_off(ma_server* S, Request* r) {
   {
     std::lock_guard<std::mutex> lk(S->mu);
+    if (S->lost) return;
     S->completing.push_back(r);
   }
   S->cv_complete.notify_one();
 }
 
-void finisher(ma_server* S, hipStream_t stream) {
+void finisher(ma_server* S) {
+  Leaving leaving{S};
+  const hipStream_t stream = S->streams.back();
   (void)hipSetDevice(S->device);
   for (;;) {
     Request* r = nullptr;
+    ma_status st = MA_OK;
     {
       std::unique_lock<std::mutex> lk(S->mu);
-      S->cv_complete.wait(lk, [&] { return S->sched_done || !S->completing.empty(); });
-      if (S->completing.empty()) return;  // the scheduler is gone and nothing is left
+      S->cv_complete.wait(lk, [&] { return S->sched_done || S->lost || !S->completing.empty(); });
+      if (S->completing.empty()) return;  // the scheduler is gone and nothing is left, or the device is
       r = S->completing.front();
       S->completing.pop_front();
+      st = r->status;
     }
     if (r->solver) ma::solver_set_stream(r->solver, stream);  // (its build ended with a wait)
-    complete(S, r);
+    complete(S, r, st);
   }
 }
 
@@ -432,8 +537,12 @@ void fail_group(ma_server* S, Group& g, const std::string& why) {
   g.act.clear();
   g.dirty = true;
   for (Request* r : all) {
-    r->status = MA_ERR_DEVICE;
-    r->error = why;
+    {
+      std::lock_guard<std::mutex> lk(S->mu);
+      if (S->lost) return;
+      r->status = MA_ERR_DEVICE;
+      r->error = why;
+    }
     hand_off(S, r);
   }
 }
@@ -442,6 +551,7 @@ void fail_group(ma_server* S, Group& g, const std::string& why) {
 // cases at a time (at most steps_in_flight ahead), cases join a group at its
 // next step and leave after their last one.
 void scheduler(ma_server* S) {
+  Leaving leaving{S};
   (void)hipSetDevice(S->device);
   std::vector<std::unique_ptr<Group>> groups;
   auto idle = [&] {
@@ -449,12 +559,19 @@ void scheduler(ma_server* S) {
       if (!g->act.empty() || !g->inflight.empty()) return false;
     return true;
   };
+  bool progress = false;
   for (;;) {
     std::vector<Request*> joining;
     bool stopping = false;
     {
       std::unique_lock<std::mutex> lk(S->mu);
-      if (idle()) S->cv_sched.wait(lk, [&] { return S->stop || !S->incoming.empty(); });
+      S->step_wait = S->round = -1.0;
+      if (idle()) S->cv_sched.wait(lk, [&] { return S->stop || S->lost || !S->incoming.empty(); });
+      if (S->lost) return;
+      S->round = S->now();
+      if (progress) S->progress = S->round;
+      for (auto& g : groups)
+        if (!g->inflight.empty() && (S->step_wait < 0.0 || g->since < S->step_wait)) S->step_wait = g->since;
       joining.assign(S->incoming.begin(), S->incoming.end());
       S->incoming.clear();
       stopping = S->stop;
@@ -489,7 +606,7 @@ void scheduler(ma_server* S) {
       }
       return;
     }
-    bool progress = false;
+    progress = false;
     for (Request* r : joining) {
       progress = true;
       if (r->total == 0) {
@@ -532,6 +649,7 @@ void scheduler(ma_server* S) {
         }
         Group::Step st = g.inflight.front();
         g.inflight.pop_front();
+        g.since = S->now();
         g.spare.push_back(st.ev);
         for (Request* r : st.finishing) {
           ma::solver_set_progress(r->solver, r->total);
@@ -578,6 +696,7 @@ void scheduler(ma_server* S) {
           g.act.swap(keep);
           g.dirty = true;
         }
+        if (g.inflight.empty()) g.since = S->now();
         g.inflight.push_back(std::move(step));
         g.parity ^= 1;
         progress = true;
@@ -637,9 +756,23 @@ extern "C" ma_status ma_server_create(const ma_server_config* cfg, ma_server** o
         ma_server_destroy(S);
         return ma::fail(MA_ERR_DEVICE, "ma_server_create: hipStreamCreate failed");
       }
-    for (int i = 0; i < c.setup_threads; ++i) S->setup.emplace_back(setup_worker, S, S->streams[i]);
-    S->sched = std::thread(scheduler, S);
-    S->finish = std::thread(finisher, S, S->streams.back());
+    S->busy.assign((size_t)c.setup_threads + 1, -1.0);
+    auto start = [&](auto&& make) {  // counted before it runs
+      {
+        std::lock_guard<std::mutex> lk(S->mu);
+        ++S->live;
+      }
+      try {
+        make();
+      } catch (...) {
+        std::lock_guard<std::mutex> lk(S->mu);
+        --S->live;
+        throw;
+      }
+    };
+    for (int i = 0; i < c.setup_threads; ++i) start([&] { S->setup.emplace_back(setup_worker, S, i); });
+    start([&] { S->sched = std::thread(scheduler, S); });
+    start([&] { S->finish = std::thread(finisher, S); });
   } catch (const std::exception&) {
     ma_server_destroy(S);
     return ma::fail(MA_ERR_DEVICE, "ma_server_create: could not start threads");
@@ -656,6 +789,8 @@ extern "C" ma_status ma_server_submit(ma_server* S, const ma_options* opts, long
   r->opt = *opts;
   {
     std::lock_guard<std::mutex> lk(S->mu);
+    check_waits(S);
+    if (S->lost) return ma::fail(MA_ERR_DEVICE, S->lost_why);
     if (S->stop) return ma::fail(MA_ERR_INVALID, "ma_server_submit: server is stopping");
     r->id = S->next_id++;
     r->t_submit = S->now();
@@ -674,8 +809,10 @@ extern "C" int ma_server_poll(ma_server* S, ma_case_result* out, int max, double
     return -1;
   }
   std::unique_lock<std::mutex> lk(S->mu);
-  if (S->done_unpolled.empty() && timeout_s > 0.0)
-    S->cv_done.wait_for(lk, std::chrono::duration<double>(timeout_s),
+  check_waits(S);
+  const double until = S->now() + (timeout_s > 0.0 ? std::min(timeout_s, 1e9) : 0.0);
+  for (double left; S->done_unpolled.empty() && !S->stop && (left = until - S->now()) > 0.0; check_waits(S))
+    S->cv_done.wait_for(lk, std::chrono::duration<double>(std::min(left, std::min(0.5, 0.25 * S->wait_limit))),
                         [&] { return !S->done_unpolled.empty() || S->stop; });
   int n = 0;
   while (n < max && !S->done_unpolled.empty()) {
@@ -716,6 +853,7 @@ extern "C" ma_status ma_server_release(ma_server* S, long long id) {
   if (!it->second->finished) return ma::fail(MA_ERR_INVALID, "ma_server_release: case not finished");
   S->done_unpolled.erase(std::remove(S->done_unpolled.begin(), S->done_unpolled.end(), it->second.get()),
                          S->done_unpolled.end());
+  if (S->lost) S->released.push_back(std::move(it->second));
   S->all.erase(it);
   return MA_OK;
 }
@@ -738,6 +876,13 @@ extern "C" ma_status ma_server_plan_cache(ma_server* S, long long* hits, long lo
   return MA_OK;
 }
 
+extern "C" ma_status ma_server_set_wait_limit(ma_server* S, double seconds) {
+  if (!S || !(seconds > 0.0)) return ma::fail(MA_ERR_INVALID, "ma_server_set_wait_limit: bad argument");
+  std::lock_guard<std::mutex> lk(S->mu);
+  S->wait_limit = seconds;
+  return MA_OK;
+}
+
 extern "C" double ma_server_now(ma_server* S) { return S ? S->now() : 0.0; }
 
 extern "C" void ma_server_destroy(ma_server* S) {
@@ -750,15 +895,31 @@ extern "C" void ma_server_destroy(ma_server* S) {
   S->cv_admit.notify_all();
   S->cv_sched.notify_all();
   S->cv_done.notify_all();
-  for (auto& t : S->setup)
-    if (t.joinable()) t.join();
-  if (S->sched.joinable()) S->sched.join();
-  {  // the finisher completes what the scheduler handed it, then stops
-    std::lock_guard<std::mutex> lk(S->mu);
-    S->sched_done = true;
+  // the finisher completes what the scheduler handed it, then stops
+  bool gone = true;
+  {
+    std::unique_lock<std::mutex> lk(S->mu);
+    // every thread ends, unless a wait on the device does not (check_waits)
+    while (S->live > 0 && !S->lost) {
+      if (S->live == 1 && S->finish.joinable() && !S->sched_done) {
+        S->sched_done = true;
+        S->cv_complete.notify_all();
+      }
+      S->cv_exit.wait_for(lk, std::chrono::duration<double>(std::min(0.5, 0.25 * S->wait_limit)));
+      check_waits(S);
+    }
+    if (S->lost) gone = S->cv_exit.wait_for(lk, std::chrono::seconds(2), [&] { return S->live == 0; });
   }
-  S->cv_complete.notify_all();
-  if (S->finish.joinable()) S->finish.join();
+  for (auto& t : S->setup)
+    if (t.joinable()) gone ? t.join() : t.detach();
+  for (std::thread* t : {&S->sched, &S->finish})
+    if (t->joinable()) gone ? t->join() : t->detach();
+  if (S->lost) {
+    // What the device may still write to stays allocated, and so does the server
+    // where a thread that will not return holds it.
+    if (gone) delete S;
+    return;
+  }
   // built after the scheduler stopped
   for (Request* r : S->incoming) retire(S, r);
   S->incoming.clear();

@@ -260,6 +260,7 @@ class Server {
     return U;
   }
   void release(long long id) { check(ma_server_release(s_, id)); }
+  void set_wait_limit(double seconds) { check(ma_server_set_wait_limit(s_, seconds)); }
   double now() { return ma_server_now(s_); }
 
  private:

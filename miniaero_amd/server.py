@@ -66,6 +66,11 @@ class Server:
         _lib.check(self._L.ma_server_plan_cache(self._h, ctypes.byref(h), ctypes.byref(m)))
         return dict(hits=h.value, misses=m.value)
 
+    def set_wait_limit(self, seconds: float) -> None:
+        """Longest wait on the device before unfinished requests fail with
+        MA_ERR_DEVICE (120 s unless set)."""
+        _lib.check(self._L.ma_server_set_wait_limit(self._h, float(seconds)))
+
     def now(self) -> float:
         return float(self._L.ma_server_now(self._h))
 
