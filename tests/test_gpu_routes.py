@@ -224,3 +224,109 @@ def test_state_read_while_another_thread_steps(graph):
             done.set()
             s.close()
     assert np.array_equal(*states)
+
+
+def _states(case, variants, steps):
+    out = []
+    for v in variants:
+        s = M.TimeSolverExplicitRK4(case[0], case[1].replace(**v.get("options", {})))
+        try:
+            if v.get("persistent"):
+                s.set_persistent(True)
+            s.initialize()
+            s.step(steps)
+            out.append([s.state(), s.residual()])
+            if case[1].second_order_space or case[1].viscous:
+                out[-1] += list(s.gradients())
+        finally:
+            s.close()
+    return out
+
+
+def _same(states):
+    assert np.isfinite(states[0][0]).all()
+    for other in states[1:]:
+        for a, b in zip(states[0], other):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(33, 17, 9), (21, 19, 11)])
+def test_own_side_form_with_partial_blocks(shape, precision):
+    """Viscous second order in tiles of more than 128 cells, where a cell's three
+    high faces are one wavefront's (pair.hpp, own_faces), and tiles of a last
+    block with fewer than 64 cells: inactive lanes, neighbours behind the block's
+    end, padded chunks.  FP64 equals the oracle; FP32 the small default tiles."""
+    from test_gpu_parity import Pair
+    tiles = [(4, 8, 8), (3, 7, 9), (5, 5, 10), (-1, 0, 0)]
+    cells = [256 if t[0] < 0 else t[0] * t[1] * t[2] for t in tiles]
+    n = shape[0] * shape[1] * shape[2]
+    assert all(c > 128 for c in cells) and cells[1] % 64 and cells[2] % 64 and n % 256 % 64
+    _same(_states(_case(shape, precision=precision),
+                  [dict(options=dict(tile_shape=t)) for t in [(0, 0, 0)] + tiles], 4))
+    if not precision:
+        for t in tiles[:3]:
+            o = _case(shape)[1]
+            p = Pair(dict({k: getattr(o, k) for k in ("problem_type", "lx", "ly", "lz", "nx", "ny", "nz", "dt", "ntimesteps",
+                                                      "second_order_space", "viscous", "limiter", "ic_kind", "perturb",
+                                                      "seed", "bc_kind")}, tile_shape=t))
+            try:
+                G, R = p.step(3)
+                assert np.array_equal(G, R)
+            finally:
+                p.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("scheme", [(1, 0, 1), (1, 1, 0), (0, 1, 0)])
+def test_skew_tiles_walked_and_long(scheme, precision):
+    """Skew meshes of 93k cells: workgroups that walk several tiles each, lists of
+    more entries than a workgroup has threads; the default layout's bits."""
+    o = _case((101, 33, 28), scheme, precision=precision)[1]
+    _same(_states((rotated_mesh(o), o),
+                  [dict(options=x) for x in ({}, dict(tile_shape=(3, 5, 7), workgroups_per_cu=1),
+                                             dict(tile_shape=(4, 8, 8)),
+                                             dict(tile_shape=(4, 8, 8), workgroups_per_cu=1))], 2))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("scheme", [(0, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 0)])
+def test_persistent_steps_on_skew_meshes(scheme, precision):
+    o = _case((19, 12, 9), scheme, precision=precision)[1]
+    _same(_states((rotated_mesh(o), o), [dict(), dict(persistent=True)], 3))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("scheme", [(0, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 0)])
+def test_internal_faces_pointing_down_their_axis(scheme, precision):
+    """A box some of whose internal faces have their cells the other way round:
+    along an axis, but of the class of faces along none."""
+    from test_skew_plan import _frames
+    md, o = _case((13, 11, 10), scheme, precision=precision)
+    f = md.internal_faces
+    turn = np.arange(f.nfaces_) % 3 == 1
+    f.face_cell_conn = np.where(turn[:, None], f.face_cell_conn[:, ::-1], f.face_cell_conn)
+    f.face_normal = np.where(turn[:, None], -f.face_normal, f.face_normal) + 0.0  # (no -0)
+    f.face_tangent, f.face_binormal = _frames(f.face_normal)
+    f.cell_flux_index = f.permute_vector = None
+    assert md.plan()["derived_frames"]
+    _solo_equals_batched((md, o), _case((6, 5, 4), scheme, precision=precision))
+
+
+@pytest.mark.parametrize("scheme", [(1, 0, 0), (1, 1, 0)])
+@pytest.mark.parametrize("stretch", [1.22, 1.28])
+def test_plates_on_both_sides_of_the_bounds(stretch, scheme):
+    """Stretched plates just inside the paired kernels' largest ratio of area times
+    displacement to volume, 2^14, and just beyond it, as the default tiles of runs
+    of this size tell: the oracle's bits."""
+    from test_gpu_parity import Pair
+    p = Pair(dict(problem_type=1, lx=1.0, ly=0.05, lz=0.025, nx=48, ny=48, nz=16, y_stretch=stretch, dt=1e-12,
+                  ntimesteps=2, second_order_space=scheme[0], viscous=scheme[1], limiter=scheme[2], ic_kind=2,
+                  perturb=0.01, seed=5))
+    try:
+        ratio = (1 / 48) / (2 * 0.05 * (stretch - 1) / (stretch ** 48 - 1))
+        assert p.gpu.tile_shape()[0] == ((4, 4, 8) if ratio < 2 ** 14 else (4, 4, 4))
+        G, R = p.step(2)
+        assert np.isfinite(R).all() and np.array_equal(G, R)
+    finally:
+        p.close()
