@@ -1,5 +1,6 @@
-// internal.hpp -- interface between the solver (solver.hip) and the served
-// form (server.hip) inside libminiaero_amd; not part of the C ABI.
+// internal.hpp -- interfaces inside libminiaero_amd, between the solver
+// (solver.hip) and the served form (server.hip) and the kernels of steps.hip;
+// not part of the C ABI.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -9,6 +10,12 @@
 #include "../../include/miniaero.h"
 
 namespace ma {
+
+// Kernel of the persistent form for the options' scheme (steps.hip); pair: 0 the
+// general kernels' phases, 1 the paired ones, 2 those for skew meshes.
+const void* steps_kernel(const ma_options& opt, bool fp32, int pair);
+// Paired flux kernel of the form whose workgroups walk several tiles (steps.hip).
+const void* walk_kernel(const ma_options& opt, bool fp32, bool skew, bool own, bool wall);
 
 struct PlannedCase;
 struct LayoutPlan;

@@ -1447,6 +1447,16 @@ __device__ __forceinline__ bool grid_sync(unsigned* gsync, unsigned& gen, long l
   return *stop == 0;
 }
 
+// The paired flux kernel of a form; wall: the run has no-slip faces.
+template <bool kSkew, bool kOwn, bool SO, bool kWalk, class Visc, class T>
+auto pair_flux_form(bool wall) {
+  constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
+  return wall ? k_flux_pair<kSkew, kOwn, SO, true, kWalk, Inviscid, Visc, T>
+              : k_flux_pair<kSkew, kOwn, SO, VW, kWalk, Inviscid, Visc, T>;
+}
+
+#ifdef MA_STEPS_UNIT  // steps.hip: the kernels of forms on request
+
 // Register budget of k_steps: the gradient and flux phases share one
 // allocation, which in FP64 does not fit the 3-wave budget of the separate
 // kernels without spilling, so FP64 runs 2 waves per SIMD (1 for the viscous
@@ -1460,7 +1470,9 @@ constexpr int kStepsWaves = sizeof(T) == 8 ? (kViscousSO ? 1 : 2) : 1;
 // kPair: 0 the general kernels' phases, 1 the paired ones, 2 those for skew meshes
 template <bool SO, class Inv, class Visc, class Lim, class T, int kPair>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(kStepsWaves<SO && Visc::isViscous, T>)))
-void k_steps(PersistArgs a, Inv inv, Visc visc) {
+void k_steps(PersistArgs a) {
+  const Visc visc{a.prandtl};
+  const Inv inv{};
   // TimeSolverExplicitRK4.h:187-195: alpha = {0, 1/2, 1/2, 1}, beta = {1/6,
   // 1/3, 1/3, 1/6}, selected rather than indexed (an indexed array would sit
   // in scratch)
@@ -1547,6 +1559,66 @@ void k_steps(PersistArgs a, Inv inv, Visc visc) {
     }
   }
 }
+
+// Kernel of the persistent form for a run's options, pair as kPair above.
+template <bool SO, class Visc, class Lim, class T>
+const void* steps_kernel_of(int pair) {
+  auto kern = k_steps<SO, Inviscid, Visc, Lim, T, 0>;
+  if constexpr (ma::pair_policies<Visc, Lim, Boundaries>) {
+    if (pair) kern = pair == 2 ? k_steps<SO, Inviscid, Visc, Lim, T, 2> : k_steps<SO, Inviscid, Visc, Lim, T, 1>;
+  }
+  return reinterpret_cast<const void*>(kern);
+}
+
+template <bool SO, class Visc, class T>
+const void* steps_lim(const ma_options& o, int pair) {
+  return o.limiter == MA_LIMITER_VANALBADA ? steps_kernel_of<SO, Visc, ma::VanAlbadaLimiter, T>(pair)
+                                           : steps_kernel_of<SO, Visc, ma::VenkatLimiter, T>(pair);
+}
+
+template <class T>
+const void* steps_t(const ma_options& o, int pair) {
+  const bool so = o.second_order_space != 0, visc = o.viscous != 0;
+  if (so && visc) return steps_lim<true, ma::NewtonianViscousFlux, T>(o, pair);
+  if (so) return steps_lim<true, ma::NoViscousFlux, T>(o, pair);
+  if (visc) return steps_lim<false, ma::NewtonianViscousFlux, T>(o, pair);
+  return steps_lim<false, ma::NoViscousFlux, T>(o, pair);
+}
+
+// The walking form of the paired flux kernel.
+template <bool SO, class Visc, class T>
+const void* walk_of(bool skew, bool own, bool wall) {
+  constexpr bool kOwn = SO && Visc::isViscous;
+  if constexpr (ma::pair_policies<Visc, ma::VenkatLimiter, Boundaries> ||
+                ma::pair_policies<Visc, ma::VanAlbadaLimiter, Boundaries>) {
+    const auto kern = skew          ? pair_flux_form<true, false, SO, true, Visc, T>(wall)
+                      : kOwn && own ? pair_flux_form<false, kOwn, SO, true, Visc, T>(wall)
+                                    : pair_flux_form<false, false, SO, true, Visc, T>(wall);
+    return reinterpret_cast<const void*>(kern);
+  }
+  return nullptr;
+}
+
+template <class T>
+const void* walk_t(const ma_options& o, bool skew, bool own, bool wall) {
+  const bool so = o.second_order_space != 0, visc = o.viscous != 0;
+  if (so && visc) return walk_of<true, ma::NewtonianViscousFlux, T>(skew, own, wall);
+  if (so) return walk_of<true, ma::NoViscousFlux, T>(skew, own, wall);
+  if (visc) return walk_of<false, ma::NewtonianViscousFlux, T>(skew, own, wall);
+  return walk_of<false, ma::NoViscousFlux, T>(skew, own, wall);
+}
+
+}  // namespace
+
+const void* ma::walk_kernel(const ma_options& o, bool fp32, bool skew, bool own, bool wall) {
+  return fp32 ? walk_t<float>(o, skew, own, wall) : walk_t<double>(o, skew, own, wall);
+}
+
+const void* ma::steps_kernel(const ma_options& o, bool fp32, int pair) {
+  return fp32 ? steps_t<float>(o, pair) : steps_t<double>(o, pair);
+}
+
+#else  // everything else
 
 // ------------------------------------------------------------- host side --
 
@@ -3434,14 +3506,12 @@ inline int resident(const ma_solver* s, int per) {
 // threads), else 4 wavefronts walking the chunks.
 inline int pair_threads(int max_faces) { return max_faces <= kPairMaxThreads ? max_faces : kTile; }
 
-template <bool kSkew, bool kOwn, bool SO, class Inv, class Visc, class T>
+template <bool kSkew, bool kOwn, bool SO, class Visc, class T>
 auto pair_flux_kernel(const ma_solver* s) {
-  constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
+  using Kernel = decltype(pair_flux_form<kSkew, kOwn, SO, false, Visc, T>(false));
   if (s->wg_per_cu > 0)
-    return s->wall ? k_flux_pair<kSkew, kOwn, SO, true, true, Inv, Visc, T>
-                   : k_flux_pair<kSkew, kOwn, SO, VW, true, Inv, Visc, T>;
-  return s->wall ? k_flux_pair<kSkew, kOwn, SO, true, false, Inv, Visc, T>
-                 : k_flux_pair<kSkew, kOwn, SO, VW, false, Inv, Visc, T>;
+    return reinterpret_cast<Kernel>(const_cast<void*>(ma::walk_kernel(s->opt, s->fp32, kSkew, kOwn, s->wall)));
+  return pair_flux_form<kSkew, kOwn, SO, false, Visc, T>(s->wall);
 }
 
 template <bool SO, class Inv, class Visc, class Lim, class T>
@@ -3486,9 +3556,9 @@ void run_stage(ma_solver* s, int irk) {
       }
       constexpr bool kOwn = SO && Visc::isViscous;
       double* time_dev = irk == 3 && !s->any_cfl ? s->time_dev : nullptr;  // see advance_time
-      const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Inv, Visc, T>(s)
-                        : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Inv, Visc, T>(s)
-                                         : pair_flux_kernel<false, false, SO, Inv, Visc, T>(s);
+      const auto kern = s->skew            ? pair_flux_kernel<true, false, SO, Visc, T>(s)
+                        : kOwn && s->own ? pair_flux_kernel<false, kOwn, SO, Visc, T>(s)
+                                         : pair_flux_kernel<false, false, SO, Visc, T>(s);
       s->launch("k_flux", [&] {
         hipLaunchKernelGGL(kern, dim3(resident(s, s->t.per_xcd) * kXcds), dim3(pair_threads(s->t.max_faces)),
                            (size_t)s->t.max_faces * 5 * sizeof(T), s->stream, m, s->t, static_cast<const T*>(Vs),
@@ -3599,22 +3669,19 @@ void dispatch(ma_solver* s, int n) {
 // tiles or cell blocks), all of them walking every phase.  Waits for the
 // device to be idle before the launch and for the launch itself, since a
 // barrier wait that ran over its limit is reported here.
-template <bool SO, class Inv, class Visc, class Lim, class T>
-ma_status run_persistent(ma_solver* s, int nsteps) {
+ma_status persist(ma_solver* s, int nsteps) {
   if (nsteps == 0) return MA_OK;
-  constexpr bool FV = SO && !Visc::isViscous;
-  auto kern = k_steps<SO, Inv, Visc, Lim, T, 0>;
-  if constexpr (ma::pair_policies<Visc, Lim, Boundaries>) {
-    if (s->pair) kern = s->skew ? k_steps<SO, Inv, Visc, Lim, T, 2> : k_steps<SO, Inv, Visc, Lim, T, 1>;
-  }
-  const size_t lds = std::max((size_t)s->t.max_faces * 5 * sizeof(T),
-                              FV || s->pair ? (size_t)0 : (size_t)kBlock * kStageRow<T> * sizeof(T));
+  const bool fv = s->opt.second_order_space && !s->opt.viscous;
+  const void* kern = ma::steps_kernel(s->opt, s->fp32, !s->pair ? 0 : s->skew ? 2 : 1);
+  const size_t row = s->fp32 ? kStageRow<float> * sizeof(float) : kStageRow<double> * sizeof(double);
+  const size_t lds = std::max((size_t)s->t.max_faces * 5 * (s->fp32 ? sizeof(float) : sizeof(double)),
+                              fv || s->pair ? (size_t)0 : (size_t)kBlock * row);
   int coop = 0, per_cu = 0, wall_khz = 0;
   MA_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, s->device));
   if (!coop) return ma::fail(MA_ERR_UNSUPPORTED, "persistent steps: the device has no cooperative launch");
   MA_HIP(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, s->device));
   hipFuncAttributes fa{};
-  MA_HIP(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(kern)));
+  MA_HIP(hipFuncGetAttributes(&fa, kern));
   if (fa.localSizeBytes > 0)
     return ma::fail(MA_ERR_UNSUPPORTED, "persistent steps: the kernel uses scratch memory, which can keep "
                                         "workgroups of a cooperative launch from being resident together");
@@ -3657,15 +3724,13 @@ ma_status run_persistent(ma_solver* s, int nsteps) {
   a.viscous = s->opt.viscous;
   a.per_blocks = (nblocks(nc) + kXcds - 1) / kXcds;
   a.prandtl = effective_prandtl(s->opt);
-  Visc visc{a.prandtl};
-  Inv inv{};
-  void* args[] = {&a, &inv, &visc};
+  void* args[] = {&a};
   // The grid is sized to every workgroup slot of the device, so no other
   // kernel of the process may hold slots while it is placed: wait for the
   // whole device (other solvers' streams included) first.
   MA_HIP(hipDeviceSynchronize());
   MA_HIP(hipMemsetAsync(s->gsync, 0, 4 * sizeof(unsigned), s->stream));
-  MA_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(grid), dim3(kTile), args, lds,
+  MA_HIP(hipLaunchCooperativeKernel(kern, dim3(grid), dim3(kTile), args, lds,
                                     s->stream));
   unsigned exceeded = 0;
   MA_HIP(hipMemcpyAsync(&exceeded, s->gsync + 2, sizeof(exceeded), hipMemcpyDeviceToHost, s->stream));
@@ -3676,23 +3741,6 @@ ma_status run_persistent(ma_solver* s, int nsteps) {
   s->v0_valid = true;
   return MA_OK;
 }
-
-template <bool SO, class Visc, class T>
-ma_status persist_lim(ma_solver* s, int n) {
-  if (s->opt.limiter == MA_LIMITER_VANALBADA) return run_persistent<SO, Inviscid, Visc, ma::VanAlbadaLimiter, T>(s, n);
-  return run_persistent<SO, Inviscid, Visc, ma::VenkatLimiter, T>(s, n);
-}
-
-template <class T>
-ma_status persist_t(ma_solver* s, int n) {
-  const bool so = s->opt.second_order_space != 0, visc = s->opt.viscous != 0;
-  if (so && visc) return persist_lim<true, ma::NewtonianViscousFlux, T>(s, n);
-  if (so) return persist_lim<true, ma::NoViscousFlux, T>(s, n);
-  if (visc) return persist_lim<false, ma::NewtonianViscousFlux, T>(s, n);
-  return persist_lim<false, ma::NoViscousFlux, T>(s, n);
-}
-
-ma_status persist(ma_solver* s, int n) { return s->fp32 ? persist_t<float>(s, n) : persist_t<double>(s, n); }
 
 void drop_graphs(ma_solver* s) {
   for (auto& g : s->graph)
@@ -4731,3 +4779,5 @@ int solver_cur(const ma_solver* s) { return s->cur; }
 void solver_set_stream(ma_solver* s, hipStream_t stream) { s->stream = stream; }
 
 }  // namespace ma
+
+#endif  // MA_STEPS_UNIT
