@@ -3461,7 +3461,7 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
   const size_t n5 = (size_t)5 * nc;
   const size_t tsize = s->fp32 ? sizeof(float) : sizeof(double);
   const size_t np = s->pair ? (size_t)s->m.ns : (size_t)nc;  // plane length of V, grad and fv
-  const size_t nu = std::max<size_t>(n5, 15);  // (download_records)
+  const size_t nu = (size_t)15 * ((nc + 2) / 3);  // 5 * nc, rounded up for download_records
   if ((st = s->alloc(&s->U[0], nu)) || (st = s->alloc(&s->U[1], nu)) || (st = s->alloc(&s->R, n5)) ||
       (st = s->alloc_bytes(&s->V, 5 * np * tsize)) || (st = s->alloc_bytes(&s->V2, 5 * np * tsize)) ||
       (st = s->alloc_bytes(&s->grad, (size_t)kRec * np * tsize)) ||
@@ -3813,12 +3813,43 @@ ma_status advance(ma_solver* s, int nsteps) {
   return MA_OK;
 }
 
-// The state or the residual to the caller's order, through the state buffer that
-// is free between steps.
+// Small runs are put into the caller's order by the host: the copy of a few
+// planes and a loop over cells that are in its caches cost less than another
+// launch, or a copy for each part that the staging buffer holds.  us, host /
+// device: states of 1k cells 13 / 25, 8k 32 / 36, 16k 57 / 49; gradients and
+// limiters, FP64, of 1k cells 20 / 137, 8k 158 to 211 / 192, 16k 287 / 247, FP32
+// 16k 191 / 244, 65k 620 to 680 / 704; limiters alone of 1k cells 15 to 18 / 25,
+// 2k 19 to 26 / 27, 4k 28 to 44 / 30.
+constexpr int kHostStateCells = 8192, kHostLimiterCells = 2048;
+template <class S>
+constexpr int kHostRecordCells = sizeof(S) == 8 ? 8192 : 65536;
+
+// n values of src in host memory (null, with the error in *st, on failure).
+template <class S>
+std::unique_ptr<S[]> planes_to_host(ma_solver* s, const S* src, size_t n, ma_status* st) {
+  std::unique_ptr<S[]> h(new (std::nothrow) S[n]);
+  *st = MA_OK;
+  if (!h) *st = ma::fail(MA_ERR_NOMEM, "out of host memory");
+  else if (hipMemcpyAsync(h.get(), src, n * sizeof(S), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
+           hipStreamSynchronize(s->stream) != hipSuccess)
+    *st = ma::fail(MA_ERR_DEVICE, "copying values to the host failed");
+  if (*st) h.reset();
+  return h;
+}
+
+// The state or the residual to the caller's order, on the device through the
+// state buffer that is free between steps.
 ma_status download_state(ma_solver* s, bool residual, double* host) {
   const int nc = s->m.nc;
   std::lock_guard<std::mutex> lock(s->queueing);
   const double* src = residual ? s->R : s->U[s->cur];
+  if (nc <= kHostStateCells) {
+    ma_status st;
+    const auto h = planes_to_host(s, src, (size_t)5 * nc, &st);
+    for (int c = 0; h && c < nc; ++c)
+      for (int k = 0; k < 5; ++k) host[(size_t)c * 5 + k] = h[(size_t)k * nc + s->dev_of[c]];
+    return st;
+  }
   double* raw = s->U[1 - s->cur];
   hipLaunchKernelGGL(k_state_out, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, s->org, src, raw);
   MA_HIP(hipGetLastError());
@@ -3828,11 +3859,24 @@ ma_status download_state(ma_solver* s, bool residual, double* host) {
 }
 
 // Gradient records to the caller's order, grad (n x 5 x 3) and lim (n x 5),
-// either may be null, through the same buffer: all limiters, or the gradients of
-// a third of the cells at a time.
+// either may be null, on the device through the same buffer: all limiters, or the
+// gradients of a third of the cells at a time.
 template <class S>
 ma_status download_records(ma_solver* s, const S* rec, double* grad, double* lim) {
   const int nc = s->m.nc, np = s->pair ? s->m.ns : 0;
+  ma_status st = MA_OK;
+  if (nc <= (grad ? kHostRecordCells<S> : kHostLimiterCells)) {
+    constexpr int W = 16 / (int)sizeof(S);
+    const auto h = planes_to_host(s, rec, (size_t)kRec * (np ? np : nc), &st);
+    for (int c = 0; h && c < nc; ++c) {
+      const size_t d = s->dev_of[c];
+      // a block per cell, or planes of vectors on paired meshes (rec_at)
+      auto at = [&](int j) { return np ? h[((size_t)(j / W) * np + d) * W + j % W] : h[d * kRec + j]; };
+      for (int j = 0; grad && j < 15; ++j) grad[(size_t)c * 15 + j] = at(j);
+      for (int k = 0; lim && k < 5; ++k) lim[(size_t)c * 5 + k] = at(15 + k);
+    }
+    return st;
+  }
   double* raw = s->U[1 - s->cur];
   auto part = [&](int j0, int nj, int c0, int n, double* host) -> ma_status {
     hipLaunchKernelGGL(k_records_out<S>, dim3(nblocks(nc)), dim3(kBlock), 0, s->stream, nc, s->org, rec, np, j0, nj,
@@ -3842,9 +3886,8 @@ ma_status download_records(ma_solver* s, const S* rec, double* grad, double* lim
                           s->stream));
     return MA_OK;
   };
-  ma_status st = MA_OK;
   if (lim && (st = part(15, 5, 0, nc, lim))) return st;
-  const int third = std::max(1, nc / 3);  // (U holds at least 15 values)
+  const int third = (nc + 2) / 3;  // (U holds 15 values for each)
   for (int c0 = 0; grad && c0 < nc; c0 += third)
     if ((st = part(0, 15, c0, std::min(third, nc - c0), grad))) return st;
   MA_HIP(hipStreamSynchronize(s->stream));

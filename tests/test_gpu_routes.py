@@ -159,6 +159,28 @@ def test_gradients_read_in_parts(shape, precision):
         s.close()
 
 
+@pytest.mark.parametrize("precision,shape", [(0, (16, 16, 8)), (0, (23, 10, 9)), (0, (32, 16, 16)), (0, (27, 19, 16)),
+                                             (1, (64, 32, 32)), (1, (41, 40, 40))])
+def test_reads_ordered_by_the_host_and_on_the_device(precision, shape):
+    """State, residual, gradients and limiters on both sides of the sizes up to
+    which the host puts them into order: 2048 and 8192 cells, 65536 in FP32."""
+    from miniaero_amd import _lib
+    case = _case(shape, precision=precision)
+    small = _case((3, 2, 2), precision=precision, **RAMP)
+    _solo_equals_batched(case, small)
+    s = M.TimeSolverExplicitRK4(*case)
+    try:
+        s.initialize()
+        s.step(2)
+        g, lim = s.gradients()
+        g1, l1 = np.empty_like(g), np.empty_like(lim)
+        _lib.check(s._L.ma_solver_get_gradients(s._h, g1.ctypes.data_as(_lib._D), None))
+        _lib.check(s._L.ma_solver_get_gradients(s._h, None, l1.ctypes.data_as(_lib._D)))
+        assert np.array_equal(g, g1) and np.array_equal(lim, l1)
+    finally:
+        s.close()
+
+
 def test_default_tiles():
     """4x4x4 up to 128 cells per CU, 4x4x8 above for runs on the paired kernels
     (4x4x4 for others: stretched beyond their bounds, a FP32 ramp whose area
