@@ -77,6 +77,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1993,7 +1994,7 @@ struct Layout {
   // geometry records of the faces (see dedupe_geometry): the record of each
   // face, and kGeoVals FP64 values per record
   std::vector<int> fgeo;
-  std::vector<double> geo;
+  RawVector<double> geo;
   // every area vector has at most one nonzero component and every cell
   // volume has a finite reciprocal in FP32 and FP64 (DevMesh::axis)
   bool axis = false;
@@ -2002,7 +2003,7 @@ struct Layout {
 };
 
 // Host threads for planning one mesh of nc cells (cases of a batch are planned
-// side by side instead, one thread each).
+// side by side and share the threads there are).
 int plan_threads(int nc) {
   return std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), 1 + nc / 8192}));
 }
@@ -2349,7 +2350,7 @@ constexpr int kGeoReuse = 8;
 class GeoTable {
  public:
   // Number of the record r, appended to geo when it is new.
-  int find(const double* r, std::vector<double>& geo) {
+  int find(const double* r, RawVector<double>& geo) {
     if (2 * count_ >= slots_.size()) grow(geo);
     for (size_t i = hash(r) & (slots_.size() - 1);; i = (i + 1) & (slots_.size() - 1)) {
       if (slots_[i] < 0) {
@@ -2371,7 +2372,7 @@ class GeoTable {
     }
     return (size_t)(h ^ (h >> 32));
   }
-  void grow(const std::vector<double>& geo) {
+  void grow(const RawVector<double>& geo) {
     slots_.assign(std::max<size_t>(1024, 4 * slots_.size()), -1);
     for (size_t k = 0; k < count_; ++k) {
       size_t i = hash(&geo[k * kGeoVals]) & (slots_.size() - 1);
@@ -2459,7 +2460,9 @@ inline bool cell_in_bounds(double vol, double area, double disp) {
 }
 
 // The runs of the loops are spread over host threads: on one, planning a mesh
-// cost up to half as much again as without the paired kernels' tables.
+// cost up to half as much again as without the paired kernels' tables.  The flags
+// are written once a run: written for every face that is along no axis, they made
+// the loops five times slower on skew meshes.
 void find_pairs(Layout& L, int threads) {
   PairPlan& P = L.pair;
   P = PairPlan();
@@ -2467,28 +2470,35 @@ void find_pairs(Layout& L, int threads) {
   if (!L.derive_frame) return;
   const size_t ng = L.geo.size() / kGeoVals;
   P.axis_of.assign(ng, -1);
-  std::vector<double> amax(ng, 0.0), dmax(ng, 0.0);
+  RawVector<double> amax(ng), dmax(ng);
   std::atomic<bool> out{false}, skew{false}, fp32{true};  // out: outside the bounds
   for_runs(threads, (int)ng, 4096, [&](int r0, int r1) {
-    for (int r = r0; r < r1 && !out; ++r) {
+    bool in = !out, small = false;
+    for (int r = r0; r < r1 && in; ++r) {
       const FaceBounds b = face_bounds(&L.geo[(size_t)r * kGeoVals], false);
       P.axis_of[r] = (signed char)b.axis;
       amax[r] = b.area;
       dmax[r] = b.disp;
-      if (!b.in) out = true;
-      if (!b.fp32) fp32 = false;
+      in = b.in;
+      small = small || !b.fp32;
     }
+    if (!in) out = true;
+    if (small) fp32 = false;
   });
   if (out) return;
   for_runs(threads, nf, 16384, [&](int f0, int f1) {
-    for (int f = f0; f < f1 && !out; ++f) {
-      if (f < nif && !apart(&L.geo[(size_t)L.fgeo[f] * kGeoVals + 6])) out = true;
-      if (face_class(L, f) == kSkewFace) skew = true;
+    bool in = !out, any = false;
+    for (int f = f0; f < f1 && in; ++f) {
+      in = f >= nif || apart(&L.geo[(size_t)L.fgeo[f] * kGeoVals + 6]);
+      any = any || face_class(L, f) == kSkewFace;
     }
+    if (!in) out = true;
+    if (any) skew = true;
   });
   if (out) return;
   for_runs(threads, nc, 4096, [&](int c0, int c1) {
-    for (int c = c0; c < c1 && !out; ++c) {
+    bool in = !out, any = skew;
+    for (int c = c0; c < c1 && in; ++c) {
       double am = 0.0, dm = 0.0;
       unsigned sides = 0;
       for (int q = 0; q < kMaxSlots; ++q) {
@@ -2500,11 +2510,13 @@ void find_pairs(Layout& L, int threads) {
         const int f = e >> 1, r = L.fgeo[f];
         am = std::max(am, amax[r]);
         dm = std::max(dm, dmax[r]);
-        if (!skew) sides |= 1u << cell_side(L, f, e & 1);
+        if (!any) sides |= 1u << cell_side(L, f, e & 1);
       }
-      if (!cell_in_bounds(L.vol[c], am, dm)) out = true;
-      if (sides != 0x3f) skew = true;  // (two faces on one side: the cell's slots are not one per direction)
+      in = cell_in_bounds(L.vol[c], am, dm);
+      any = any || sides != 0x3f;  // (two faces on one side: the cell's slots are not one per direction)
     }
+    if (!in) out = true;
+    if (any) skew = true;
   });
   if (out) return;
   P.fp32 = fp32;
@@ -2519,9 +2531,9 @@ void list_pairs(Layout& L, int threads) {
   const int nc = L.nc, nif = L.nif, nf = L.nf, ntiles = L.ntiles;
   const size_t ng = L.geo.size() / kGeoVals;
   const int* fslot = nullptr;  // skew: a face's slot in its left and its right cell
-  std::vector<int> fslots;
+  RawVector<int> fslots;
   if (P.skew) {
-    fslots.assign(2 * (size_t)nf, 0);
+    fslots.resize(2 * (size_t)nf);
     fslot = fslots.data();
   }
   P.nbr.resize((size_t)kMaxSlots * nc);
@@ -2720,7 +2732,12 @@ void list_pairs(Layout& L, int threads) {
       x = now[k] | (x & ~mask);
     }
   };
-  renumber(P.ent, 2 * ng, -1, P.srec);
+  if (ng == (size_t)nf) {  // a record per face: every slot has one of its own
+    P.srec.assign(P.ent.begin(), P.ent.end());
+    std::iota(P.ent.begin(), P.ent.end(), 0);
+  } else {
+    renumber(P.ent, 2 * ng, -1, P.srec);
+  }
   renumber(P.gid, ng, (1 << kCellBits) - 1, P.frec);
   if (P.srec.size() >= (1u << kCellBits)) {  // 32-bit byte offsets into the record planes
     P = PairPlan();
@@ -3124,11 +3141,15 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
     std::vector<ma_status> status(ncases, MA_OK);
     std::vector<std::string> message(ncases);
     const int nthreads = std::min(16, (int)std::thread::hardware_concurrency());
+    // batches of fewer cases than threads: the rest helps inside the cases
+    auto inside = [&](int k) {
+      return std::max(1, std::min(nthreads / ncases, plan_threads(mds[k]->num_owned_cells)));
+    };
     for_runs(nthreads, ncases, 1, [&](int k, int) {
       try {
-        status[k] = plan_layout(mds[k], shape, 1, parts[k]);
+        status[k] = plan_layout(mds[k], shape, inside(k), parts[k]);
         if (status[k]) message[k] = ma::last_error();
-        else if (pairs != Pairs::none) find_pairs(parts[k], 1);
+        else if (pairs != Pairs::none) find_pairs(parts[k], inside(k));
       } catch (const std::bad_alloc&) {
         status[k] = MA_ERR_NOMEM;
         message[k] = "plan: out of host memory";
@@ -3141,7 +3162,7 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
     // the paired kernels take the batch if they take every case, in one form
     bool all = true;
     for (const Layout& x : parts) all = all && usable(x) && x.pair.skew == parts[0].pair.skew;
-    if (all) for_runs(nthreads, ncases, 1, [&](int k, int) { list_pairs(parts[k], 1); });
+    if (all) for_runs(nthreads, ncases, 1, [&](int k, int) { list_pairs(parts[k], inside(k)); });
     else
       for (Layout& x : parts) x.pair = PairPlan();
     merge_layouts(parts, L, P.tile_case, P.case_tiles, P.bc_case, P.cell_case, nthreads);
