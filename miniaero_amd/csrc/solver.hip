@@ -1410,6 +1410,16 @@ struct PersistArgs {
   double prandtl;
 };
 
+// The paired flux kernel of a form; wall: the run has no-slip faces.
+template <bool kSkew, bool kOwn, bool SO, bool kWalk, class Visc, class T>
+auto pair_flux_form(bool wall) {
+  constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
+  return wall ? k_flux_pair<kSkew, kOwn, SO, true, kWalk, Inviscid, Visc, T>
+              : k_flux_pair<kSkew, kOwn, SO, VW, kWalk, Inviscid, Visc, T>;
+}
+
+#ifdef MA_STEPS_UNIT  // steps.hip: the kernels of forms on request
+
 // Grid-wide barrier: every workgroup of the launch arrives once per call.
 // The arrivals are counted in gsync[0]; the last one resets the count and
 // advances the generation gsync[1], for which the others wait.  The fences
@@ -1447,16 +1457,6 @@ __device__ __forceinline__ bool grid_sync(unsigned* gsync, unsigned& gen, long l
   __syncthreads();
   return *stop == 0;
 }
-
-// The paired flux kernel of a form; wall: the run has no-slip faces.
-template <bool kSkew, bool kOwn, bool SO, bool kWalk, class Visc, class T>
-auto pair_flux_form(bool wall) {
-  constexpr bool VW = Visc::isViscous;  // viscous kernels have the no-slip wall's flux in any case
-  return wall ? k_flux_pair<kSkew, kOwn, SO, true, kWalk, Inviscid, Visc, T>
-              : k_flux_pair<kSkew, kOwn, SO, VW, kWalk, Inviscid, Visc, T>;
-}
-
-#ifdef MA_STEPS_UNIT  // steps.hip: the kernels of forms on request
 
 // Register budget of k_steps: the gradient and flux phases share one
 // allocation, which in FP64 does not fit the 3-wave budget of the separate
@@ -2004,8 +2004,9 @@ struct Layout {
 
 // Host threads for planning one mesh of nc cells (cases of a batch are planned
 // side by side and share the threads there are).
+constexpr int kPlanThreads = 16;
 int plan_threads(int nc) {
-  return std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), 1 + nc / 8192}));
+  return std::max(1, std::min({kPlanThreads, (int)std::thread::hardware_concurrency(), 1 + nc / 8192}));
 }
 
 // fn(begin, end) for [0, n) in runs of `grain`, spread over up to `threads` host
@@ -3107,7 +3108,10 @@ bool expects_pairs(int ncases, const ma_mesh_data* const* mds, Pairs pairs) {
   return true;
 }
 
-ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, Pairs pairs, RunPlan& P) {
+// most: host threads it may take (the served form plans on its setup threads,
+// whose number the server's user chooses, and on no others).
+ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& shape, Pairs pairs, int most,
+                   RunPlan& P) {
   if (!valid_shape(shape)) return ma::fail(MA_ERR_INVALID, "tile shape: extents >= 1 with product <= 256, or all 0");
   P.case_cell_off.assign(ncases + 1, 0);
   long long total_cells = 0, total_faces = 0;
@@ -3124,7 +3128,7 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
   ma_status st = MA_OK;
   Layout& L = P.L;
   auto usable = [&](const Layout& x) { return x.pair.ok && (pairs == Pairs::fp64 || x.pair.fp32); };
-  const int threads = ncases == 1 ? plan_threads(mds[0]->num_owned_cells) : 16;
+  const int threads = std::min(most, ncases == 1 ? plan_threads(mds[0]->num_owned_cells) : kPlanThreads);
   if (ncases == 1) {
     if ((st = plan_layout(mds[0], shape, threads, L))) return st;
     if (pairs != Pairs::none) find_pairs(L, threads);
@@ -3140,7 +3144,7 @@ ma_status plan_run(int ncases, const ma_mesh_data* const* mds, const TileShape& 
     std::vector<Layout> parts(ncases);
     std::vector<ma_status> status(ncases, MA_OK);
     std::vector<std::string> message(ncases);
-    const int nthreads = std::min(16, (int)std::thread::hardware_concurrency());
+    const int nthreads = std::min(most, (int)std::thread::hardware_concurrency());
     // batches of fewer cases than threads: the rest helps inside the cases
     auto inside = [&](int k) {
       return std::max(1, std::min(nthreads / ncases, plan_threads(mds[k]->num_owned_cells)));
@@ -3505,11 +3509,11 @@ ma_status build_planned(ma_solver* s, const RunPlan& P) {
 // paired kernels (null: none).
 ma_status build(ma_solver* s, int ncases, const ma_mesh_data* const* mds, const TileShape* otherwise) {
   RunPlan P;
-  ma_status st = plan_run(ncases, mds, s->shape, pairs_of(s->opt), P);
+  ma_status st = plan_run(ncases, mds, s->shape, pairs_of(s->opt), kPlanThreads, P);
   if (!st && otherwise && !P.L.pair.ok) {
     s->shape = *otherwise;
     P = RunPlan();
-    st = plan_run(ncases, mds, s->shape, Pairs::none, P);
+    st = plan_run(ncases, mds, s->shape, Pairs::none, kPlanThreads, P);
   }
   if (st) return st;
   return build_planned(s, P);
@@ -3924,7 +3928,7 @@ extern "C" ma_status ma_batch_plan(int ncases, const ma_mesh_data* const* meshes
   RunPlan P;
   ma_status st = MA_OK;
   try {
-    st = plan_run(ncases, meshes, kDefaultShape, Pairs::fp64, P);
+    st = plan_run(ncases, meshes, kDefaultShape, Pairs::fp64, kPlanThreads, P);
   } catch (const std::bad_alloc&) {
     st = ma::fail(MA_ERR_NOMEM, "plan: out of host memory");
   }
@@ -4551,7 +4555,7 @@ ma_status plan_layout_shared(const ma_mesh_data* md, const ma_options* opt, std:
   try {
     std::shared_ptr<LayoutPlan> lp = std::make_shared<LayoutPlan>();
     lp->shape = shape;
-    if ((st = plan_run(1, &md, shape, Pairs::none, lp->P))) return st;
+    if ((st = plan_run(1, &md, shape, Pairs::none, 1, lp->P))) return st;
     const Layout& L = lp->P.L;
     lp->host_bytes = vbytes(L.dev_of) + vbytes(L.org_of) + vbytes(L.tile_cptr) + vbytes(L.tptr) +
                      vbytes(L.tfaces) + vbytes(L.slot) + vbytes(L.tslot) + vbytes(L.fl) + vbytes(L.fr) +

@@ -2,11 +2,17 @@
 // times 24 requests through one server, all of which finish.  server_check stall:
 // a server whose device stops (STUB_STALL) fails every unfinished request with
 // MA_ERR_DEVICE within its wait limit, refuses more, and can be destroyed.
+// server_check threads: planning a request takes the server's setup thread alone.
+#include <dirent.h>
+
+#include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <set>
+#include <thread>
 #include <vector>
 #include "miniaero.h"
 
@@ -39,7 +45,45 @@ static ma_options request(int i) {
     }                                                        \
   } while (0)
 
+static int threads_here() {
+  int n = 0;
+  DIR* d = opendir("/proc/self/task");
+  while (const dirent* e = readdir(d)) n += e->d_name[0] != '.';
+  closedir(d);
+  return n;
+}
+
+static int threads() {
+  ma_server_config cfg = {600ll << 20, 1, 1, 0, 0};
+  ma_server* S = nullptr;
+  CHECK(ma_server_create(&cfg, &S) == MA_OK);
+  std::atomic<bool> done{false};
+  std::atomic<int> most{0};
+  std::thread watch([&] {
+    while (!done) most = std::max(most.load(), threads_here());
+  });
+  const int idle = threads_here();
+  ma_options o = request(0);
+  o.nx = 96;
+  o.ny = 48;
+  o.nz = 24;
+  o.ntimesteps = 1;
+  long long id = 0;
+  CHECK(ma_server_submit(S, &o, &id) == MA_OK);
+  ma_case_result r;
+  const double t0 = now();
+  while (ma_server_poll(S, &r, 1, 0.2) == 0) CHECK(now() - t0 < 60.0);
+  CHECK(r.status == MA_OK);
+  done = true;
+  watch.join();
+  std::printf("%d threads, at most %d while planning\n", idle, most.load());
+  CHECK(most <= idle);
+  ma_server_destroy(S);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc > 1 && !std::strcmp(argv[1], "threads")) return threads();
   const bool stall = argc > 1 && !std::strcmp(argv[1], "stall");
   const int passes = stall ? 1 : std::atoi(argv[1]);
   ma_server_config cfg = {600ll << 20, 16, 8, 0, 0};

@@ -48,6 +48,11 @@ def test_requests_through_one_server(check):
     check("80")
 
 
+def test_planning_takes_one_thread_a_request(check):
+    """ma_server_config.setup_threads is how many host threads plan requests."""
+    check("threads")
+
+
 @pytest.mark.parametrize("kind,after,says", [
     ("event", 0, "a step"), ("event", 40, "a step"),   # (a table's upload event may be the one that stops)
     ("sync", 0, "building a case"), ("sync", 100, "building a case|copying a result back")])
