@@ -1,5 +1,6 @@
-// pair.hpp -- kernels for meshes of cells with six faces each (find_pairs in
-// solver.hip has the conditions).  Two forms: axial meshes, where a cell has
+// pair.hpp -- kernels for meshes of cells with six faces each whose geometry is
+// inside the bounds that find_pairs in solver.hip names (plates with cells over
+// 30,000 times as long as high are outside).  Two forms: axial meshes, where a cell has
 // two faces per axis, one on each side, and every area vector lies along an
 // axis (box meshes, stretched or not), and skew meshes (kSkew: ramps, boxes
 // whose area vectors carry rounding noise), where the slots stay in slot order
@@ -43,13 +44,14 @@
 // Measured against the general kernels, microseconds per launch (k_grad,
 // k_flux): FP64 viscous 256 x 128 x 64 plate 227 -> 155, 367 -> 300; FP32
 // viscous 211 x 127 x 45 plate 99 -> 53, 139 -> 107; 48 batched FP32 shock
-// tubes 320 -> 194, 384 -> 318; 4096-cell FP64 plate 10.3 -> 5.3, 14.3 -> 7.3;
+// tubes 320 -> 194, 384 -> 318; 1024-cell FP64 plate 10.5 -> 5.4, 14.5 -> 6.1;
 // first-order 64 x 16 x 16 shock tube 14.1 with its boundary launch -> 5.2.
-// Skew: FP64 321 x 157 x 11 ramp 126 -> 74, 120 -> 97; 2240-cell ramp 13.1 -> 7.0,
-// 10.5 -> 8.0 (its boundary faces were in the gradient launch).
-// At 2.1M cells the flux kernel is bound by HBM and L2: 1.7 GB a launch at 5.5
-// TB/s, most of it records fetched again by the tiles around (96 tiles in flight
-// per XCD against a 4 MB L2); the gradient kernel has its data return 86% busy.
+// Skew: FP64 321 x 157 x 11 ramp 126 -> 74, 120 -> 97; 4096-cell ramp 13.5 -> 7.4,
+// 10.6 -> 5.8 (its boundary faces were in the gradient launch).
+// At 2.1M cells the flux kernel is bound by HBM and L2: 1.39 GB fetched and 0.20
+// written in 285 us, 5.5 TB/s, most of it records fetched again by the tiles
+// around (96 tiles in flight per XCD against a 4 MB L2); the gradient kernel has
+// its data return 86% busy.
 //
 // Every value the kernels keep is formed with the general kernels' operations
 // in the same order, and the terms left out are +-0, so results are the same
@@ -879,7 +881,9 @@ __device__ __forceinline__ void flux_tile_pair(const DevMesh& m, const TileMap& 
 // neighbour of the same 64-cell block from the lane that has it, leaves a load
 // of the cell, one of its neighbour in the next block and the block's edges
 // instead of 6 (L2 reads 31 -> 23 million a launch, k_flux of the 2.1M-cell FP64
-// plate 338 -> 300 us, of the 1.2M-cell FP32 plate 117 -> 107).
+// plate 338 -> 300 us, of the 1.2M-cell FP32 plate 117 -> 107), although a tile's
+// low faces, which come after all blocks, load their own cell a second time: HBM
+// fetches went from 1.11 to 1.39 GB.
 // kWalk: fewer workgroups than tiles, each walking its XCD's run (see k_flux);
 // otherwise one tile per workgroup, a form of its own because the walk's
 // loop-carried values cost the FP64 viscous kernel spills and the FP64 inviscid

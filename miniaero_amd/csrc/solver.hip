@@ -26,9 +26,10 @@
 //            V buffer (stage 3: the next step's, from the new U; R itself
 //            is stored on stage 3 only)
 //
-// Meshes whose cells all have six faces run k_grad_pair and k_flux_pair
-// instead, with their own layout and no boundary launch (pair.hpp); the
-// kernels above are for other meshes, mixed batches and the served form.
+// Meshes whose cells all have six faces and whose geometry is inside the bounds
+// of find_pairs run k_grad_pair and k_flux_pair instead, with their own layout
+// and no boundary launch (pair.hpp); the kernels above are for other meshes,
+// batches of axial and skew meshes together and the served form.
 //
 // Determinism and parity.  The reference scatters face results into cells
 // with atomics; with one thread the additions land in a fixed order: internal
@@ -3548,7 +3549,7 @@ void run_stage(ma_solver* s, int irk) {
   const int nb = nblocks(m.nc);
   double* Un = s->U[s->cur];
   double* Uacc = s->U[1 - s->cur];
-    // the stage's primitives: V for stages 0 and 2, V2 for 1 and 3; stage 0's
+  // the stage's primitives: V for stages 0 and 2, V2 for 1 and 3; stage 0's
   // come from k_prim, the others from the previous stage's flux kernel
   // (stage 3 writes the next step's stage-0 primitives into V, so k_prim
   // runs only when V does not hold them yet)
