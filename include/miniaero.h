@@ -306,7 +306,8 @@ ma_status ma_server_plan_cache(ma_server* srv, long long* hits, long long* misse
  * result back; 120 s unless set here).  When one takes longer and nothing else
  * ends meanwhile, every unfinished request finishes with MA_ERR_DEVICE and
  * ma_server_submit fails with it; destroying the server then frees nothing that
- * the device may still write to.  Looked at by submit, poll and destroy. */
+ * the device may still write to.  Looked at by submit, poll and destroy; the time
+ * from one of these to the next counts up to half the limit. */
 ma_status ma_server_set_wait_limit(ma_server* srv, double seconds);
 /* Cancels cases not yet admitted, waits for the active ones to finish their
  * launched steps, frees everything. */

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
@@ -255,6 +256,11 @@ struct ma_server {
   std::vector<double> busy;
   double step_wait = -1.0, round = -1.0;
   double progress = 0.0;       // last time that a wait or a round ended
+  // The clock of these times: it runs while check_waits is called, by at most half
+  // the limit from one call to the next, so that time in which the process was
+  // stopped (or no one asked) is not taken for a wait on the device.
+  std::atomic<double> watched{0.0};
+  double checked = 0.0;        // last call of check_waits
   double wait_limit = 120.0;   // ma_server_set_wait_limit
   bool lost = false;           // a wait did not end: every request has failed, no thread touches the device
   std::string lost_why;
@@ -291,7 +297,10 @@ void fail_request(ma_server* S, Request* r, ma_status st, const std::string& err
 // has).  The threads that can still leave do, without touching the device.
 void check_waits(ma_server* S) {
   if (S->lost) return;
-  const double t = S->now();
+  const double called = S->now();
+  const double t = S->watched + std::min(called - S->checked, 0.5 * S->wait_limit);
+  S->checked = called;
+  S->watched = t;
   double oldest = 0.0;
   const char* what = nullptr;
   auto look = [&](double since, const char* name) {
@@ -329,12 +338,12 @@ struct Wait {
   size_t i;
   Wait(ma_server* server, size_t thread) : S(server), i(thread) {
     std::lock_guard<std::mutex> lk(S->mu);
-    S->busy[i] = S->now();
+    S->busy[i] = S->watched;
   }
   ~Wait() {
     std::lock_guard<std::mutex> lk(S->mu);
     S->busy[i] = -1.0;
-    S->progress = S->now();
+    S->progress = S->watched;
   }
 };
 
@@ -568,7 +577,7 @@ void scheduler(ma_server* S) {
       S->step_wait = S->round = -1.0;
       if (idle()) S->cv_sched.wait(lk, [&] { return S->stop || S->lost || !S->incoming.empty(); });
       if (S->lost) return;
-      S->round = S->now();
+      S->round = S->watched;
       if (progress) S->progress = S->round;
       for (auto& g : groups)
         if (!g->inflight.empty() && (S->step_wait < 0.0 || g->since < S->step_wait)) S->step_wait = g->since;
@@ -649,7 +658,7 @@ void scheduler(ma_server* S) {
         }
         Group::Step st = g.inflight.front();
         g.inflight.pop_front();
-        g.since = S->now();
+        g.since = S->watched;
         g.spare.push_back(st.ev);
         for (Request* r : st.finishing) {
           ma::solver_set_progress(r->solver, r->total);
@@ -696,7 +705,7 @@ void scheduler(ma_server* S) {
           g.act.swap(keep);
           g.dirty = true;
         }
-        if (g.inflight.empty()) g.since = S->now();
+        if (g.inflight.empty()) g.since = S->watched;
         g.inflight.push_back(std::move(step));
         g.parity ^= 1;
         progress = true;

@@ -2,6 +2,8 @@
 // times 24 requests through one server, all of which finish.  server_check stall:
 // a server whose device stops (STUB_STALL) fails every unfinished request with
 // MA_ERR_DEVICE within its wait limit, refuses more, and can be destroyed.
+// server_check pause: many passes with a limit of a second, for a process that is
+// stopped and continued meanwhile.
 // server_check threads: planning a request takes the server's setup thread alone.
 #include <dirent.h>
 
@@ -85,14 +87,16 @@ static int threads() {
 int main(int argc, char** argv) {
   if (argc > 1 && !std::strcmp(argv[1], "threads")) return threads();
   const bool stall = argc > 1 && !std::strcmp(argv[1], "stall");
-  const int passes = stall ? 1 : std::atoi(argv[1]);
+  const bool pause = argc > 1 && !std::strcmp(argv[1], "pause");
+  const int passes = stall ? 1 : pause ? 1 << 30 : std::atoi(argv[1]);
+  const double end = now() + 6.0;
   ma_server_config cfg = {600ll << 20, 16, 8, 0, 0};
   ma_server* S = nullptr;
   CHECK(ma_server_create(&cfg, &S) == MA_OK);
   CHECK(ma_server_set_wait_limit(S, 0.0) == MA_ERR_INVALID);
-  CHECK(ma_server_set_wait_limit(S, stall ? 0.4 : 20.0) == MA_OK);
+  CHECK(ma_server_set_wait_limit(S, stall ? 0.4 : pause ? 1.0 : 20.0) == MA_OK);
   int failed = 0;
-  for (int p = 0; p < passes; ++p) {
+  for (int p = 0; p < passes && (!pause || now() < end); ++p) {
     std::set<long long> ids;
     const double t0 = now();
     for (int i = 0; i < 24; ++i) {

@@ -4,7 +4,9 @@ errors and not in a server that hangs."""
 import os
 import re
 import shutil
+import signal
 import subprocess
+import time
 
 import pytest
 
@@ -35,17 +37,34 @@ def check(tmp_path_factory):
         os.path.join(checks, "server_check.cpp"), "-Wl,--unresolved-symbols=ignore-in-shared-libs",
         "-L", os.path.dirname(LIB), "-lminiaero_amd", "-o", exe)
 
-    def go(what, **env):
-        r = subprocess.run([exe, what], capture_output=True, text=True, timeout=100,
-                           env=dict(os.environ, LD_LIBRARY_PATH=str(tmp) + ":" + os.path.dirname(LIB), **env))
-        print(r.stdout)
-        assert r.returncode == 0, r.stdout + r.stderr
-        return r.stdout
+    def go(what, meanwhile=None, **env):
+        r = subprocess.Popen([exe, what], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                             env=dict(os.environ, LD_LIBRARY_PATH=str(tmp) + ":" + os.path.dirname(LIB), **env))
+        try:
+            if meanwhile:
+                meanwhile(r)
+            out = r.communicate(timeout=100)[0]
+        finally:
+            r.kill()
+        print(out)
+        assert r.returncode == 0, out
+        return out
     return go
 
 
 def test_requests_through_one_server(check):
     check("80")
+
+
+def test_a_process_that_was_stopped_has_lost_nothing(check):
+    """Time in which the process does not run is not a wait on the device."""
+    def stop_and_continue(p):
+        for _ in range(2):
+            time.sleep(0.7)
+            p.send_signal(signal.SIGSTOP)
+            time.sleep(1.5)
+            p.send_signal(signal.SIGCONT)
+    check("pause", meanwhile=stop_and_continue)
 
 
 def test_planning_takes_one_thread_a_request(check):
