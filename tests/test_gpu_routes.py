@@ -352,3 +352,35 @@ def test_plates_on_both_sides_of_the_bounds(stretch, scheme):
         assert np.isfinite(R).all() and np.array_equal(G, R)
     finally:
         p.close()
+
+
+FIRST_CAPTURE = """
+import sys
+sys.path[:0] = %r
+import numpy as np
+import miniaero_amd as M
+from test_gpu_routes import _case
+md, o = _case((33, 17, 9), workgroups_per_cu=1)
+states = []
+for graph in (2, 0):
+    s = M.TimeSolverExplicitRK4(md, o)
+    if graph:
+        s.set_graph(graph)
+    s.initialize()
+    s.step(4)
+    states.append(s.state())
+    s.close()
+assert np.isfinite(states[0]).all() and np.array_equal(*states)
+"""
+
+
+def test_first_use_of_the_walking_kernels_in_a_capture():
+    """A process whose first launch of these kernels, in a code object that nothing
+    else of the run has loaded, is recorded into a graph."""
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c", FIRST_CAPTURE % [here, os.path.dirname(here)]], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
